@@ -578,6 +578,17 @@ void winding_taylor_noalloc(
 // Zero-fill helper (a kernel, not hipMemsetAsync, so that captured graphs replay it safely).
 void fill_u32(std::uint32_t *ptr, std::uint32_t value, std::size_t n, hipStream_t stream);
 
+// Whether work enqueued on `stream` is being captured into a graph (also true where the runtime
+// will not say, as for the null stream while another stream captures).
+inline bool stream_capturing(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return status != hipStreamCaptureStatusNone;
+}
+
 inline unsigned grid_for(std::size_t n, int block) {
     std::size_t g = (n + static_cast<std::size_t>(block) - 1) / static_cast<std::size_t>(block);
     return static_cast<unsigned>(g == 0 ? 1 : g);

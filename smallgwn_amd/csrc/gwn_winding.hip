@@ -22,6 +22,7 @@
 // default across statements), so every kernel that evaluates a term -- per-lane, wave, gradient,
 // batched -- rounds it identically and their results agree bit for bit.
 #include <mutex>
+#include <type_traits>
 
 #include "gwn_core.hpp"
 #include "../../include/gwn/detail/gwn_device_winding.hpp"
@@ -42,61 +43,282 @@ constexpr std::uint32_t k_invalid = 0xffffffffu;
 
 constexpr int k_exact_block = 256;
 
-template <int Prec, class Out>
-__global__ __launch_bounds__(k_exact_block) void exact_kernel(
+// What one triangle contributes to every query's solid angle, formed once per tile while the
+// record is staged: 64 bytes, so a lane's broadcast reads are four aligned 16-byte LDS reads.
+// Plain: the reference's corners v0, v0 + (v1 - v0), v0 + (v2 - v0).  Split: v0, the edges
+// e1, e2, their cross product n, |e1|^2, |e2|^2, e1 . e2 and the squared near-field radius.
+struct __align__(16) exact_item {
+    float f[16];
+    __device__ static exact_item load(exact_item const &src) {
+        exact_item t;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            reinterpret_cast<float4 *>(t.f)[j] = reinterpret_cast<float4 const *>(src.f)[j];
+        return t;
+    }
+};
+
+template <int Prec>
+__device__ inline void stage_exact_item(tri_record const &t, exact_item &o) {
+    float const e1x = t.v1x - t.v0x, e1y = t.v1y - t.v0y, e1z = t.v1z - t.v0z;
+    float const e2x = t.v2x - t.v0x, e2y = t.v2y - t.v0y, e2z = t.v2z - t.v0z;
+    float4 *const d = reinterpret_cast<float4 *>(o.f);
+    d[0] = {t.v0x, t.v0y, t.v0z, Prec == GWN_PRECISION_PLAIN ? t.v0x + e1x : e1x};
+    if constexpr (Prec == GWN_PRECISION_PLAIN) {
+        d[1] = {t.v0y + e1y, t.v0z + e1z, t.v0x + e2x, t.v0y + e2y};
+        d[2] = {t.v0z + e2z, 0.0f, 0.0f, 0.0f};
+    } else {
+        float const s1 = e1x * e1x + e1y * e1y + e1z * e1z;
+        float const s2 = e2x * e2x + e2y * e2y + e2z * e2z;
+        d[1] = {e1y, e1z, e2x, e2y};
+        d[2] = {e2z, e1y * e2z - e1z * e2y, e1z * e2x - e1x * e2z, e1x * e2y - e1y * e2x};
+        d[3] = {s1, s2, e1x * e2x + e1y * e2y + e1z * e2z, k_split_near_scale2 * fmaxf(s1, s2)};
+    }
+}
+
+// solid_angle_plain on the staged corners (the same operations from there on).
+__device__ inline float solid_angle_plain_staged(exact_item const &t, float qx, float qy, float qz) {
+    float ax = t.f[0] - qx, ay = t.f[1] - qy, az = t.f[2] - qz;
+    float bx = t.f[3] - qx, by = t.f[4] - qy, bz = t.f[5] - qz;
+    float cx = t.f[6] - qx, cy = t.f[7] - qy, cz = t.f[8] - qz;
+    float const al = sqrtf(ax * ax + ay * ay + az * az);
+    float const bl = sqrtf(bx * bx + by * by + bz * bz);
+    float const cl = sqrtf(cx * cx + cy * cy + cz * cz);
+    if (al == 0.0f || bl == 0.0f || cl == 0.0f)
+        return 0.0f;
+    ax /= al; ay /= al; az /= al;
+    bx /= bl; by /= bl; bz /= bl;
+    cx /= cl; cy /= cl; cz /= cl;
+    float const ux = bx - ax, uy = by - ay, uz = bz - az;
+    float const vx = cx - ax, vy = cy - ay, vz = cz - az;
+    float const num = ax * (uy * vz - uz * vy) + ay * (uz * vx - ux * vz) + az * (ux * vy - uy * vx);
+    if (num == 0.0f)
+        return 0.0f;
+    float const den = 1.0f + (ax * bx + ay * by + az * bz) + (ax * cx + ay * cy + az * cz) +
+                      (bx * cx + by * cy + bz * cz);
+    return 2.0f * atan2f(num, den);
+}
+
+// Half the solid angle of a staged far triangle (|a| > 4 max(|e1|, |e2|), a = v0 - q), split form;
+// any value where `near`.  With s1 = a . e1 and s2 = a . e2 every length and dot product of the
+// corners b = a + e1 and c = a + e2 is a short sum: |b|^2 = |a|^2 + 2 s1 + |e1|^2, a . b = |a|^2 + s1,
+// b . c = a . b + s2 + e1 . e2 (and so on), none of which cancels, since |e| < |a| / 4.  The same
+// bound gives |num| <= |a|^3 / 16 and den >= 2.1 |a|^3, so u = num / den <= 0.03 and
+// u - u^3 / 3 + u^5 / 5 is atan(u) to u^7 / 7 < 1e-10 of u: 42 operations and 4 half-rate ones
+// where the two-argument arctangent and the edges formed per pair took 109.  A denominator outside
+// the reciprocal's range (coordinates near the ends of the float range) takes the arctangent.
+__device__ inline float half_angle_far_staged(exact_item const &t, float ax, float ay, float az, float aa, bool near) {
+    float const s1 = ax * t.f[3] + ay * t.f[4] + az * t.f[5];
+    float const s2 = ax * t.f[6] + ay * t.f[7] + az * t.f[8];
+    float const num = ax * t.f[9] + ay * t.f[10] + az * t.f[11];
+    float const la = __builtin_amdgcn_sqrtf(aa);
+    float const lb = __builtin_amdgcn_sqrtf(aa + (2.0f * s1 + t.f[12]));
+    float const lc = __builtin_amdgcn_sqrtf(aa + (2.0f * s2 + t.f[13]));
+    float const ab = aa + s1;
+    float const ac = aa + s2;
+    float const bc = ab + (s2 + t.f[14]);
+    float const den = la * lb * lc + ab * lc + ac * lb + bc * la;
+    float const u = num * __builtin_amdgcn_rcpf(den);
+    float const u2 = u * u;
+    float h = u + u * (u2 * (u2 * 0.2f - 0.33333334f));
+    constexpr std::uint32_t k_lo = 0x01000000u, k_hi = 0x7e000000u;  // 2^-125, 2^125
+    if (__float_as_uint(den) - k_lo >= k_hi - k_lo && !near)
+        h = atan2f(num, den);
+    return h;
+}
+
+// Adds the values of a group's Lanes lanes to its running sum in lane order (the group's lanes are
+// Lanes consecutive lanes of a 16-lane row; every one ends with the same sum).
+template <int Lanes, int J = 0> __device__ inline void add_in_lane_order(float &sum, float v) {
+    if constexpr (Lanes == 1) {
+        sum += v;
+    } else if constexpr (J < Lanes) {
+        constexpr int k_ctrl = Lanes == 4 ? J * 0x55 : 0x150 + J;  // quad_perm [J, J, J, J] / row_newbcast:J
+        sum += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), k_ctrl, 0xf, 0xf, false));
+        add_in_lane_order<Lanes, J + 1>(sum, v);
+    }
+}
+
+// Plain exact batch, Lanes (1, 4 or 16) lanes per query: lane j of a query's group evaluates
+// triangles j, j + Lanes, ... of each 256-record tile, and the group adds each round's angles in
+// record order, so every query's float sum is formed over the records in the reference's order
+// whatever Lanes is (a lane past the tile's end adds zero, which changes no sum).
+//
+// VALU bound: about 220 issue slots a pair (nine correctly rounded quotients, three square roots,
+// one arctangent), one to sixteen for the ordered add.  One lane per query leaves the chip idle
+// below some hundred thousand queries.  Measured with one lane against the widest groups that fill
+// the chip, 131,044 triangles: 1,000 queries 74.0 against 5.6 ms, 65,536 queries 74.1 against 49.8 ms,
+// 131,072 queries 110 against 96 ms.
+template <int Lanes, class Out>
+__global__ __launch_bounds__(k_exact_block) void exact_plain_kernel(
     tri_record const *__restrict__ tris, std::size_t nt, float const *__restrict__ qx,
     float const *__restrict__ qy, float const *__restrict__ qz, Out *__restrict__ out, std::size_t nq
 ) {
-    __shared__ tri_record tile[k_exact_block];
+    static_assert(Lanes == 1 || Lanes == 4 || Lanes == 16, "groups are a lane, a quad or a row");
+    __shared__ exact_item tile[k_exact_block];
+    std::size_t const qi = (static_cast<std::size_t>(blockIdx.x) * k_exact_block + threadIdx.x) / Lanes;
+    int const j = static_cast<int>(threadIdx.x) % Lanes;
+    bool const active = qi < nq;
+    float const x = active ? qx[qi] : 0.0f;
+    float const y = active ? qy[qi] : 0.0f;
+    float const z = active ? qz[qi] : 0.0f;
+    float sum = 0.0f;
+    for (std::size_t base = 0; base < nt; base += k_exact_block) {
+        int const count = static_cast<int>((nt - base) < k_exact_block ? (nt - base) : k_exact_block);
+        __syncthreads();
+        if (static_cast<int>(threadIdx.x) < count)
+            stage_exact_item<GWN_PRECISION_PLAIN>(tris[base + threadIdx.x], tile[threadIdx.x]);
+        __syncthreads();
+        for (int k = 0; k < count; k += Lanes) {
+            float v = 0.0f;
+            if (Lanes == 1 || k + j < count)
+                v = solid_angle_plain_staged(tile[k + j], x, y, z);
+            add_in_lane_order<Lanes>(sum, v);
+        }
+    }
+    if (active && j == 0)
+        out[qi] = static_cast<Out>(sum / (4.0f * k_pi_f));
+}
+
+// Split and FP64 exact batches: one query per lane; the block streams its share of the leaf-ordered
+// records through LDS in 256-record tiles.  blockIdx.y is the share: tiles [y, y + 1) *
+// tiles_per_share.  With one share the winding number goes to `out`; with more, the share's FP64 sum
+// goes to part[y * nq + q] and exact_combine_kernel adds the shares in order.
+//
+// VALU bound (a split pair costs 49 issue slots), so what counts is that every SIMD has waves: a
+// launch of nq / 256 blocks alone left 32,749 queries on half of the CUs with one wave per SIMD.
+// Measured, split, one share with per-pair edges and arctangents against this form: 100,000 triangles
+// x 32,749 queries 38.1 against 5.0 ms, 131,044 x 1,000 52.3 against 0.48 ms, 25,600 x 600,000 (one
+// share in both) 56.9 against 37.0 ms.
+template <int Prec>
+__global__ __launch_bounds__(k_exact_block) void exact_kernel(
+    tri_record const *__restrict__ tris, std::size_t nt, float const *__restrict__ qx,
+    float const *__restrict__ qy, float const *__restrict__ qz, double *__restrict__ out, double *__restrict__ part,
+    std::size_t nq, std::size_t tiles_per_share
+) {
+    static_assert(Prec == GWN_PRECISION_SPLIT || Prec == GWN_PRECISION_FP64, "FP64 sums");
+    constexpr bool k_raw = Prec == GWN_PRECISION_FP64;
+    __shared__ std::conditional_t<k_raw, tri_record, exact_item> tile[k_exact_block];
     std::size_t const qi = static_cast<std::size_t>(blockIdx.x) * k_exact_block + threadIdx.x;
     bool const active = qi < nq;
     float const x = active ? qx[qi] : 0.0f;
     float const y = active ? qy[qi] : 0.0f;
     float const z = active ? qz[qi] : 0.0f;
-    float sum_f = 0.0f;   // plain: the reference's running float sum
-    double sum_d = 0.0;   // split / fp64
-    for (std::size_t base = 0; base < nt; base += k_exact_block) {
-        std::size_t const count = (nt - base) < k_exact_block ? (nt - base) : k_exact_block;
+    double sum = 0.0;
+    std::size_t const share = tiles_per_share * k_exact_block;
+    std::size_t const first = static_cast<std::size_t>(blockIdx.y) * share;
+    std::size_t const last = nt - first < share ? nt : first + share;
+    for (std::size_t base = first; base < last; base += k_exact_block) {
+        int const count = static_cast<int>((last - base) < k_exact_block ? (last - base) : k_exact_block);
         __syncthreads();
-        {
-            float const *src = reinterpret_cast<float const *>(tris + base);
-            float *dst = reinterpret_cast<float *>(tile);
-            std::size_t const words = count * 9;
-            for (std::size_t w = threadIdx.x; w < words; w += k_exact_block)
-                dst[w] = src[w];
+        if (static_cast<int>(threadIdx.x) < count) {
+            if constexpr (k_raw)
+                tile[threadIdx.x] = tris[base + threadIdx.x];
+            else
+                stage_exact_item<Prec>(tris[base + threadIdx.x], tile[threadIdx.x]);
         }
         __syncthreads();
-        if constexpr (Prec == GWN_PRECISION_PLAIN) {
-            for (std::size_t k = 0; k < count; ++k)
-                sum_f += solid_angle_plain(tile[k], x, y, z);
-        } else if constexpr (Prec == GWN_PRECISION_FP64) {
-            for (std::size_t k = 0; k < count; ++k)
-                sum_d += solid_angle_f64(tile[k], x, y, z);
+        if constexpr (k_raw) {
+            for (int k = 0; k < count; ++k)
+                sum += solid_angle_f64(tile[k], x, y, z);
         } else {
             // Per-tile FP32 partial sums of the far triangles, folded into the FP64 total.
             float far = 0.0f;
-            for (std::size_t k = 0; k < count; ++k) {
-                tri_record const &t = tile[k];
-                float const e1x = t.v1x - t.v0x, e1y = t.v1y - t.v0y, e1z = t.v1z - t.v0z;
-                float const e2x = t.v2x - t.v0x, e2y = t.v2y - t.v0y, e2z = t.v2z - t.v0z;
-                float const ax = t.v0x - x, ay = t.v0y - y, az = t.v0z - z;
-                float const e1 = e1x * e1x + e1y * e1y + e1z * e1z;
-                float const e2 = e2x * e2x + e2y * e2y + e2z * e2z;
-                float const dq = ax * ax + ay * ay + az * az;
-                if (!(dq > k_split_near_scale2 * fmaxf(e1, e2)))
-                    sum_d += solid_angle_split_near(t, x, y, z);
-                else
-                    far += solid_angle_far_f32(ax, ay, az, e1x, e1y, e1z, e2x, e2y, e2z);
+            for (int k = 0; k < count; ++k) {
+                exact_item const t = exact_item::load(tile[k]);
+                float const ax = t.f[0] - x, ay = t.f[1] - y, az = t.f[2] - z;
+                float const aa = ax * ax + ay * ay + az * az;
+                bool const near = !(aa > t.f[15]);
+                float const h = half_angle_far_staged(t, ax, ay, az, aa, near);
+                far += near ? 0.0f : h;
+                if (near)
+                    sum += solid_angle_split_near(tris[base + k], x, y, z);
             }
-            sum_d += double(far);
+            sum += 2.0 * double(far);
         }
     }
     if (!active)
         return;
-    if constexpr (Prec == GWN_PRECISION_PLAIN)
-        out[qi] = static_cast<Out>(sum_f / (4.0f * k_pi_f));
+    if (part != nullptr)
+        part[static_cast<std::size_t>(blockIdx.y) * nq + qi] = sum;
     else
-        out[qi] = static_cast<Out>(sum_d / (4.0 * k_pi_d));
+        out[qi] = sum / (4.0 * k_pi_d);
+}
+
+// Winding numbers from the shares' sums, added in share order (the same bits on every run).
+__global__ __launch_bounds__(256) void exact_combine_kernel(
+    double const *__restrict__ part, std::size_t shares, double *__restrict__ out, std::size_t nq
+) {
+    std::size_t const q = static_cast<std::size_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (q >= nq)
+        return;
+    double s = 0.0;
+    for (std::size_t k = 0; k < shares; ++k)
+        s += part[k * nq + q];
+    out[q] = s / (4.0 * k_pi_d);
+}
+
+// Shares of the triangles per query block.  Up to 8 blocks of 256 fit a CU (LDS and registers), so
+// 16 per CU give every SIMD eight waves and a second round to even out the last one.  A share is at
+// least one tile (256 pairs a lane, beside which its staging and its sum are small), and the shares'
+// sums take at most 64 MiB.
+std::size_t exact_shares(std::size_t nt, std::size_t nq) {
+    std::size_t const blocks = (nq + k_exact_block - 1) / k_exact_block;
+    std::size_t const tiles = (nt + k_exact_block - 1) / k_exact_block;
+    std::size_t const target = 16 * 256;
+    if (blocks >= target)
+        return 1;
+    std::size_t s = (target + blocks - 1) / blocks;
+    std::size_t const by_bytes = (std::size_t(64) << 20) / (nq * sizeof(double));
+    s = s < tiles ? s : tiles;
+    s = s < by_bytes ? s : by_bytes;
+    return s == 0 ? 1 : s;
+}
+
+template <int Prec>
+void launch_exact(
+    gwn_bvh_handle const &bvh, float const *qx, float const *qy, float const *qz, double *out, std::size_t nq,
+    hipStream_t stream
+) {
+    std::size_t const nt = bvh.triangle_count;
+    std::size_t const tiles = (nt + k_exact_block - 1) / k_exact_block;
+    std::size_t shares = exact_shares(nt, nq);
+    if (shares > 1 && stream_capturing(stream))  // a captured batch stays one launch without an allocation
+        shares = 1;
+    std::size_t const tiles_per_share = tiles == 0 ? 1 : (tiles + shares - 1) / shares;
+    shares = tiles == 0 ? 1 : (tiles + tiles_per_share - 1) / tiles_per_share;  // none is empty
+    device_buffer<double> part;
+    if (shares > 1)
+        part.allocate(shares * nq, stream);
+    dim3 const grid(grid_for(nq, k_exact_block), static_cast<unsigned>(shares));
+    exact_kernel<Prec><<<grid, k_exact_block, 0, stream>>>(bvh.triangles.ptr, nt, qx, qy, qz, out, part.ptr, nq,
+                                                           tiles_per_share);
+    GWN_LAUNCH_CHECK();
+    if (shares > 1) {
+        exact_combine_kernel<<<grid_for(nq, 256), 256, 0, stream>>>(part.ptr, shares, out, nq);
+        GWN_LAUNCH_CHECK();
+    }
+}
+
+// Plain: the widest groups whose launch still holds eight waves per SIMD, since the ordered add costs
+// up to 16 issue slots a pair with 16 lanes against one with one lane.
+template <class Out>
+void launch_exact_plain(
+    gwn_bvh_handle const &bvh, float const *qx, float const *qy, float const *qz, Out *out, std::size_t nq,
+    hipStream_t stream
+) {
+    std::size_t const full = std::size_t(256) * 8 * k_exact_block;  // lanes of eight waves on every SIMD
+#define GWN_EXACT_PLAIN(L)                                                                        \
+    exact_plain_kernel<L, Out><<<grid_for(nq * L, k_exact_block), k_exact_block, 0, stream>>>(    \
+        bvh.triangles.ptr, bvh.triangle_count, qx, qy, qz, out, nq)
+    if (nq >= full)
+        GWN_EXACT_PLAIN(1);
+    else if (nq * 4 >= full)
+        GWN_EXACT_PLAIN(4);
+    else
+        GWN_EXACT_PLAIN(16);
+#undef GWN_EXACT_PLAIN
+    GWN_LAUNCH_CHECK();
 }
 
 // ------------------------------------------------------------------------------------------
@@ -990,27 +1212,21 @@ void winding_exact(
     gwn_bvh_handle const &bvh, float const *qx, float const *qy, float const *qz, void *out,
     std::size_t n, int precision, query_launch const &, hipStream_t stream
 ) {
-    unsigned const grid = grid_for(n, k_exact_block);
     switch (precision) {
     case -1: // reference-form float output
-        exact_kernel<GWN_PRECISION_PLAIN, float><<<grid, k_exact_block, 0, stream>>>(
-            bvh.triangles.ptr, bvh.triangle_count, qx, qy, qz, static_cast<float *>(out), n);
+        launch_exact_plain(bvh, qx, qy, qz, static_cast<float *>(out), n, stream);
         break;
     case GWN_PRECISION_PLAIN:
-        exact_kernel<GWN_PRECISION_PLAIN, double><<<grid, k_exact_block, 0, stream>>>(
-            bvh.triangles.ptr, bvh.triangle_count, qx, qy, qz, static_cast<double *>(out), n);
+        launch_exact_plain(bvh, qx, qy, qz, static_cast<double *>(out), n, stream);
         break;
     case GWN_PRECISION_SPLIT:
-        exact_kernel<GWN_PRECISION_SPLIT, double><<<grid, k_exact_block, 0, stream>>>(
-            bvh.triangles.ptr, bvh.triangle_count, qx, qy, qz, static_cast<double *>(out), n);
+        launch_exact<GWN_PRECISION_SPLIT>(bvh, qx, qy, qz, static_cast<double *>(out), n, stream);
         break;
     case GWN_PRECISION_FP64:
-        exact_kernel<GWN_PRECISION_FP64, double><<<grid, k_exact_block, 0, stream>>>(
-            bvh.triangles.ptr, bvh.triangle_count, qx, qy, qz, static_cast<double *>(out), n);
+        launch_exact<GWN_PRECISION_FP64>(bvh, qx, qy, qz, static_cast<double *>(out), n, stream);
         break;
     default: throw_invalid("Unknown winding precision mode.");
     }
-    GWN_LAUNCH_CHECK();
 }
 
 namespace {
