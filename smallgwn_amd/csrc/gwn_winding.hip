@@ -7,8 +7,8 @@
 // LDS in 256-record tiles, so every record is read from HBM/L2 once per block and broadcast to
 // all 256 lanes.  VALU bound (solid angle: 3 sqrt, 3 div, 1 atan2 per pair).
 //
-// Taylor batch: one query per lane, queries optionally visited in Hilbert order (results are
-// written back in input order).  Per-lane stack of internal node ids; the last internal child
+// Taylor batch: four lanes per query, or 64 queries per wave where Hilbert-ordered queries are dense
+// (results are written back in input order).  A stack of internal node ids; the last internal child
 // of a node is entered directly, the others are pushed, leaves are evaluated in slot order --
 // the reference's traversal order, so float sums are formed in the same sequence.  The node
 // data is one traversal record per node (compact child refs + field-SoA coefficients), so a
@@ -27,6 +27,7 @@
 #include "gwn_core.hpp"
 #include "../../include/gwn/detail/gwn_device_winding.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 #pragma clang fp contract(on)
@@ -390,29 +391,6 @@ __global__ __launch_bounds__(256) void query_key_kernel(
 }
 
 
-template <int Order, int Prec, bool Grad, int StackCap>
-__global__ __launch_bounds__(k_taylor_block) void taylor_kernel(
-    float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node,
-    float const *__restrict__ qx, float const *__restrict__ qy, float const *__restrict__ qz,
-    std::uint32_t const *__restrict__ order, taylor_outputs o, std::size_t n, float beta2
-) {
-    std::size_t const i = static_cast<std::size_t>(blockIdx.x) * k_taylor_block + threadIdx.x;
-    if (i >= n)
-        return;
-    std::size_t const q = order ? order[i] : i;
-    float const x = qx[q], y = qy[q], z = qz[q];
-    taylor_sums<Prec, Grad> acc;
-    std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;
-    bool const overflow =
-        taylor_traverse<Order, Prec, Grad, StackCap>(records, tris, root_node, x, y, z, beta2, acc, n_tests, n_accept, n_leaf);
-    acc.store(overflow, q, o.out, o.gx, o.gy, o.gz);
-    if (o.counters != nullptr) {
-        o.counters[3 * q + 0] = n_tests;
-        o.counters[3 * q + 1] = n_accept;
-        o.counters[3 * q + 2] = n_leaf;
-    }
-}
-
 // Wave-cooperative traversal (defined below; the batched kernel uses it too).
 template <int Order, int Prec, bool Grad, int StackCap>
 __device__ inline bool taylor_wave_traverse(
@@ -649,6 +627,181 @@ __global__ __launch_bounds__(256) void leaf_root_kernel(
     }
 }
 
+// Every lane of a quad (lanes 4k..4k+3) receives lane S's value.
+template <int S, class T> __device__ inline T quad_bcast(T v) {
+    if constexpr (sizeof(T) == 8) {
+        std::uint64_t const b = __builtin_bit_cast(std::uint64_t, v);
+        std::uint64_t const lo = quad_bcast<S>(static_cast<std::uint32_t>(b));
+        std::uint64_t const hi = quad_bcast<S>(static_cast<std::uint32_t>(b >> 32));
+        return __builtin_bit_cast(T, (hi << 32) | lo);
+    } else {
+        return __builtin_bit_cast(
+            T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), S * 0x55, 0xf, 0xf, false));  // quad_perm [S, S, S, S]
+    }
+}
+
+// Adds the four lanes' terms to a quad's sum in slot order.  A slot without a term holds zero, which
+// leaves every sum it meets as it is (a sum starts at +0 and never becomes -0).
+template <class T> __device__ inline void quad_add(T &sum, T v) {
+    sum += quad_bcast<0>(v);
+    sum += quad_bcast<1>(v);
+    sum += quad_bcast<2>(v);
+    sum += quad_bcast<3>(v);
+}
+
+// What one lane of a quad reads of a node: its slot's reference, acceptance fields and coefficients.
+template <int Order, bool Grad> struct quad_slot {
+    static constexpr int k_fields = moment_field_count(Order);
+    static constexpr int k_block = eval_slot_floats(Order);
+    std::uint32_t ref;
+    float mp, cx, cy, cz;
+    float c[Grad ? 4 * k_fields : k_block];  // Grad: field k at [4 k]
+
+    __device__ static quad_slot load(float4 const *__restrict__ records, std::uint32_t node, int j) {
+        constexpr int RV = Grad ? moment_record_vec4(Order) : eval_record_vec4(Order);
+        float const *const w = reinterpret_cast<float const *>(records + static_cast<std::size_t>(node) * RV) + j;
+        quad_slot s;
+        s.ref = __float_as_uint(w[0]);
+        s.mp = w[4];
+        s.cx = w[8];
+        s.cy = w[12];
+        s.cz = w[16];
+        if constexpr (Grad) {
+#pragma unroll
+            for (int k = 4; k < k_fields; ++k)
+                s.c[4 * k] = w[4 + 4 * k];
+        } else {
+            float4 const *const b = reinterpret_cast<float4 const *>(w - j + 20 + j * k_block);
+#pragma unroll
+            for (int k = 0; k < k_block / 4; ++k) {
+                float4 const v = b[k];
+                s.c[4 * k] = v.x;
+                s.c[4 * k + 1] = v.y;
+                s.c[4 * k + 2] = v.z;
+                s.c[4 * k + 3] = v.w;
+            }
+        }
+        return s;
+    }
+};
+
+// Taylor traversal with four lanes per query, lane j of the quad owning child slot j: the four
+// acceptance tests, expansions and leaf triangles of a node are evaluated side by side and their terms
+// added in slot order (quad_add); descended children are pushed in slot order and the last one entered,
+// as taylor_traverse does.  Decisions, terms and the order of every sum are those of the per-lane
+// traversal, so the results are too, bit for bit.  The stack is the quad's column of an LDS array.
+//
+// Latency bound: a small batch is one chain of dependent node reads per query, so what counts is the
+// reads on the chain.  One lane per query waited for the header, then for each accepted slot's
+// coefficients and each leaf's triangle in turn (about eight waits a node); here a node's header and
+// all four slots' coefficients arrive together, and the next node's are requested as soon as the
+// decisions are known, before the leaf triangles are evaluated.  Measured, per-lane against this form:
+// 1,000 queries of 5,120 triangles (order 1, beta 2) 749 against 153 us.  Holding a quad's leaf triangles
+// back until half of the wave's quads have some (so that they are evaluated with more lanes active)
+// made every size 5-20 % slower.
+template <int Order, int Prec, bool Grad, int StackCap>
+__global__ __launch_bounds__(k_taylor_block) void taylor_quad_kernel(
+    float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node,
+    float const *__restrict__ qx, float const *__restrict__ qy, float const *__restrict__ qz,
+    std::uint32_t const *__restrict__ order, taylor_outputs o, std::size_t n, float beta2
+) {
+    constexpr int k_quads = k_taylor_block / 4;
+    __shared__ std::uint32_t s_stack[StackCap * k_quads];  // entry e of quad k at [e * k_quads + k]
+    std::size_t const i = (static_cast<std::size_t>(blockIdx.x) * k_taylor_block + threadIdx.x) >> 2;
+    if (i >= n)
+        return;  // whole quads
+    int const j = static_cast<int>(threadIdx.x & 3);
+    int const quad_shift = static_cast<int>(threadIdx.x & 60);
+    std::uint32_t *const stack = s_stack + (threadIdx.x >> 2);
+    std::size_t const q = order ? order[i] : i;
+    float const x = qx[q], y = qy[q], z = qz[q];
+    taylor_sums<Prec, Grad> acc;
+    std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;
+    int sp = 0;
+    bool overflow = false;
+    bool live = true;
+    quad_slot<Order, Grad> slot = quad_slot<Order, Grad>::load(records, root_node, j);
+    while (live) {
+        std::uint32_t const c = slot.ref;
+        bool const valid = c != k_invalid;
+        float const qrx = x - slot.cx, qry = y - slot.cy, qrz = z - slot.cz;
+        float const ql2 = squared_norm_unfused(qrx, qry, qrz);
+        bool const far = !(!(ql2 > 0.0f) || ql2 <= product_unfused(slot.mp, beta2));
+        float g[3];
+        float w;
+        if constexpr (Grad)
+            w = taylor_term<Order, true>(slot.c, 0, qrx, qry, qrz, ql2, g);
+        else
+            w = taylor_value<Order>(slot.c, qrx, qry, qrz, ql2);
+        bool const accepted = valid && far && isfinite(w);
+        bool const descend = valid && !accepted;
+        bool const leaf = descend && (c & k_cref_leaf) != 0u;
+        bool const inner = descend && (c & k_cref_leaf) == 0u;
+        n_tests += valid ? 1u : 0u;
+        n_accept += accepted ? 1u : 0u;
+        n_leaf += leaf ? 1u : 0u;
+        // The node's triangles, requested before the next node.
+        tri_record t{};
+        if (__ballot(leaf) != 0ull)
+            t = tris[leaf ? (c & ~k_cref_leaf) : 0u];
+        // The last descended internal child is entered, the others are pushed in slot order.
+        std::uint32_t const bits = static_cast<std::uint32_t>(__ballot(inner) >> quad_shift) & 15u;
+        std::uint32_t const c0 = quad_bcast<0>(c), c1 = quad_bcast<1>(c), c2 = quad_bcast<2>(c), c3 = quad_bcast<3>(c);
+        int const pushed = __popc(bits) - 1;
+        std::uint32_t next = bits & 8u ? c3 : (bits & 4u ? c2 : (bits & 2u ? c1 : c0));
+        int const at = sp + __popc(bits & ((1u << j) - 1u));
+        if (inner && (bits >> j) != 1u && at < StackCap)
+            stack[at * k_quads] = c;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (pushed >= 0) {
+            sp += pushed;
+            overflow = sp > StackCap;
+            live = !overflow;
+        } else if (sp > 0) {
+            next = stack[--sp * k_quads];
+        } else {
+            live = false;
+        }
+        quad_slot<Order, Grad> const ahead = quad_slot<Order, Grad>::load(records, live ? next : root_node, j);
+        taylor_sums<Prec, Grad> term;
+        if (accepted)
+            term.far_term(w, g);
+        if (leaf)
+            term.leaf(t, x, y, z);
+        if constexpr (Prec == GWN_PRECISION_PLAIN) {
+            quad_add(acc.omega, term.omega);
+            if constexpr (Grad) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+                    quad_add(acc.gf[k], term.gf[k]);
+            }
+        } else {
+            quad_add(acc.near, term.near);
+            if constexpr (Grad) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+                    quad_add(acc.gd[k], term.gd[k]);
+            }
+        }
+        slot = ahead;
+    }
+    if (j == 0)
+        acc.store(overflow, q, o.out, o.gx, o.gy, o.gz);
+    if (o.counters != nullptr) {
+        auto const total = [](std::uint32_t v) {
+            return quad_bcast<0>(v) + quad_bcast<1>(v) + quad_bcast<2>(v) + quad_bcast<3>(v);
+        };
+        n_tests = total(n_tests);
+        n_accept = total(n_accept);
+        n_leaf = total(n_leaf);
+        if (j == 0) {
+            o.counters[3 * q + 0] = n_tests;
+            o.counters[3 * q + 1] = n_accept;
+            o.counters[3 * q + 2] = n_leaf;
+        }
+    }
+}
+
 // Reciprocal square root and reciprocal in FP64 from the hardware approximations and Newton
 // steps (relative error at FP64 rounding level, not correctly rounded).  x > 0 / x != 0.
 __device__ inline double rsq_f64_fast(double x) {
@@ -767,7 +920,7 @@ __device__ inline void adjoint_leaf(
         atomicAdd(d + k, t9[k]);
 }
 
-// Adjoint of sum_q u_q w_q (orders 0, 1): the per-lane traversal of taylor_kernel with the same
+// Adjoint of sum_q u_q w_q (orders 0, 1): the per-lane traversal (taylor_traverse) with the same
 // accept/descend decisions.  An accepted child adds u/(4 pi) (dw/dP, dw/dN, dw/dT) to its slot's
 // 12 entries (dw/dP = -dw/dq); a near triangle adds u/(4 pi) dW/d(a, b, c) to its record's 9
 // entries; the query gradient goes to dq.  root_node = k_invalid evaluates the leaf root instead.
@@ -872,6 +1025,21 @@ __global__ __launch_bounds__(k_taylor_block) void taylor_adjoint_kernel(
     }
 }
 
+// Whether Hilbert-ordered queries are dense enough for 64 of them to walk the tree together.  The wave
+// traversal does little per query, but its time does not fall below that of its longest wave, whose
+// union of paths grows with the square root of the triangles near it and with beta; the quad
+// traversal's time is proportional to the queries.  Measured (MI355X, mixed queries, sort included),
+// wave against quad, order 2:
+//   beta 2:    5,120 triangles, 262k queries 463 / 463 us, 1M 696 / 963 us; 131,072, 1M 1.88 / 1.44 ms,
+//              4M 2.75 / 4.31 ms; 1,048,576, 1M 5.23 / 2.30 ms, 4M 5.86 / 4.88 ms
+//   beta 6.25 (split): 5,120, 66k 1.47 / 0.95 ms, 262k 1.57 / 2.12 ms; 131,072, 262k 4.78 / 4.09 ms,
+//              1M 6.62 / 9.97 ms; 1,048,576, 262k 13.1 / 6.6 ms, 1M 13.4 / 14.1 ms
+// The crossings lie near 4500 sqrt(triangles) (2 / beta)^1.5.
+bool dense_queries(std::size_t triangles, std::size_t n, float beta2) {
+    double const beta = std::sqrt(std::max(1.0, double(beta2)));
+    return double(n) >= 4500.0 * std::sqrt(double(triangles)) * std::pow(2.0 / beta, 1.5);
+}
+
 template <int Order, int Prec, bool Grad, int Cap>
 void launch_taylor_cap(
     gwn_bvh_handle const &bvh, gwn_moment_handle const &m, float const *qx, float const *qy,
@@ -881,13 +1049,13 @@ void launch_taylor_cap(
     std::uint32_t const root = static_cast<std::uint32_t>(ref_offset(bvh.root.reference));
     // The value alone reads the evaluation records; the gradient the traversal records.
     float4 const *records = Grad ? m.records.ptr : m.eval_records.ptr;
-    if (order != nullptr) {
-        // Hilbert-ordered queries: neighbouring lanes share most of their paths.
+    if (order != nullptr && dense_queries(bvh.triangle_count, n, beta2)) {
+        // Hilbert-ordered dense queries: neighbouring lanes share most of their paths.
         taylor_wave_kernel<Order, Prec, Grad, Cap><<<grid_for(n, k_taylor_block), k_taylor_block, 0, stream>>>(
             records, bvh.triangles.ptr, root, qx, qy, qz, order, o, n, beta2
         );
     } else {
-        taylor_kernel<Order, Prec, Grad, Cap><<<grid_for(n, k_taylor_block), k_taylor_block, 0, stream>>>(
+        taylor_quad_kernel<Order, Prec, Grad, Cap><<<grid_for(4 * n, k_taylor_block), k_taylor_block, 0, stream>>>(
             records, bvh.triangles.ptr, root, qx, qy, qz, order, o, n, beta2
         );
     }

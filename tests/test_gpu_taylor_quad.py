@@ -1,0 +1,58 @@
+"""The four-lanes-per-query Taylor traversal against the wave traversal: values, gradients and work
+counters equal bit for bit, at the edges of quads, waves and blocks and on both sides of the density
+rule that chooses between them."""
+
+import numpy as np
+import pytest
+
+from smallgwn_amd import synth
+from tests.test_gpu_build import build_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+def _first(q, n, dev):
+    import torch
+
+    return [torch.from_numpy(np.ascontiguousarray(a[:n])).to(dev) for a in q]
+
+
+def _run(gwn, dev, bvh, mom, d, sort, precision, beta, grad):
+    import torch
+
+    n = d[0].numel()
+    out = torch.full((n,), 7.0, dtype=torch.float32, device=dev)
+    cnt = torch.zeros(3 * n, dtype=torch.int32, device=dev)
+    cfg = gwn.QueryConfig(sort_queries=sort)
+    if grad:
+        g = [torch.full_like(out, 7.0) for _ in range(3)]
+        gwn.gwn_compute_winding_gradient_taylor_batch(bvh, mom, *d, *g, accuracy_scale=beta, config=cfg,
+                                                      precision=precision, out=out, counters=cnt).raise_if_error()
+    else:
+        g = []
+        gwn.gwn_compute_winding_number_taylor_batch(bvh, mom, *d, out, accuracy_scale=beta, config=cfg,
+                                                    precision=precision, counters=cnt).raise_if_error()
+    torch.cuda.synchronize()
+    return [t.cpu().numpy().view(np.uint32) for t in (out, cnt, *g)]
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("order", [0, 1, 2])
+def test_quad_equals_wave_bit_for_bit(gwn, dev, order, split, grad):
+    precision = gwn.Precision.SPLIT if split else gwn.Precision.PLAIN
+    # 8 triangles: dense from 12,728 queries at scale 2; 320: from one query at scale 1e6.
+    for mesh, beta, n_wave in ((synth.octahedron(), 2.0, 14000), (synth.icosphere(2), 1e6, 400)):
+        _, bvh = build_gpu(gwn, mesh)
+        mom = gwn.MomentObject(order)
+        gwn.gwn_refit_bvh_moment(bvh, mom).raise_if_error()
+        q = synth.mixed_queries(mesh, n_wave, seed=order + 11)
+        q[0][5], q[1][6] = np.nan, np.inf
+        want = _run(gwn, dev, bvh, mom, _first(q, n_wave, dev), 1, precision, beta, grad)
+        for n in (1, 15, 16, 17, 63, 65, 255, 257):
+            got = _run(gwn, dev, bvh, mom, _first(q, n, dev), 0, precision, beta, grad)
+            for k, (a, b) in enumerate(zip(got, want)):
+                b = b[:3 * n] if k == 1 else b[:n]
+                fa, fb = a.view(np.float32), b.view(np.float32)
+                same = (a == b) | (np.isnan(fa) & np.isnan(fb) if k != 1 else False)
+                assert same.all(), (beta, n, k)
