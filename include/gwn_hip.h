@@ -67,7 +67,7 @@ typedef struct gwn_batch_handle *gwn_batch_t;
  * for its 64 points, each point pruning by its own best distance).  Its distances are each
  * point's minimum over the triangles it reaches, which can differ from the reference order's in
  * the last FP32 bits where a box distance rounds above a contained triangle's distance.
- * lanes_per_point (unsigned distance batch only; other batches ignore it): 0 (default: four),
+ * lanes_per_point (unsigned distance batch only; other batches ignore it): 0 (default: four or 16),
  * 1, or 4.  With four, the lanes of a quad share each BVH4 node, one child slot each; distances
  * and nearest records equal the one-lane traversal's bit for bit.  Ignored with
  * sort_queries = 2. */

@@ -3,8 +3,8 @@
 // Reference: include/gwn/detail/gwn_query_distance_impl.cuh:20-192,
 // include/gwn/detail/gwn_query_geometry_impl.cuh:46-114, include/gwn/gwn_query.cuh:109-180.
 //
-// Near-first culled traversal of the canonical BVH4 (one lane per point in distance_kernel, four
-// in distance_quad_kernel, the default, with the same results): the culling band
+// Near-first culled traversal of the canonical BVH4 (one lane per point in distance_kernel, four or
+// 16 in distance_quad_kernel, the default, with the same results): the culling band
 // (clamped at zero) is the initial squared bound and the result when nothing is closer; children
 // whose box is no closer than the current best are skipped; the survivors are ordered by box
 // distance with a five-comparator network; leaves of a node are evaluated before its internal
@@ -16,6 +16,8 @@
 //
 // Arithmetic is unfused and the square root correctly rounded, so every result equals the CPU
 // oracle's replay bit for bit.
+#include <algorithm>
+
 #include "gwn_core.hpp"
 #include "../../include/gwn/detail/gwn_device_distance.hpp"
 
@@ -144,150 +146,526 @@ __device__ inline std::uint32_t quad_bcast(std::uint32_t v) {
         __builtin_amdgcn_update_dpp(0, static_cast<int>(v), S * 0x55, 0xf, 0xf, false));  // quad_perm [S,S,S,S]
 }
 
-// Quad form of distance_traverse: four lanes per point, lane j of the quad owning child slot j of
-// each node.  Lane j computes its child's box distance and, for a leaf child nearer than the best
-// at node entry, its triangles' minimum and first record attaining it (a triangle's distance does
-// not depend on the best found before it).  The quad shares the four results, and every lane
-// replays distance_traverse's steps on them: compaction of the children nearer than the best,
-// the same five-comparator sort, leaves near-first each against the running best (a leaf's
-// minimum replaces the best when strictly smaller, as visit_leaf's strict per-triangle updates
-// do), internal children pushed far-to-near.  Distances, records and statuses are therefore those
-// of distance_traverse bit for bit; the speculative leaf work only costs lanes that would
-// otherwise idle.  The stack is the quad's column of an LDS array (entry e at stack[e * stride]),
-// written with the same value by all four lanes.
-template <int StackCap>
-__device__ inline int distance_quad_traverse(
-    distance_scene const &sc, int j, float x, float y, float z, float &best, std::uint32_t &best_rec,
-    std::uint32_t *stack, int stride
-) {
-    int sp = 0;
-    int status = k_dist_done;
-    std::uint64_t reference = sc.root_ref;
-    while (reference != 0 && status == k_dist_done) {
-        std::uint64_t next = 0;
-        if (ref_leaf(reference)) {
-            if (!visit_leaf(sc.tris, sc.nt, reference, x, y, z, best, &best_rec))
-                status = k_dist_zero;
-        } else if (ref_internal(reference) && ref_offset(reference) < sc.node_count) {
-            bvh_child const ch = sc.nodes[ref_offset(reference)].children[j];
-            float const d2 = box_distance2(x, y, z, ch.bounds);
-            float lmin = INFINITY;
-            std::uint32_t lrec = k_nearest_none;
-            if (ref_valid(ch.reference) && d2 < best && ref_leaf(ch.reference))
-                visit_leaf(sc.tris, sc.nt, ch.reference, x, y, z, lmin, &lrec);
-            std::uint32_t const d_bits = __float_as_uint(d2), m_bits = __float_as_uint(lmin);
-            std::uint32_t const r_lo = static_cast<std::uint32_t>(ch.reference);
-            std::uint32_t const r_hi = static_cast<std::uint32_t>(ch.reference >> 32);
-            float sd[4], sm[4];
-            std::uint64_t sr[4];
-            std::uint32_t sq[4];
-#define GWN_QUAD_TAKE(S)                                                                               \
-    sd[S] = __uint_as_float(quad_bcast<S>(d_bits));                                                     \
-    sm[S] = __uint_as_float(quad_bcast<S>(m_bits));                                                     \
-    sr[S] = (static_cast<std::uint64_t>(quad_bcast<S>(r_hi)) << 32) | quad_bcast<S>(r_lo);              \
-    sq[S] = quad_bcast<S>(lrec)
-            GWN_QUAD_TAKE(0);
-            GWN_QUAD_TAKE(1);
-            GWN_QUAD_TAKE(2);
-            GWN_QUAD_TAKE(3);
-#undef GWN_QUAD_TAKE
-            // Compaction of the surviving slots in slot order, as selects on each slot's prefix
-            // position (no dynamically indexed arrays, which would live in scratch memory).
-            float cd[4] = {INFINITY, INFINITY, INFINITY, INFINITY}, cm[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
-            std::uint64_t cr[4] = {0, 0, 0, 0};
-            std::uint32_t cq[4] = {k_nearest_none, k_nearest_none, k_nearest_none, k_nearest_none};
-            int m = 0;
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                bool const pass = ref_valid(sr[s]) && !(sd[s] >= best);
-#pragma unroll
-                for (int t = 0; t <= s; ++t) {
-                    if (pass && m == t) {
-                        cd[t] = sd[s];
-                        cr[t] = sr[s];
-                        cm[t] = sm[s];
-                        cq[t] = sq[s];
-                    }
-                }
-                m += pass ? 1 : 0;
-            }
-            auto cswap = [&](int a, int b) {
-                if (!(cd[a] > cd[b]))
-                    return;
-                float const td = cd[a];
-                cd[a] = cd[b];
-                cd[b] = td;
-                std::uint64_t const tr = cr[a];
-                cr[a] = cr[b];
-                cr[b] = tr;
-                float const tm = cm[a];
-                cm[a] = cm[b];
-                cm[b] = tm;
-                std::uint32_t const tq = cq[a];
-                cq[a] = cq[b];
-                cq[b] = tq;
-            };
-            cswap(0, 1);
-            cswap(2, 3);
-            cswap(0, 2);
-            cswap(1, 3);
-            cswap(1, 2);
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                if (status != k_dist_done || s >= m || !ref_leaf(cr[s]) || !(cd[s] < best))
-                    continue;
-                if (cm[s] < best) {
-                    best = cm[s];
-                    best_rec = cq[s];
-                }
-                if (!(best > 0.0f))
-                    status = k_dist_zero;
-            }
-#pragma unroll
-            for (int s = 3; s >= 0; --s) {
-                if (status != k_dist_done || s >= m || !ref_internal(cr[s]) || cd[s] >= best)
-                    continue;
-                if (next != 0) {
-                    if (sp < StackCap)
-                        stack[(sp++) * stride] = static_cast<std::uint32_t>(ref_offset(next));
-                    else
-                        status = k_dist_overflow;
-                }
-                next = cr[s];
-            }
-        }
-        if (next == 0 && sp > 0)
-            next = encode_internal(stack[(--sp) * stride]);
-        reference = next;
-    }
-    return status;
+// The other lane's value: quad_perm [1, 0, 3, 2] and [2, 3, 0, 1].
+__device__ inline std::uint32_t quad_swap1(std::uint32_t v) {
+    return static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xb1, 0xf, 0xf, false));
+}
+__device__ inline std::uint32_t quad_swap2(std::uint32_t v) {
+    return static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4e, 0xf, 0xf, false));
+}
+__device__ inline std::uint32_t quad_or(std::uint32_t v) {
+    v |= quad_swap1(v);
+    return v | quad_swap2(v);
+}
+__device__ inline float quad_min(float v) {  // no NaN
+    v = fminf(v, __uint_as_float(quad_swap1(__float_as_uint(v))));
+    return fminf(v, __uint_as_float(quad_swap2(__float_as_uint(v))));
+}
+__device__ inline std::uint32_t quad_min(std::uint32_t v) {
+    v = min(v, quad_swap1(v));
+    return min(v, quad_swap2(v));
 }
 
-// Four lanes per point (distance_quad_traverse); the grid covers 4 n lanes and whole quads exit
-// together.
-template <int StackCap>
+// Over the 16 lanes of a row: row_half_mirror joins quads 0-1 and 2-3, row_mirror the two halves.
+__device__ inline std::uint32_t row_or(std::uint32_t v) {
+    v = quad_or(v);
+    v |= static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xf, 0xf, false));
+    return v | static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xf, 0xf, false));
+}
+__device__ inline std::uint32_t row_min(std::uint32_t v) {
+    v = quad_min(v);
+    v = min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xf, 0xf, false)));
+    return min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xf, 0xf, false)));
+}
+
+// box_distance2 for a child's box (min <= max): at most one of the two excesses of an axis is positive,
+// so their sum is the larger of them and zero.
+__device__ inline float child_box_distance2(float x, float y, float z, aabb const &b) {
+    float const dx = fmaxf(fmaxf(b.min_x - x, x - b.max_x), 0.0f);
+    float const dy = fmaxf(fmaxf(b.min_y - y, y - b.max_y), 0.0f);
+    float const dz = fmaxf(fmaxf(b.min_z - z, z - b.max_z), 0.0f);
+    return dx * dx + dy * dy + dz * dz;
+}
+
+// point_triangle_distance2 of a record without branches: the region (vertex, edge or face) is decided
+// by the same comparisons in the same order, one quotient serves every region, and the closest point is
+// formed by the region's own operations, so the result is the same bits.  64 lanes over 16 points meet
+// every region, and the branched form then runs all of them one after the other with four quotients.
+__device__ inline float record_distance2(tri_record const &t, float px, float py, float pz) {
+    float const ax = t.v0x, ay = t.v0y, az = t.v0z;
+    float const bx = t.v0x + (t.v1x - t.v0x), by = t.v0y + (t.v1y - t.v0y), bz = t.v0z + (t.v1z - t.v0z);
+    float const cx = t.v0x + (t.v2x - t.v0x), cy = t.v0y + (t.v2y - t.v0y), cz = t.v0z + (t.v2z - t.v0z);
+    float const abx = bx - ax, aby = by - ay, abz = bz - az;
+    float const acx = cx - ax, acy = cy - ay, acz = cz - az;
+    float const apx = px - ax, apy = py - ay, apz = pz - az;
+    float const bpx = px - bx, bpy = py - by, bpz = pz - bz;
+    float const cpx = px - cx, cpy = py - cy, cpz = pz - cz;
+    float const d1 = dot3(abx, aby, abz, apx, apy, apz), d2 = dot3(acx, acy, acz, apx, apy, apz);
+    float const d3 = dot3(abx, aby, abz, bpx, bpy, bpz), d4 = dot3(acx, acy, acz, bpx, bpy, bpz);
+    float const d5 = dot3(abx, aby, abz, cpx, cpy, cpz), d6 = dot3(acx, acy, acz, cpx, cpy, cpz);
+    float const vc = d1 * d4 - d3 * d2, vb = d5 * d2 - d1 * d6, va = d3 * d6 - d5 * d4;
+    float const d43 = d4 - d3, d56 = d5 - d6;
+    bool const at_a = d1 <= 0.0f && d2 <= 0.0f;
+    bool const at_b = !at_a && d3 >= 0.0f && d4 <= d3;
+    bool const on_ab = !at_a && !at_b && vc <= 0.0f && d1 >= 0.0f && d3 <= 0.0f;
+    bool const at_c = !at_a && !at_b && !on_ab && d6 >= 0.0f && d5 <= d6;
+    bool const before = at_a || at_b || on_ab || at_c;
+    bool const on_ac = !before && vb <= 0.0f && d2 >= 0.0f && d6 <= 0.0f;
+    bool const on_bc = !before && !on_ac && va <= 0.0f && d43 >= 0.0f && d56 >= 0.0f;
+    bool const edge = on_ab || on_ac || on_bc;
+    bool const vertex = at_a || at_b || at_c;
+    float const num = on_ab ? d1 : (on_ac ? d2 : (on_bc ? d43 : 1.0f));
+    float const den = on_ab ? d1 - d3 : (on_ac ? d2 - d6 : (on_bc ? d43 + d56 : va + vb + vc));
+    float const quo = num / den;
+    // Edges: base + quo * e; face: (a + (vb quo) ab) + (vc quo) ac.
+    float const s = edge ? quo : vb * quo;
+    bool const base_b = at_b || on_bc;
+    float const ox = at_c ? cx : (base_b ? bx : ax), oy = at_c ? cy : (base_b ? by : ay),
+                oz = at_c ? cz : (base_b ? bz : az);
+    float const ex = on_bc ? cx - bx : (on_ac ? acx : abx), ey = on_bc ? cy - by : (on_ac ? acy : aby),
+                ez = on_bc ? cz - bz : (on_ac ? acz : abz);
+    float const w = vc * quo;
+    float const hx = ox + s * ex, hy = oy + s * ey, hz = oz + s * ez;
+    float const fx = hx + w * acx, fy = hy + w * acy, fz = hz + w * acz;
+    float const rx = px - (vertex ? ox : (edge ? hx : fx)), ry = py - (vertex ? oy : (edge ? hy : fy)),
+                rz = pz - (vertex ? oz : (edge ? hz : fz));
+    return dot3(rx, ry, rz, rx, ry, rz);
+}
+
+// Slot lists of the 16 passing masks: bits 2t..2t+1 hold the t-th slot, the passing ones first, each
+// kind in slot order.
+constexpr std::uint32_t quad_slots(std::uint32_t mask) {
+    std::uint32_t list = 0, t = 0;
+    for (int pass = 1; pass >= 0; --pass)
+        for (std::uint32_t s = 0; s < 4; ++s)
+            if (static_cast<int>((mask >> s) & 1u) == pass)
+                list |= s << (2 * t++);
+    return list;
+}
+constexpr std::uint32_t quad_slots4(std::uint32_t first) {
+    return quad_slots(first) | (quad_slots(first + 1) << 8) | (quad_slots(first + 2) << 16) | (quad_slots(first + 3) << 24);
+}
+
+// By value: through a closure's references the selects became indexed scratch loads.
+__device__ inline float pick4(std::uint32_t i, float k0, float k1, float k2, float k3) {
+    float const a = i & 1u ? k1 : k0;
+    float const b = i & 1u ? k3 : k2;
+    return i & 2u ? b : a;
+}
+__device__ inline void compare_swap(float &a, float &b, std::uint32_t &ia, std::uint32_t &ib) {
+    bool const gt = a > b;
+    float const ka = gt ? b : a, kb = gt ? a : b;
+    std::uint32_t const xa = gt ? ib : ia, xb = gt ? ia : ib;
+    a = ka;
+    b = kb;
+    ia = xa;
+    ib = xb;
+}
+
+// Position of this lane's slot in distance_traverse's near-first order of a node's surviving children
+// (those past the survivors are in no order).  `d` is the lane's box distance, `mask` the quad's
+// surviving slots.  Distinct distances have one order; with equal ones (or NaN) anywhere in the wave it
+// is that of the compaction in slot order and the five-comparator network, which is not stable, run on
+// (distance, slot) pairs.
+// `ties`: the wave's lanes that share a distance with another survivor of their node.
+__device__ inline std::uint32_t near_first_position(
+    float d, bool pass, std::uint32_t mask, std::uint32_t j, std::uint64_t &ties
+) {
+    float const k = pass ? d : INFINITY;
+    std::uint32_t const kb = __float_as_uint(k);
+    float const n1 = __uint_as_float(quad_swap1(kb)), n2 = __uint_as_float(quad_swap2(kb));
+    float const n3 = __uint_as_float(quad_swap2(quad_swap1(kb)));
+    bool const apart = (n1 < k || n1 > k) && (n2 < k || n2 > k) && (n3 < k || n3 > k);
+    std::uint32_t pos = (n1 < k ? 1u : 0u) + (n2 < k ? 1u : 0u) + (n3 < k ? 1u : 0u);
+    ties = __ballot(pass && !apart);
+    if (ties != 0ull) {
+        float const k0 = __uint_as_float(quad_bcast<0>(kb)), k1 = __uint_as_float(quad_bcast<1>(kb)),
+                    k2 = __uint_as_float(quad_bcast<2>(kb)), k3 = __uint_as_float(quad_bcast<3>(kb));
+        std::uint32_t const lo = mask & 4u ? quad_slots4(4) : quad_slots4(0);
+        std::uint32_t const hi = mask & 4u ? quad_slots4(12) : quad_slots4(8);
+        std::uint32_t const list = (mask & 8u ? hi : lo) >> ((mask & 3u) * 8u);
+        std::uint32_t i0 = list & 3u, i1 = (list >> 2) & 3u, i2 = (list >> 4) & 3u, i3 = (list >> 6) & 3u;
+        float c0 = pick4(i0, k0, k1, k2, k3), c1 = pick4(i1, k0, k1, k2, k3), c2 = pick4(i2, k0, k1, k2, k3),
+              c3 = pick4(i3, k0, k1, k2, k3);
+        compare_swap(c0, c1, i0, i1);
+        compare_swap(c2, c3, i2, i3);
+        compare_swap(c0, c2, i0, i2);
+        compare_swap(c1, c3, i1, i3);
+        compare_swap(c1, c2, i1, i2);
+        pos = i0 == j ? 0u : (i1 == j ? 1u : (i2 == j ? 2u : 3u));
+    }
+    return pos;
+}
+
+constexpr int k_stack_stride = k_block / 4 + 1;  // entry e of quad k's stack at [e * k_stack_stride + k]
+
+// The rest of a point's traversal with a row of 16 lanes: quad g of the row tests the g-th entry from the
+// top of the stack.  Entries are settled in stack order up to the first whose node has internal children
+// to enter; those are pushed, and what the quads behind it found is dropped (their entries stay on the
+// stack).  So the nodes, and the leaves of each, take effect in the quad traversal's order; an entry
+// excluded by a leaf of one before it needs no undoing, as none of its leaves is below the best then (the
+// rounding case goes leaf by leaf).  The order among equal box distances depends on which children
+// survive, so an entry with such children waits until it is the top one and the best is settled.  A long
+// traversal is mostly nodes with only leaves near its best
+// distance, of which this settles up to four at a time.
+template <int StackCap, bool WantRec, class Finish>
+__device__ inline void distance_row_tail(
+    distance_scene const &sc, bool alive, std::size_t q, float x, float y, float z, float best, std::uint32_t rec,
+    int sp, std::uint32_t *st_node, float *st_dist, Finish const &finish
+) {
+    std::uint32_t const lane = threadIdx.x & 63u;
+    std::uint32_t const j = lane & 3u;
+    std::uint32_t const g = (lane >> 2) & 3u;
+    std::uint32_t const shift = lane & 60u, row_shift = lane & 48u;
+    bool held = false;      // `slot` is this lane's child of the quad's entry
+    float entry_d = 0.0f;
+    bvh_child slot{};
+    auto const fetch = [&] {
+        int const e = sp - 1 - static_cast<int>(g);
+        held = e >= 0;
+        if (held) {
+            entry_d = st_dist[e * k_stack_stride];
+            held = !(entry_d >= best);
+            if (held)
+                slot = sc.nodes[st_node[e * k_stack_stride]].children[j];
+        }
+    };
+    if (alive)
+        fetch();
+    while (__ballot(alive) != 0ull) {
+        if (alive) {
+            int status = k_dist_done;
+            bool const test = held && !(entry_d >= best);
+            float const node_d = entry_d;
+            float const d = child_box_distance2(x, y, z, slot.bounds);
+            bool const pass = test && ref_valid(slot.reference) && !(d >= best);
+            bool const inner = pass && ref_internal(slot.reference);
+            std::uint32_t const mask = static_cast<std::uint32_t>(__ballot(pass) >> shift) & 15u;
+            std::uint64_t ties;
+            std::uint32_t const pos = near_first_position(d, pass, mask, j, ties);
+            std::uint32_t const inners = static_cast<std::uint32_t>(__ballot(inner) >> row_shift) & 0xffffu;
+            std::uint32_t last = inners != 0u ? static_cast<std::uint32_t>(__builtin_ctz(inners)) >> 2 : 3u;
+            std::uint32_t const tied = static_cast<std::uint32_t>(ties >> row_shift) & 0xfff0u;
+            if (tied != 0u)
+                last = min(last, (static_cast<std::uint32_t>(__builtin_ctz(tied)) >> 2) - 1u);
+            bool const enter = inner && g == last;
+            bool const leaf = pass && g <= last && ref_leaf(slot.reference) && d < best && ref_offset(slot.reference) < sc.nt;
+            std::uint32_t const child = static_cast<std::uint32_t>(ref_offset(slot.reference));
+            bool const many = leaf && ref_count(slot.reference) > 1u;
+            std::uint64_t const leaf_ref = slot.reference;
+            tri_record t{};
+            if (leaf)
+                t = sc.tris[child];
+            sp = sp > static_cast<int>(last) + 1 ? sp - static_cast<int>(last) - 1 : 0;
+            std::uint32_t const at = row_or(enter ? 1u << pos : 0u);
+            int const count = __popc(at);
+            int const to = sp + count - 1 - __popc(at & ((1u << pos) - 1u));
+            if (enter && to <= StackCap) {
+                st_node[to * k_stack_stride] = child;
+                st_dist[to * k_stack_stride] = d;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            sp += count;
+            if (sp > StackCap + 1)
+                status = k_dist_overflow;
+            else
+                fetch();  // requested before the leaf triangles are evaluated
+            if (__ballot(leaf) != 0ull) {
+                float cm = INFINITY;
+                std::uint32_t crec = child;
+                float const td = record_distance2(t, x, y, z);
+                if (leaf && td < cm)
+                    cm = td;
+                if (many) {
+                    cm = INFINITY;
+                    visit_leaf(sc.tris, sc.nt, leaf_ref, x, y, z, cm, &crec);
+                }
+                if (__ballot(leaf && cm < d) != 0ull) {
+                    for (std::uint32_t k = 0; k < 16; ++k) {
+                        bool const take = leaf && g * 4 + pos == k && !(node_d >= best) && d < best && cm < best;
+                        if (row_or(take ? 1u : 0u) != 0u) {
+                            best = __uint_as_float(row_or(take ? __float_as_uint(cm) : 0u));
+                            if constexpr (WantRec)
+                                rec = row_or(take ? crec : 0u);
+                        }
+                    }
+                } else {
+                    float const m = __uint_as_float(row_min(__float_as_uint(cm)));  // not negative
+                    if (m < best) {
+                        best = m;
+                        if constexpr (WantRec) {
+                            std::uint32_t const first = cm == m ? g * 4 + pos : 16u;
+                            rec = row_or(first == row_min(first) ? crec : 0u);
+                        }
+                    }
+                }
+                if (!(best > 0.0f) && status == k_dist_done)
+                    status = k_dist_zero;
+            }
+            if (sp == 0 || status != k_dist_done) {
+                alive = false;
+                if ((lane & 15u) == 0u) {
+                    float const p[3] = {x, y, z};
+                    finish(q, status, best, rec, p);
+                }
+            }
+        }
+    }
+}
+
+// Quad form of distance_traverse: four lanes per point, lane j of the quad owning child slot j of
+// each node, with distances, nearest records (kept where WantRec) and statuses equal to
+// distance_traverse's bit for bit.  Lane j computes its child's box distance and, for a surviving
+// leaf child, its triangle's distance (which does not depend on the best found before it); the quad
+// then takes distance_traverse's steps together:
+//   - leaves, near first, each against the running best.  A leaf distance below its box's is a rounding
+//     case that needs the order; without one in the wave the smallest distance wins, and among equal
+//     ones the first in order, whichever leaves the running best would have skipped;
+//   - internal children far to near onto the stack (the quad's column of an LDS array), the nearest
+//     entered.  The stack keeps each entry's box distance, and an entry no closer than the best is
+//     dropped when popped: its children's boxes lie inside its own, and every operation of
+//     box_distance2 is monotone in the bounds, so none of them would have survived.  So children can be
+//     pushed before the node's leaves are evaluated, and the next node's read overlaps them.
+// Each wave hands its next point to a quad that has finished: queries' work spreads over two orders of
+// magnitude (240 nodes on average, 7,000 at most, on the 1M-triangle mesh), and a wave of 16 fixed points
+// lasts as long as its longest.  A wave's points are runs of 4 neighbours from places spread over the
+// whole visiting order, since the long ones lie together (1M points of 1M triangles: 14.3 ms, runs of 16
+// 16.8 ms, all of a wave's points in a row 42 ms).
+// When a wave has no further point to hand out and at most four left, each of them gets a row of 16
+// lanes (distance_row_tail).  A batch of no more points than the grid has rows starts that way.
+//
+// VALU bound from some million points on (84 % of the issue slots at 4M), below that by the instructions
+// of the longest point's chain.  Measured against 16 fixed points a wave with the box of every popped node
+// tested: 1,000 points of 5,120 triangles 653 -> 160 us; of 1,048,576 8.4 -> 1.8 ms; 1,000,003 of
+// 1,048,576 28.5 -> 14.3 ms; 4,000,000 55 -> 41 ms.
+//
+// `finish(q, status, best, rec, point)` is called by one lane per point.
+template <int StackCap, bool WantRec, class Finish>
+__device__ inline void distance_quad_range(
+    distance_scene const &sc, float const *__restrict__ qx, float const *__restrict__ qy,
+    float const *__restrict__ qz, std::uint32_t const *__restrict__ order, std::size_t n, float best0,
+    std::uint32_t *s_node, float *s_dist, Finish const &finish
+) {
+    constexpr int k_stride = k_stack_stride;
+    std::uint32_t const lane = threadIdx.x & 63u;
+    std::uint32_t const j = lane & 3u;
+    std::uint32_t const shift = lane & 60u;
+    std::uint32_t *const st_node = s_node + (threadIdx.x >> 2);
+    float *const st_dist = s_dist + (threadIdx.x >> 2);
+    // The wave's t-th point: 4 consecutive ones of the visiting order, then 4 one grid further on.
+    std::size_t const wave = static_cast<std::size_t>(blockIdx.x) * (k_block / 64) + (threadIdx.x >> 6);
+    std::size_t const waves = static_cast<std::size_t>(gridDim.x) * (k_block / 64);
+    auto const point = [=](std::size_t t) { return ((t >> 2) * waves + wave) * 4 + (t & 3); };
+    bool const rows = n <= waves * 4;  // a row per point from the start
+    if (!ref_internal(sc.root_ref)) {  // a leaf (or nothing) for a root: one lane per point
+        for (std::size_t i = wave * 64 + lane; i < n; i += waves * 64) {
+            std::size_t const q = order ? order[i] : i;
+            float const p[3] = {qx[q], qy[q], qz[q]};
+            float best = best0;
+            std::uint32_t rec = k_nearest_none;
+            int const status = ref_leaf(sc.root_ref) &&
+                                       !visit_leaf(sc.tris, sc.nt, sc.root_ref, p[0], p[1], p[2], best, &rec)
+                                   ? k_dist_zero
+                                   : k_dist_done;
+            finish(q, status, best, rec, p);
+        }
+        return;
+    }
+    std::size_t taken = 16;  // points handed out so far, wave-uniform
+    std::size_t i = rows ? ((lane & 12u) == 0u ? wave * 4 + (lane >> 4) : n) : point(lane >> 2);
+    bool live = i < n;
+    bool more = !rows;  // the wave may have further points
+    std::size_t q = 0;
+    float x = 0.0f, y = 0.0f, z = 0.0f, best = best0;
+    std::uint32_t rec = k_nearest_none;
+    int sp = 0;
+    bvh_child slot{};            // this lane's child of `node`
+    std::uint32_t node = 0;
+    float node_d = 0.0f;         // the box distance it was entered with
+    std::uint32_t const root = static_cast<std::uint32_t>(ref_offset(sc.root_ref));
+    auto const begin_point = [&] {
+        q = order ? order[i] : i;
+        x = qx[q];
+        y = qy[q];
+        z = qz[q];
+        best = best0;
+        rec = k_nearest_none;
+        sp = 0;
+        node = root;
+        node_d = -1.0f;
+        slot = sc.nodes[root].children[j];
+    };
+    if (live)
+        begin_point();
+    for (;;) {
+        std::uint64_t const alive = __ballot(live);
+        if (alive == 0ull)
+            return;
+        if (!more && __popcll(alive) <= 16)
+            break;
+        bool finished = false;
+        int status = k_dist_done;
+        if (live) {
+            float const d = child_box_distance2(x, y, z, slot.bounds);
+            bool const pass = ref_valid(slot.reference) && !(d >= best);
+            bool const leaf = pass && ref_leaf(slot.reference) && d < best && ref_offset(slot.reference) < sc.nt;
+            bool const enter = pass && ref_internal(slot.reference);
+            std::uint32_t const child = static_cast<std::uint32_t>(ref_offset(slot.reference));
+            tri_record t{};
+            if (leaf)
+                t = sc.tris[child];
+            std::uint32_t const mask = static_cast<std::uint32_t>(__ballot(pass) >> shift) & 15u;
+            std::uint64_t ties;
+            std::uint32_t const pos = near_first_position(d, pass, mask, j, ties);
+            // Internal children far to near onto the stack, the nearest next.
+            std::uint32_t const at = quad_or(enter ? 1u << pos : 0u);
+            int const count = __popc(at);
+            int const rank = __popc(at & ((1u << pos) - 1u));
+            std::uint32_t next = quad_or(enter && rank == 0 ? child : 0u);
+            float next_d = __uint_as_float(quad_or(enter && rank == 0 ? __float_as_uint(d) : 0u));
+            int const to = sp + count - 1 - rank;
+            if (enter && rank > 0 && to < StackCap) {
+                st_node[to * k_stride] = child;
+                st_dist[to * k_stride] = d;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            bool found = count > 0;
+            if (found) {
+                sp += count - 1;
+                status = sp > StackCap ? k_dist_overflow : k_dist_done;
+            }
+            // The nearest stack entry that the best does not exclude, four at a time.
+            auto const pop = [&] {
+                while (!found && sp > 0) {
+                    int const e = sp - 1 - static_cast<int>(j);
+                    float const ed = e >= 0 ? st_dist[e * k_stride] : 0.0f;
+                    std::uint32_t const en = e >= 0 ? st_node[e * k_stride] : 0u;
+                    std::uint32_t const keep = static_cast<std::uint32_t>(__ballot(e >= 0 && !(ed >= best)) >> shift) & 15u;
+                    if (keep != 0u) {
+                        std::uint32_t const top = static_cast<std::uint32_t>(__builtin_ctz(keep));
+                        next = quad_or(j == top ? en : 0u);
+                        next_d = __uint_as_float(quad_or(j == top ? __float_as_uint(ed) : 0u));
+                        sp -= static_cast<int>(top) + 1;
+                        found = true;
+                    } else {
+                        sp = sp > 4 ? sp - 4 : 0;
+                    }
+                }
+            };
+            if (status == k_dist_done)
+                pop();
+            // The next node is requested before the leaf triangles are evaluated, and given up if they
+            // bring the best below its box.
+            bvh_child ahead = slot;
+            if (found && status == k_dist_done)
+                ahead = sc.nodes[next].children[j];
+            if (__ballot(leaf) != 0ull) {
+                float cm = INFINITY;
+                std::uint32_t crec = child;
+                float const td = record_distance2(t, x, y, z);
+                if (leaf && td < cm)
+                    cm = td;
+                if (leaf && ref_count(slot.reference) > 1u) {
+                    cm = INFINITY;
+                    visit_leaf(sc.tris, sc.nt, slot.reference, x, y, z, cm, &crec);
+                }
+                if (__ballot(leaf && cm < d) != 0ull) {
+                    for (std::uint32_t s = 0; s < 4; ++s) {
+                        bool const take = leaf && pos == s && d < best && cm < best;
+                        if (quad_or(take ? 1u : 0u) != 0u) {
+                            best = __uint_as_float(quad_or(take ? __float_as_uint(cm) : 0u));
+                            if constexpr (WantRec)
+                                rec = quad_or(take ? crec : 0u);
+                            if (!(best > 0.0f) && status == k_dist_done)
+                                status = k_dist_zero;
+                        }
+                    }
+                } else {
+                    float const m = quad_min(cm);
+                    if (m < best) {
+                        best = m;
+                        if constexpr (WantRec) {
+                            std::uint32_t const first = cm == m ? pos : 4u;
+                            rec = quad_or(first == quad_min(first) ? crec : 0u);
+                        }
+                        if (!(best > 0.0f) && status == k_dist_done)
+                            status = k_dist_zero;
+                    }
+                }
+                if (found && next_d >= best && status == k_dist_done) {
+                    found = false;
+                    pop();
+                    if (found)
+                        ahead = sc.nodes[next].children[j];
+                }
+            }
+            slot = ahead;
+            node = next;
+            node_d = next_d;
+            finished = !found || status != k_dist_done;
+        }
+        std::uint64_t const ended = __ballot(finished);
+        if (ended != 0ull) {
+            if (finished) {
+                if (j == 0u) {
+                    float const p[3] = {x, y, z};
+                    finish(q, status, best, rec, p);
+                }
+                i = point(taken + static_cast<std::size_t>(__popcll(ended & ((1ull << shift) - 1ull)) >> 2));
+                live = i < n;
+                if (live)
+                    begin_point();
+            }
+            taken += static_cast<std::size_t>(__popcll(ended) >> 2);
+            more = more && __ballot(finished && !live) == 0ull;
+        }
+    }
+    // The k-th point left goes to row k, its next node on top of its stack.
+    if (live && j == 0u) {
+        st_node[sp * k_stride] = node;
+        st_dist[sp * k_stride] = node_d;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    std::uint64_t left = __ballot(live) & 0x1111111111111111ull;
+    for (std::uint32_t k = 0; k < 3; ++k)
+        left = k < (lane >> 4) ? left & (left - 1ull) : left;
+    bool const has = left != 0ull;
+    int const from = has ? static_cast<int>(__builtin_ctzll(left)) : static_cast<int>(lane);
+    distance_row_tail<StackCap, WantRec>(
+        sc, has, static_cast<std::size_t>(__shfl(static_cast<unsigned long long>(q), from)), __shfl(x, from),
+        __shfl(y, from), __shfl(z, from), __shfl(best, from), static_cast<std::uint32_t>(__shfl(static_cast<int>(rec), from)),
+        __shfl(sp, from) + 1, s_node + (threadIdx.x >> 6) * 16 + (from >> 2), s_dist + (threadIdx.x >> 6) * 16 + (from >> 2),
+        finish);
+}
+
+// Up to this many points every point has a row of 16 lanes from the start: their rows hardly fill the
+// chip, and the batch lasts as long as its longest point.  Measured, a row per point against a quad per
+// point: 65,536 points of 1,048,576 triangles 3.6 / 7.9 ms, 262,144 6.1 / 10.0 ms, of 131,072 2.3 / 3.6 ms;
+// 1,000,000 points of 1,048,576 15.4 / 14.3 ms, of 5,120 1.7 / 1.3 ms.
+constexpr std::size_t k_row_points = std::size_t(1) << 18;
+
+// Blocks of the quad traversal.  A quad per point: two waves for each of the 8,192 that fit the chip
+// (half or twice as many measured 5-25 % slower from 1M points on).
+inline unsigned distance_quad_grid(std::size_t n) {
+    return n <= k_row_points ? grid_for(16 * n, k_block) : std::min(grid_for(4 * n, k_block), 4096u);
+}
+
+template <int StackCap, bool WantRec>
 __global__ __launch_bounds__(k_block) void distance_quad_kernel(
     distance_scene sc, float const *__restrict__ qx, float const *__restrict__ qy, float const *__restrict__ qz,
     std::uint32_t const *__restrict__ order, float *__restrict__ out, std::size_t n, float culling_band,
     std::uint32_t *__restrict__ nearest
 ) {
-    constexpr int k_quads = k_block / 4;
-    __shared__ std::uint32_t s_stack[StackCap * k_quads];  // entry e of quad k at [e * k_quads + k]
-    std::size_t const i = (static_cast<std::size_t>(blockIdx.x) * k_block + threadIdx.x) >> 2;
-    if (i >= n)
-        return;
-    int const j = static_cast<int>(threadIdx.x & 3);
-    std::size_t const q = order ? order[i] : i;
+    __shared__ std::uint32_t s_node[(StackCap + 1) * k_stack_stride];
+    __shared__ float s_dist[(StackCap + 1) * k_stack_stride];
     float const band = culling_band < 0.0f ? 0.0f : culling_band;
-    float best = band * band;
-    std::uint32_t rec = k_nearest_none;
-    int const st = distance_quad_traverse<StackCap>(sc, j, qx[q], qy[q], qz[q], best, rec,
-                                                    s_stack + (threadIdx.x >> 2), k_quads);
-    if (j == 0) {
-        out[q] = st == k_dist_zero ? 0.0f : (st == k_dist_overflow ? __builtin_nanf("") : sqrtf(best));
-        if (nearest != nullptr)
-            nearest[q] = nearest_code(st, rec);
-    }
+    distance_quad_range<StackCap, WantRec>(
+        sc, qx, qy, qz, order, n, band * band, s_node, s_dist,
+        [&](std::size_t q, int st, float best, std::uint32_t rec, float const (&)[3]) {
+            out[q] = st == k_dist_zero ? 0.0f : (st == k_dist_overflow ? __builtin_nanf("") : sqrtf(best));
+            if constexpr (WantRec)
+                nearest[q] = nearest_code(st, rec);
+        });
 }
 
 template <int StackCap>
@@ -424,28 +802,21 @@ __device__ inline void distance_adjoint_finish(
 template <int StackCap>
 __global__ __launch_bounds__(k_block) void distance_adjoint_kernel(
     distance_scene sc, float const *__restrict__ px, float const *__restrict__ py, float const *__restrict__ pz,
-    float const *__restrict__ u, std::uint32_t const *__restrict__ order, std::size_t n, float culling_band,
-    std::uint32_t const *__restrict__ prim, std::uint32_t const *__restrict__ i0, std::uint32_t const *__restrict__ i1,
+    float const *__restrict__ u, std::uint32_t const *__restrict__ order, std::size_t n,
+    float culling_band, std::uint32_t const *__restrict__ prim, std::uint32_t const *__restrict__ i0, std::uint32_t const *__restrict__ i1,
     std::uint32_t const *__restrict__ i2, float *dvx, float *dvy, float *dvz, float *__restrict__ dpx,
     float *__restrict__ dpy, float *__restrict__ dpz
 ) {
-    // Four lanes per point (distance_quad_traverse: the nearest record of distance_traverse); the
-    // quad's first lane finishes the point.  The grid covers 4 n lanes.
-    constexpr int k_quads = k_block / 4;
-    __shared__ std::uint32_t s_stack[StackCap * k_quads];
-    std::size_t const i = (static_cast<std::size_t>(blockIdx.x) * k_block + threadIdx.x) >> 2;
-    if (i >= n)
-        return;
-    int const j = static_cast<int>(threadIdx.x & 3);
-    std::size_t const q = order ? order[i] : i;
-    float const p[3] = {px[q], py[q], pz[q]};
+    // Four lanes per point (the nearest record of distance_traverse); the quad's first lane finishes
+    // the point.
+    __shared__ std::uint32_t s_node[(StackCap + 1) * k_stack_stride];
+    __shared__ float s_dist[(StackCap + 1) * k_stack_stride];
     float const band = culling_band < 0.0f ? 0.0f : culling_band;
-    float best = band * band;
-    std::uint32_t rec = 0xffffffffu;
-    int const st = distance_quad_traverse<StackCap>(sc, j, p[0], p[1], p[2], best, rec,
-                                                    s_stack + (threadIdx.x >> 2), k_quads);
-    if (j == 0)
-        distance_adjoint_finish(sc, p, q, st, rec, u[q], prim, i0, i1, i2, dvx, dvy, dvz, dpx, dpy, dpz);
+    distance_quad_range<StackCap, true>(
+        sc, px, py, pz, order, n, band * band, s_node, s_dist,
+        [&](std::size_t q, int st, float, std::uint32_t rec, float const (&p)[3]) {
+            distance_adjoint_finish(sc, p, q, st, rec, u[q], prim, i0, i1, i2, dvx, dvy, dvz, dpx, dpy, dpz);
+        });
 }
 
 
@@ -477,9 +848,12 @@ void launch_distance(
     if (wave && order != nullptr)
         distance_wave_kernel<Cap><<<grid_for(n, k_block), k_block, 0, stream>>>(sc, qx, qy, qz, order, out, n, band,
                                                                                   nearest);
+    else if (quad && nearest != nullptr)
+        distance_quad_kernel<Cap, true><<<distance_quad_grid(n), k_block, 0, stream>>>(
+            sc, qx, qy, qz, order, out, n, band, nearest);
     else if (quad)
-        distance_quad_kernel<Cap><<<grid_for(4 * n, k_block), k_block, 0, stream>>>(sc, qx, qy, qz, order, out, n,
-                                                                                      band, nearest);
+        distance_quad_kernel<Cap, false><<<distance_quad_grid(n), k_block, 0, stream>>>(
+            sc, qx, qy, qz, order, out, n, band, nullptr);
     else
         distance_kernel<Cap><<<grid_for(n, k_block), k_block, 0, stream>>>(sc, qx, qy, qz, order, out, n, band,
                                                                              nearest);
@@ -496,8 +870,7 @@ void unsigned_distance(
         return;
     bool const sort = cfg.sort_queries > 0 || (cfg.sort_queries < 0 && n >= (1u << 16));
     bool const wave = cfg.sort_queries == 2;
-    // Four lanes per point unless one is asked for: the results are the same, and on MI355X the
-    // quad traversal measured 2.2-2.8x faster from 65,536 to 16,777,216 points.
+    // Four lanes per point (or 16, distance_quad_range) unless one is asked for: the results are the same.
     bool const quad = cfg.lanes_per_point != 1;
     device_buffer<std::uint32_t> order;
     if (sort) {
@@ -559,7 +932,7 @@ void unsigned_distance_adjoint(
     distance_scene const sc{bvh.nodes.ptr, bvh.node_count, bvh.triangles.ptr, bvh.triangle_count, bvh.root.reference};
     int const need = static_cast<int>(bvh.internal_stack_bound);
 #define GWN_DADJ(C)                                                                                            \
-    distance_adjoint_kernel<C><<<grid_for(4 * n, k_block), k_block, 0, stream>>>(                             \
+    distance_adjoint_kernel<C><<<distance_quad_grid(n), k_block, 0, stream>>>(                                \
         sc, px, py, pz, u, order.ptr, n, culling_band, bvh.primitive_indices.ptr, g.i0.ptr, g.i1.ptr, g.i2.ptr, \
         dvx, dvy, dvz, dpx, dpy, dpz)
     if (need <= 32)
