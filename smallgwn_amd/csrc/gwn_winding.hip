@@ -7,7 +7,7 @@
 // LDS in 256-record tiles, so every record is read from HBM/L2 once per block and broadcast to
 // all 256 lanes.  VALU bound (solid angle: 3 sqrt, 3 div, 1 atan2 per pair).
 //
-// Taylor batch: four lanes per query, or 64 queries per wave where Hilbert-ordered queries are dense
+// Taylor batch: 16 or four lanes per query, or 64 queries per wave where Hilbert-ordered queries are dense
 // (results are written back in input order).  A stack of internal node ids; the last internal child
 // of a node is entered directly, the others are pushed, leaves are evaluated in slot order --
 // the reference's traversal order, so float sums are formed in the same sequence.  The node
@@ -640,15 +640,6 @@ template <int S, class T> __device__ inline T quad_bcast(T v) {
     }
 }
 
-// Adds the four lanes' terms to a quad's sum in slot order.  A slot without a term holds zero, which
-// leaves every sum it meets as it is (a sum starts at +0 and never becomes -0).
-template <class T> __device__ inline void quad_add(T &sum, T v) {
-    sum += quad_bcast<0>(v);
-    sum += quad_bcast<1>(v);
-    sum += quad_bcast<2>(v);
-    sum += quad_bcast<3>(v);
-}
-
 // What one lane of a quad reads of a node: its slot's reference, acceptance fields and coefficients.
 template <int Order, bool Grad> struct quad_slot {
     static constexpr int k_fields = moment_field_count(Order);
@@ -685,72 +676,126 @@ template <int Order, bool Grad> struct quad_slot {
     }
 };
 
+__device__ inline std::uint32_t quad_sum(std::uint32_t v) {
+    return quad_bcast<0>(v) + quad_bcast<1>(v) + quad_bcast<2>(v) + quad_bcast<3>(v);
+}
+// Over the 16 lanes of a row: row_half_mirror joins quads 0-1 and 2-3, row_mirror the halves.
+__device__ inline std::uint32_t row_sum(std::uint32_t v) {
+    v = quad_sum(v);
+    v += static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xf, 0xf, false));
+    return v + static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xf, 0xf, false));
+}
+
+// Adds the terms of a row's 16 lanes (or a quad's four) to the sum in lane order.
+template <int Lanes> __device__ inline void ordered_add(float &sum, float v) { add_in_lane_order<Lanes>(sum, v); }
+template <int Lanes, int J = 0> __device__ inline void ordered_add(double &sum, double v) {
+    if constexpr (J < Lanes) {
+        constexpr int k_ctrl = Lanes == 4 ? J * 0x55 : 0x150 + J;
+        std::uint64_t const b = __builtin_bit_cast(std::uint64_t, v);
+        std::uint32_t const lo = static_cast<std::uint32_t>(
+            __builtin_amdgcn_update_dpp(0, static_cast<int>(b), k_ctrl, 0xf, 0xf, false));
+        std::uint32_t const hi = static_cast<std::uint32_t>(
+            __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), k_ctrl, 0xf, 0xf, false));
+        sum += __builtin_bit_cast(double, (static_cast<std::uint64_t>(hi) << 32) | lo);
+        ordered_add<Lanes, J + 1>(sum, v);
+    }
+}
+template <int Lanes, int Prec, bool Grad>
+__device__ inline void add_terms(taylor_sums<Prec, Grad> &acc, taylor_sums<Prec, Grad> const &term) {
+    if constexpr (Prec == GWN_PRECISION_PLAIN) {
+        ordered_add<Lanes>(acc.omega, term.omega);
+        if constexpr (Grad) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                ordered_add<Lanes>(acc.gf[k], term.gf[k]);
+        }
+    } else {
+        ordered_add<Lanes>(acc.near, term.near);
+        if constexpr (Grad) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                ordered_add<Lanes>(acc.gd[k], term.gd[k]);
+        }
+    }
+}
+
+// One query's decisions at one child slot.
+template <int Order, bool Grad> struct slot_test {
+    float w;
+    float g[3];
+    bool valid, accepted, leaf, inner;
+
+    __device__ slot_test(quad_slot<Order, Grad> const &slot, float x, float y, float z, float beta2, bool held) {
+        float const qrx = x - slot.cx, qry = y - slot.cy, qrz = z - slot.cz;
+        float const ql2 = squared_norm_unfused(qrx, qry, qrz);
+        bool const far = !(!(ql2 > 0.0f) || ql2 <= product_unfused(slot.mp, beta2));
+        if constexpr (Grad)
+            w = taylor_term<Order, true>(slot.c, 0, qrx, qry, qrz, ql2, g);
+        else
+            w = taylor_value<Order>(slot.c, qrx, qry, qrz, ql2);
+        valid = held && slot.ref != k_invalid;
+        accepted = valid && far && isfinite(w);
+        leaf = valid && !accepted && (slot.ref & k_cref_leaf) != 0u;
+        inner = valid && !accepted && (slot.ref & k_cref_leaf) == 0u;
+    }
+};
+
 // Taylor traversal with four lanes per query, lane j of the quad owning child slot j: the four
 // acceptance tests, expansions and leaf triangles of a node are evaluated side by side and their terms
-// added in slot order (quad_add); descended children are pushed in slot order and the last one entered,
-// as taylor_traverse does.  Decisions, terms and the order of every sum are those of the per-lane
+// added in slot order (add_terms; a slot without a term adds zero, which leaves every sum as it is, since
+// a sum starts at +0 and never becomes -0); descended children are pushed in slot order and the last one
+// entered, as taylor_traverse does.  Decisions, terms and the order of every sum are those of the per-lane
 // traversal, so the results are too, bit for bit.  The stack is the quad's column of an LDS array.
 //
-// Latency bound: a small batch is one chain of dependent node reads per query, so what counts is the
-// reads on the chain.  One lane per query waited for the header, then for each accepted slot's
-// coefficients and each leaf's triangle in turn (about eight waits a node); here a node's header and
-// all four slots' coefficients arrive together, and the next node's are requested as soon as the
-// decisions are known, before the leaf triangles are evaluated.  Measured, per-lane against this form:
-// 1,000 queries of 5,120 triangles (order 1, beta 2) 749 against 153 us.  Holding a quad's leaf triangles
-// back until half of the wave's quads have some (so that they are evaluated with more lanes active)
-// made every size 5-20 % slower.
+// A chain of dependent node reads per query: one lane per query waited for the header, then for each
+// accepted slot's coefficients and each leaf's triangle in turn (about eight waits a node); here a node's
+// header and all four slots' coefficients arrive together, and the next node's are requested as soon as
+// the decisions are known, before the leaf triangles are evaluated.  Measured (sort included), the wave
+// traversal against this form: 500,009 queries of 131,072 triangles (order 2, scale 2) 1.80 / 1.05 ms;
+// unsorted, one lane per query against this form: 262,144 of 131,072 2.26 / 1.38 ms.
+// Tried and slower: holding a quad's leaf triangles back until half of the wave's quads have some, so that
+// they are evaluated with more lanes active (5-20 %); handing a finished quad another query of the wave
+// (0-40 %: a wave's queries are then no longer neighbours, and their reads no longer shared).
 template <int Order, int Prec, bool Grad, int StackCap>
 __global__ __launch_bounds__(k_taylor_block) void taylor_quad_kernel(
     float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node,
     float const *__restrict__ qx, float const *__restrict__ qy, float const *__restrict__ qz,
     std::uint32_t const *__restrict__ order, taylor_outputs o, std::size_t n, float beta2
 ) {
+    using slot_type = quad_slot<Order, Grad>;
     constexpr int k_quads = k_taylor_block / 4;
     __shared__ std::uint32_t s_stack[StackCap * k_quads];  // entry e of quad k at [e * k_quads + k]
     std::size_t const i = (static_cast<std::size_t>(blockIdx.x) * k_taylor_block + threadIdx.x) >> 2;
     if (i >= n)
         return;  // whole quads
     int const j = static_cast<int>(threadIdx.x & 3);
-    int const quad_shift = static_cast<int>(threadIdx.x & 60);
+    int const shift = static_cast<int>(threadIdx.x & 60);
     std::uint32_t *const stack = s_stack + (threadIdx.x >> 2);
     std::size_t const q = order ? order[i] : i;
     float const x = qx[q], y = qy[q], z = qz[q];
     taylor_sums<Prec, Grad> acc;
-    std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;
+    std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;  // this lane's
     int sp = 0;
     bool overflow = false;
     bool live = true;
-    quad_slot<Order, Grad> slot = quad_slot<Order, Grad>::load(records, root_node, j);
+    slot_type slot = slot_type::load(records, root_node, j);
     while (live) {
+        slot_test<Order, Grad> const v(slot, x, y, z, beta2, true);
         std::uint32_t const c = slot.ref;
-        bool const valid = c != k_invalid;
-        float const qrx = x - slot.cx, qry = y - slot.cy, qrz = z - slot.cz;
-        float const ql2 = squared_norm_unfused(qrx, qry, qrz);
-        bool const far = !(!(ql2 > 0.0f) || ql2 <= product_unfused(slot.mp, beta2));
-        float g[3];
-        float w;
-        if constexpr (Grad)
-            w = taylor_term<Order, true>(slot.c, 0, qrx, qry, qrz, ql2, g);
-        else
-            w = taylor_value<Order>(slot.c, qrx, qry, qrz, ql2);
-        bool const accepted = valid && far && isfinite(w);
-        bool const descend = valid && !accepted;
-        bool const leaf = descend && (c & k_cref_leaf) != 0u;
-        bool const inner = descend && (c & k_cref_leaf) == 0u;
-        n_tests += valid ? 1u : 0u;
-        n_accept += accepted ? 1u : 0u;
-        n_leaf += leaf ? 1u : 0u;
+        n_tests += v.valid ? 1u : 0u;
+        n_accept += v.accepted ? 1u : 0u;
+        n_leaf += v.leaf ? 1u : 0u;
         // The node's triangles, requested before the next node.
         tri_record t{};
-        if (__ballot(leaf) != 0ull)
-            t = tris[leaf ? (c & ~k_cref_leaf) : 0u];
+        if (__ballot(v.leaf) != 0ull)
+            t = tris[v.leaf ? (c & ~k_cref_leaf) : 0u];
         // The last descended internal child is entered, the others are pushed in slot order.
-        std::uint32_t const bits = static_cast<std::uint32_t>(__ballot(inner) >> quad_shift) & 15u;
+        std::uint32_t const bits = static_cast<std::uint32_t>(__ballot(v.inner) >> shift) & 15u;
         std::uint32_t const c0 = quad_bcast<0>(c), c1 = quad_bcast<1>(c), c2 = quad_bcast<2>(c), c3 = quad_bcast<3>(c);
         int const pushed = __popc(bits) - 1;
         std::uint32_t next = bits & 8u ? c3 : (bits & 4u ? c2 : (bits & 2u ? c1 : c0));
         int const at = sp + __popc(bits & ((1u << j) - 1u));
-        if (inner && (bits >> j) != 1u && at < StackCap)
+        if (v.inner && (bits >> j) != 1u && at < StackCap)
             stack[at * k_quads] = c;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         if (pushed >= 0) {
@@ -762,38 +807,20 @@ __global__ __launch_bounds__(k_taylor_block) void taylor_quad_kernel(
         } else {
             live = false;
         }
-        quad_slot<Order, Grad> const ahead = quad_slot<Order, Grad>::load(records, live ? next : root_node, j);
+        slot = slot_type::load(records, live ? next : root_node, j);
         taylor_sums<Prec, Grad> term;
-        if (accepted)
-            term.far_term(w, g);
-        if (leaf)
+        if (v.accepted)
+            term.far_term(v.w, v.g);
+        if (v.leaf)
             term.leaf(t, x, y, z);
-        if constexpr (Prec == GWN_PRECISION_PLAIN) {
-            quad_add(acc.omega, term.omega);
-            if constexpr (Grad) {
-#pragma unroll
-                for (int k = 0; k < 3; ++k)
-                    quad_add(acc.gf[k], term.gf[k]);
-            }
-        } else {
-            quad_add(acc.near, term.near);
-            if constexpr (Grad) {
-#pragma unroll
-                for (int k = 0; k < 3; ++k)
-                    quad_add(acc.gd[k], term.gd[k]);
-            }
-        }
-        slot = ahead;
+        add_terms<4>(acc, term);
     }
     if (j == 0)
         acc.store(overflow, q, o.out, o.gx, o.gy, o.gz);
     if (o.counters != nullptr) {
-        auto const total = [](std::uint32_t v) {
-            return quad_bcast<0>(v) + quad_bcast<1>(v) + quad_bcast<2>(v) + quad_bcast<3>(v);
-        };
-        n_tests = total(n_tests);
-        n_accept = total(n_accept);
-        n_leaf = total(n_leaf);
+        n_tests = quad_sum(n_tests);
+        n_accept = quad_sum(n_accept);
+        n_leaf = quad_sum(n_leaf);
         if (j == 0) {
             o.counters[3 * q + 0] = n_tests;
             o.counters[3 * q + 1] = n_accept;
@@ -801,6 +828,92 @@ __global__ __launch_bounds__(k_taylor_block) void taylor_quad_kernel(
         }
     }
 }
+
+// The quad traversal with a row of 16 lanes per query: quad g tests the g-th entry from the top of the
+// stack.  Entries are settled in stack order up to the first whose node has children to descend into, and
+// those are pushed (what the quads behind it found is dropped, their entries stay on the stack), so nodes
+// take effect and terms are added in the quad traversal's order.  Most nodes of a traversal have no
+// children to descend into, so a row settles two to four at a time.
+template <int Order, int Prec, bool Grad, int StackCap>
+__global__ __launch_bounds__(k_taylor_block) void taylor_row_kernel(
+    float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node,
+    float const *__restrict__ qx, float const *__restrict__ qy, float const *__restrict__ qz,
+    std::uint32_t const *__restrict__ order, taylor_outputs o, std::size_t n, float beta2
+) {
+    using slot_type = quad_slot<Order, Grad>;
+    constexpr int k_rows = k_taylor_block / 16;
+    // Entry e of row k at [e * k_rows + k]; the entered node is on the stack too.
+    __shared__ std::uint32_t s_stack[(StackCap + 1) * k_rows];
+    std::size_t const i = (static_cast<std::size_t>(blockIdx.x) * k_taylor_block + threadIdx.x) >> 4;
+    if (i >= n)
+        return;  // whole rows
+    std::uint32_t const lane = threadIdx.x & 15u;
+    int const j = static_cast<int>(lane & 3u);
+    std::uint32_t const g = lane >> 2;
+    std::uint32_t const shift = threadIdx.x & 48u;
+    std::uint32_t *const stack = s_stack + (threadIdx.x >> 4);
+    std::size_t const q = order ? order[i] : i;
+    float const x = qx[q], y = qy[q], z = qz[q];
+    taylor_sums<Prec, Grad> acc;
+    std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;  // this lane's
+    bool overflow = false;
+    bool live = true;
+    int sp = 1;
+    bool held = g == 0u;
+    if (held)
+        stack[0] = root_node;
+    slot_type slot = slot_type::load(records, root_node, j);
+    while (live) {
+        slot_test<Order, Grad> const v(slot, x, y, z, beta2, held);
+        std::uint32_t const c = slot.ref;
+        std::uint32_t const inners = static_cast<std::uint32_t>(__ballot(v.inner) >> shift) & 0xffffu;
+        std::uint32_t const last = inners != 0u ? static_cast<std::uint32_t>(__builtin_ctz(inners)) >> 2 : 3u;
+        bool const settled = g <= last;
+        bool const leaf = v.leaf && settled;
+        n_tests += v.valid && settled ? 1u : 0u;
+        n_accept += v.accepted && settled ? 1u : 0u;
+        n_leaf += leaf ? 1u : 0u;
+        tri_record t{};
+        if (__ballot(leaf) != 0ull)
+            t = tris[leaf ? (c & ~k_cref_leaf) : 0u];
+        sp = sp > static_cast<int>(last) + 1 ? sp - static_cast<int>(last) - 1 : 0;
+        std::uint32_t const bits = (inners >> (4u * last)) & 15u;  // zero without one
+        int const at = sp + __popc(bits & ((1u << j) - 1u));
+        if (v.inner && g == last && at <= StackCap)
+            stack[at * k_rows] = c;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        sp += __popc(bits);
+        overflow = sp > StackCap + 1;
+        live = sp > 0 && !overflow;
+        int const e = sp - 1 - static_cast<int>(g);
+        held = live && e >= 0;
+        slot = slot_type::load(records, held ? stack[e * k_rows] : root_node, j);
+        taylor_sums<Prec, Grad> term;
+        if (v.accepted && settled)
+            term.far_term(v.w, v.g);
+        if (leaf)
+            term.leaf(t, x, y, z);
+        add_terms<16>(acc, term);
+    }
+    if (lane == 0u)
+        acc.store(overflow, q, o.out, o.gx, o.gy, o.gz);
+    if (o.counters != nullptr) {
+        n_tests = row_sum(n_tests);
+        n_accept = row_sum(n_accept);
+        n_leaf = row_sum(n_leaf);
+        if (lane == 0u) {
+            o.counters[3 * q + 0] = n_tests;
+            o.counters[3 * q + 1] = n_accept;
+            o.counters[3 * q + 2] = n_leaf;
+        }
+    }
+}
+
+// Up to this many queries each has a row: the chip is not full, and the batch lasts as long as its longest
+// query.  Measured, a row against a quad per query (scale 2): 1,000 of 5,120 triangles 90 / 177 us, 8,000
+// of 131,072 280 / 590 us, 65,536 of 131,072 430 / 600 us, 4,096 of 1,048,576 600 / 1,180 us; but 200,000
+// of 5,120 468 / 415 us, of 131,072 754 / 720 us, and 262,144 of 131,072 at scale 6.25 5.4 / 4.1 ms.
+constexpr std::size_t k_row_queries = std::size_t(1) << 16;
 
 // Reciprocal square root and reciprocal in FP64 from the hardware approximations and Newton
 // steps (relative error at FP64 rounding level, not correctly rounded).  x > 0 / x != 0.
@@ -1052,6 +1165,10 @@ void launch_taylor_cap(
     if (order != nullptr && dense_queries(bvh.triangle_count, n, beta2)) {
         // Hilbert-ordered dense queries: neighbouring lanes share most of their paths.
         taylor_wave_kernel<Order, Prec, Grad, Cap><<<grid_for(n, k_taylor_block), k_taylor_block, 0, stream>>>(
+            records, bvh.triangles.ptr, root, qx, qy, qz, order, o, n, beta2
+        );
+    } else if (n <= k_row_queries) {
+        taylor_row_kernel<Order, Prec, Grad, Cap><<<grid_for(16 * n, k_taylor_block), k_taylor_block, 0, stream>>>(
             records, bvh.triangles.ptr, root, qx, qy, qz, order, o, n, beta2
         );
     } else {

@@ -1,6 +1,6 @@
-"""The four-lanes-per-query Taylor traversal against the wave traversal: values, gradients and work
-counters equal bit for bit, at the edges of quads, waves and blocks and on both sides of the density
-rule that chooses between them."""
+"""The Taylor traversals with 16 and four lanes per query against the wave traversal: values, gradients and work
+counters equal bit for bit, at the edges of rows, quads, waves and blocks and on both sides of the rules
+that choose between them."""
 
 import numpy as np
 import pytest
@@ -42,14 +42,14 @@ def _run(gwn, dev, bvh, mom, d, sort, precision, beta, grad):
 def test_quad_equals_wave_bit_for_bit(gwn, dev, order, split, grad):
     precision = gwn.Precision.SPLIT if split else gwn.Precision.PLAIN
     # 8 triangles: dense from 12,728 queries at scale 2; 320: from one query at scale 1e6.
-    for mesh, beta, n_wave in ((synth.octahedron(), 2.0, 14000), (synth.icosphere(2), 1e6, 400)):
+    for mesh, beta, n_wave in ((synth.octahedron(), 2.0, 66000), (synth.icosphere(2), 1e6, 66000)):
         _, bvh = build_gpu(gwn, mesh)
         mom = gwn.MomentObject(order)
         gwn.gwn_refit_bvh_moment(bvh, mom).raise_if_error()
         q = synth.mixed_queries(mesh, n_wave, seed=order + 11)
         q[0][5], q[1][6] = np.nan, np.inf
         want = _run(gwn, dev, bvh, mom, _first(q, n_wave, dev), 1, precision, beta, grad)
-        for n in (1, 15, 16, 17, 63, 65, 255, 257):
+        for n in (1, 3, 4, 5, 15, 17, 65, 257, 65536, 65537):
             got = _run(gwn, dev, bvh, mom, _first(q, n, dev), 0, precision, beta, grad)
             for k, (a, b) in enumerate(zip(got, want)):
                 b = b[:3 * n] if k == 1 else b[:n]
