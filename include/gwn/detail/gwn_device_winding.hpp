@@ -27,23 +27,74 @@ namespace gwn::detail::winding {
 constexpr float k_pi_f = 3.14159265358979323846f;
 constexpr double k_pi_d = 3.14159265358979323846;
 
-// Reference-form FP32 solid angle: rebuild b = v0 + (v1 - v0), c = v0 + (v2 - v0) as the
-// reference's (v0, e1, e2) record does, then Van Oosterom-Strackee.
-__device__ inline float solid_angle_plain(tri_record const &t, float qx, float qy, float qz) {
+// atan2(y, x) for max(|x|, |y|) in [2^-100, 2^100]: |t| <= 1 by one reciprocal, an odd polynomial of
+// degree 17 (a weighted minimax fit of atan(t) / t in t^2, 1.7e-8 relative) and the octants.  Within 3 ulps;
+// 22 issue slots where the library's arctangent, with its exponent scaling and special cases, takes 35.
+__device__ inline float atan2_in_range(float y, float x) {
 #pragma clang fp contract(on)
-    float const e1x = t.v1x - t.v0x, e1y = t.v1y - t.v0y, e1z = t.v1z - t.v0z;
-    float const e2x = t.v2x - t.v0x, e2y = t.v2y - t.v0y, e2z = t.v2z - t.v0z;
-    float ax = t.v0x - qx, ay = t.v0y - qy, az = t.v0z - qz;
-    float bx = (t.v0x + e1x) - qx, by = (t.v0y + e1y) - qy, bz = (t.v0z + e1z) - qz;
-    float cx = (t.v0x + e2x) - qx, cy = (t.v0y + e2y) - qy, cz = (t.v0z + e2z) - qz;
-    float const al = sqrtf(ax * ax + ay * ay + az * az);
-    float const bl = sqrtf(bx * bx + by * by + bz * bz);
-    float const cl = sqrtf(cx * cx + cy * cy + cz * cz);
-    if (al == 0.0f || bl == 0.0f || cl == 0.0f)
-        return 0.0f;
-    ax /= al; ay /= al; az /= al;
-    bx /= bl; by /= bl; bz /= bl;
-    cx /= cl; cy /= cl; cz /= cl;
+    float const ax = fabsf(x), ay = fabsf(y);
+    float const t = fminf(ax, ay) * __builtin_amdgcn_rcpf(fmaxf(ax, ay));
+    float const s = t * t;
+    float p = 0.0029206891f * s - 0.016367916f;
+    p = p * s + 0.043211844f;
+    p = p * s - 0.075522125f;
+    p = p * s + 0.10666004f;
+    p = p * s - 0.14211056f;
+    p = p * s + 0.19993773f;
+    p = p * s - 0.33333153f;
+    float r = t * (s * p) + t;
+    r = ay > ax ? 0.5f * k_pi_f - r : r;
+    r = x < 0.0f ? k_pi_f - r : r;
+    return copysignf(r, y);
+}
+
+// (x, y, z) / sqrt(ss) for ss = |(x, y, z)|^2 in [2^-96, 2^96], the square root and the quotients correctly
+// rounded as `sqrtf` and `/` are (a quotient below 2^-100 of the length may lose its last bit): the root by
+// two Newton steps from the reciprocal square root, whose half also starts the reciprocal of the root, and
+// each quotient by two residual corrections.  In this range no operand or residual needs the scaling that
+// the general expansions carry, and one reciprocal serves three quotients: 27 operations a vector against 47.
+__device__ inline void normalize_in_range(float ss, float &x, float &y, float &z) {
+#pragma clang fp contract(off)
+    float const r0 = __builtin_amdgcn_rsqf(ss);
+    float g = ss * r0, h = 0.5f * r0;
+    float const e0 = __builtin_fmaf(-h, g, 0.5f);
+    g = __builtin_fmaf(g, e0, g);
+    h = __builtin_fmaf(h, e0, h);
+    float const l = __builtin_fmaf(__builtin_fmaf(-g, g, ss), h, g);
+    float r = h + h;
+    r = __builtin_fmaf(__builtin_fmaf(-l, r, 1.0f), r, r);
+    float *const v[3] = {&x, &y, &z};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        float q = *v[k] * r;
+        q = __builtin_fmaf(__builtin_fmaf(-l, q, *v[k]), r, q);
+        *v[k] = __builtin_fmaf(__builtin_fmaf(-l, q, *v[k]), r, q);
+    }
+}
+
+// Van Oosterom-Strackee angle of the corner vectors a, b, c (relative to the query) in the reference's
+// FP32 form: normalized corners, qa . ((qb - qa) x (qc - qa)) over 1 + qa . qb + qa . qc + qb . qc.
+// The usual range of lengths takes the operations above, any other the general ones.
+__device__ inline float solid_angle_corners(
+    float ax, float ay, float az, float bx, float by, float bz, float cx, float cy, float cz
+) {
+#pragma clang fp contract(on)
+    float const aa = ax * ax + ay * ay + az * az;
+    float const bb = bx * bx + by * by + bz * bz;
+    float const cc = cx * cx + cy * cy + cz * cz;
+    bool const usual = fminf(fminf(aa, bb), cc) >= 0x1p-96f && fmaxf(fmaxf(aa, bb), cc) <= 0x1p96f;
+    if (usual) {
+        normalize_in_range(aa, ax, ay, az);
+        normalize_in_range(bb, bx, by, bz);
+        normalize_in_range(cc, cx, cy, cz);
+    } else {
+        float const al = sqrtf(aa), bl = sqrtf(bb), cl = sqrtf(cc);
+        if (al == 0.0f || bl == 0.0f || cl == 0.0f)
+            return 0.0f;
+        ax /= al; ay /= al; az /= al;
+        bx /= bl; by /= bl; bz /= bl;
+        cx /= cl; cy /= cl; cz /= cl;
+    }
     float const ux = bx - ax, uy = by - ay, uz = bz - az;
     float const vx = cx - ax, vy = cy - ay, vz = cz - az;
     float const num = ax * (uy * vz - uz * vy) + ay * (uz * vx - ux * vz) + az * (ux * vy - uy * vx);
@@ -51,7 +102,20 @@ __device__ inline float solid_angle_plain(tri_record const &t, float qx, float q
         return 0.0f;
     float const den = 1.0f + (ax * bx + ay * by + az * bz) + (ax * cx + ay * cy + az * cz) +
                       (bx * cx + by * cy + bz * cz);
-    return 2.0f * atan2f(num, den);
+    if (!(fmaxf(fabsf(num), fabsf(den)) >= 0x1p-100f))
+        return 2.0f * atan2f(num, den);
+    return 2.0f * atan2_in_range(num, den);
+}
+
+// Reference-form FP32 solid angle: rebuild b = v0 + (v1 - v0), c = v0 + (v2 - v0) as the
+// reference's (v0, e1, e2) record does, then Van Oosterom-Strackee.
+__device__ inline float solid_angle_plain(tri_record const &t, float qx, float qy, float qz) {
+#pragma clang fp contract(on)
+    float const e1x = t.v1x - t.v0x, e1y = t.v1y - t.v0y, e1z = t.v1z - t.v0z;
+    float const e2x = t.v2x - t.v0x, e2y = t.v2y - t.v0y, e2z = t.v2z - t.v0z;
+    return solid_angle_corners(
+        t.v0x - qx, t.v0y - qy, t.v0z - qz, (t.v0x + e1x) - qx, (t.v0y + e1y) - qy, (t.v0z + e1z) - qz,
+        (t.v0x + e2x) - qx, (t.v0y + e2y) - qy, (t.v0z + e2z) - qz);
 }
 
 // Solid angle without normalizing the corner vectors: with a = v0 - q, b = v1 - q, c = v2 - q,
@@ -106,7 +170,7 @@ __device__ inline double sqrt_f64_fast(double x) {
 
 // Precision-split near triangle: corner vectors (exact differences of the float vertices and
 // query), lengths, numerator and denominator in FP64, where the cancellation happens; the final
-// angle by FP32 atan2 of the FP64 pair scaled by a power of two into range.  The angle's absolute
+// angle by FP32 atan2 of the FP64 pair scaled by a power of two into range (the larger to [1/2, 1)).  The angle's absolute
 // error is a few 1e-7 rad, 1e-8 of W, per triangle.
 __device__ inline double solid_angle_split_near(tri_record const &t, float x, float y, float z) {
 #pragma clang fp contract(on)
@@ -135,27 +199,35 @@ __device__ inline double solid_angle_split_near(tri_record const &t, float x, fl
     int const e = __builtin_amdgcn_frexp_exp(fmax(fabs(num), fabs(den)));
     float const fn = static_cast<float>(__builtin_amdgcn_ldexp(num, -e));
     float const fd = static_cast<float>(__builtin_amdgcn_ldexp(den, -e));
-    return 2.0 * static_cast<double>(atan2f(fn, fd));
+    return 2.0 * static_cast<double>(atan2_in_range(fn, fd));
 }
 
-// FP32 far-field solid angle (precision split): same form with hardware square roots.
-__device__ inline float solid_angle_far_f32(float ax, float ay, float az, float e1x, float e1y, float e1z,
-                                            float e2x, float e2y, float e2z) {
+// Half the FP32 solid angle of a far triangle (precision split: |a| > 4 max(|e1|, |e2|), a = v0 - q).  With
+// s1 = a . e1 and s2 = a . e2 every length and dot product of the corners b = a + e1 and c = a + e2 is a
+// short sum: |b|^2 = |a|^2 + 2 s1 + |e1|^2, a . b = |a|^2 + s1, b . c = a . b + s2 + e1 . e2 (and so on),
+// none of which cancels, since |e| < |a| / 4.  The same bound gives |num| <= |a|^3 / 16 (num = a . (e1 x e2))
+// and den >= 2.1 |a|^3, so u = num / den <= 0.03 and u - u^3 / 3 + u^5 / 5 is atan(u) to u^7 / 7 < 1e-10 of
+// u.  A denominator outside the reciprocal's range (coordinates near the ends of the float range) takes
+// the arctangent.  Any value unless `far`.
+__device__ inline float half_angle_far(
+    float aa, float s1, float s2, float num, float ee1, float ee2, float e12, bool far
+) {
 #pragma clang fp contract(on)
-    float const bx = ax + e1x, by = ay + e1y, bz = az + e1z;
-    float const cx = ax + e2x, cy = ay + e2y, cz = az + e2z;
-    float const la = __builtin_amdgcn_sqrtf(ax * ax + ay * ay + az * az);
-    float const lb = __builtin_amdgcn_sqrtf(bx * bx + by * by + bz * bz);
-    float const lc = __builtin_amdgcn_sqrtf(cx * cx + cy * cy + cz * cz);
-    float const nx = e1y * e2z - e1z * e2y;
-    float const ny = e1z * e2x - e1x * e2z;
-    float const nz = e1x * e2y - e1y * e2x;
-    float const num = ax * nx + ay * ny + az * nz;
-    float const den = la * lb * lc + (ax * bx + ay * by + az * bz) * lc + (ax * cx + ay * cy + az * cz) * lb +
-                      (bx * cx + by * cy + bz * cz) * la;
-    return 2.0f * atan2f(num, den);
+    float const la = __builtin_amdgcn_sqrtf(aa);
+    float const lb = __builtin_amdgcn_sqrtf(aa + (2.0f * s1 + ee1));
+    float const lc = __builtin_amdgcn_sqrtf(aa + (2.0f * s2 + ee2));
+    float const ab = aa + s1;
+    float const ac = aa + s2;
+    float const bc = ab + (s2 + e12);
+    float const den = la * lb * lc + ab * lc + ac * lb + bc * la;
+    float const u = num * __builtin_amdgcn_rcpf(den);
+    float const u2 = u * u;
+    float h = u + u * (u2 * (u2 * 0.2f - 0.33333334f));
+    constexpr std::uint32_t k_lo = 0x01000000u, k_hi = 0x7e000000u;  // 2^-125, 2^125
+    if (__float_as_uint(den) - k_lo >= k_hi - k_lo && far)
+        h = atan2f(num, den);
+    return h;
 }
-
 
 // Near-field radius of the precision split, in units of the triangle's longest edge from v0.
 constexpr float k_split_near_scale2 = 16.0f; // (4 * edge)^2
@@ -257,7 +329,10 @@ __device__ inline void split_leaf(tri_record const &t, float x, float y, float z
             gsum[2] += o[2];
         }
     } else {
-        sum += double(solid_angle_far_f32(ax, ay, az, e1x, e1y, e1z, e2x, e2y, e2z));
+        float const num = ax * (e1y * e2z - e1z * e2y) + ay * (e1z * e2x - e1x * e2z) + az * (e1x * e2y - e1y * e2x);
+        sum += 2.0 * double(half_angle_far(
+                         dq, ax * e1x + ay * e1y + az * e1z, ax * e2x + ay * e2y + az * e2z, num, le1, le2,
+                         e1x * e2x + e1y * e2y + e1z * e2z, true));
         if constexpr (Grad) {
             float const g[3][3] = {{ax, ay, az}, {t.v1x - x, t.v1y - y, t.v1z - z}, {t.v2x - x, t.v2y - y, t.v2z - z}};
             float o[3];

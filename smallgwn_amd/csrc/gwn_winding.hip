@@ -77,55 +77,16 @@ __device__ inline void stage_exact_item(tri_record const &t, exact_item &o) {
     }
 }
 
-// solid_angle_plain on the staged corners (the same operations from there on).
+// solid_angle_plain on the staged corners.
 __device__ inline float solid_angle_plain_staged(exact_item const &t, float qx, float qy, float qz) {
-    float ax = t.f[0] - qx, ay = t.f[1] - qy, az = t.f[2] - qz;
-    float bx = t.f[3] - qx, by = t.f[4] - qy, bz = t.f[5] - qz;
-    float cx = t.f[6] - qx, cy = t.f[7] - qy, cz = t.f[8] - qz;
-    float const al = sqrtf(ax * ax + ay * ay + az * az);
-    float const bl = sqrtf(bx * bx + by * by + bz * bz);
-    float const cl = sqrtf(cx * cx + cy * cy + cz * cz);
-    if (al == 0.0f || bl == 0.0f || cl == 0.0f)
-        return 0.0f;
-    ax /= al; ay /= al; az /= al;
-    bx /= bl; by /= bl; bz /= bl;
-    cx /= cl; cy /= cl; cz /= cl;
-    float const ux = bx - ax, uy = by - ay, uz = bz - az;
-    float const vx = cx - ax, vy = cy - ay, vz = cz - az;
-    float const num = ax * (uy * vz - uz * vy) + ay * (uz * vx - ux * vz) + az * (ux * vy - uy * vx);
-    if (num == 0.0f)
-        return 0.0f;
-    float const den = 1.0f + (ax * bx + ay * by + az * bz) + (ax * cx + ay * cy + az * cz) +
-                      (bx * cx + by * cy + bz * cz);
-    return 2.0f * atan2f(num, den);
+    return solid_angle_corners(t.f[0] - qx, t.f[1] - qy, t.f[2] - qz, t.f[3] - qx, t.f[4] - qy, t.f[5] - qz,
+                               t.f[6] - qx, t.f[7] - qy, t.f[8] - qz);
 }
 
-// Half the solid angle of a staged far triangle (|a| > 4 max(|e1|, |e2|), a = v0 - q), split form;
-// any value where `near`.  With s1 = a . e1 and s2 = a . e2 every length and dot product of the
-// corners b = a + e1 and c = a + e2 is a short sum: |b|^2 = |a|^2 + 2 s1 + |e1|^2, a . b = |a|^2 + s1,
-// b . c = a . b + s2 + e1 . e2 (and so on), none of which cancels, since |e| < |a| / 4.  The same
-// bound gives |num| <= |a|^3 / 16 and den >= 2.1 |a|^3, so u = num / den <= 0.03 and
-// u - u^3 / 3 + u^5 / 5 is atan(u) to u^7 / 7 < 1e-10 of u: 42 operations and 4 half-rate ones
-// where the two-argument arctangent and the edges formed per pair took 109.  A denominator outside
-// the reciprocal's range (coordinates near the ends of the float range) takes the arctangent.
-__device__ inline float half_angle_far_staged(exact_item const &t, float ax, float ay, float az, float aa, bool near) {
-    float const s1 = ax * t.f[3] + ay * t.f[4] + az * t.f[5];
-    float const s2 = ax * t.f[6] + ay * t.f[7] + az * t.f[8];
-    float const num = ax * t.f[9] + ay * t.f[10] + az * t.f[11];
-    float const la = __builtin_amdgcn_sqrtf(aa);
-    float const lb = __builtin_amdgcn_sqrtf(aa + (2.0f * s1 + t.f[12]));
-    float const lc = __builtin_amdgcn_sqrtf(aa + (2.0f * s2 + t.f[13]));
-    float const ab = aa + s1;
-    float const ac = aa + s2;
-    float const bc = ab + (s2 + t.f[14]);
-    float const den = la * lb * lc + ab * lc + ac * lb + bc * la;
-    float const u = num * __builtin_amdgcn_rcpf(den);
-    float const u2 = u * u;
-    float h = u + u * (u2 * (u2 * 0.2f - 0.33333334f));
-    constexpr std::uint32_t k_lo = 0x01000000u, k_hi = 0x7e000000u;  // 2^-125, 2^125
-    if (__float_as_uint(den) - k_lo >= k_hi - k_lo && !near)
-        h = atan2f(num, den);
-    return h;
+// half_angle_far of a staged triangle.
+__device__ inline float half_angle_far_staged(exact_item const &t, float ax, float ay, float az, float aa, bool far) {
+    return half_angle_far(aa, ax * t.f[3] + ay * t.f[4] + az * t.f[5], ax * t.f[6] + ay * t.f[7] + az * t.f[8],
+                          ax * t.f[9] + ay * t.f[10] + az * t.f[11], t.f[12], t.f[13], t.f[14], far);
 }
 
 // Adds the values of a group's Lanes lanes to its running sum in lane order (the group's lanes are
@@ -145,11 +106,11 @@ template <int Lanes, int J = 0> __device__ inline void add_in_lane_order(float &
 // record order, so every query's float sum is formed over the records in the reference's order
 // whatever Lanes is (a lane past the tile's end adds zero, which changes no sum).
 //
-// VALU bound: about 220 issue slots a pair (nine correctly rounded quotients, three square roots,
+// VALU bound: about 165 issue slots a pair (nine correctly rounded quotients, three square roots,
 // one arctangent), one to sixteen for the ordered add.  One lane per query leaves the chip idle
-// below some hundred thousand queries.  Measured with one lane against the widest groups that fill
-// the chip, 131,044 triangles: 1,000 queries 74.0 against 5.6 ms, 65,536 queries 74.1 against 49.8 ms,
-// 131,072 queries 110 against 96 ms.
+// below some hundred thousand queries.  Measured with one lane and the general quotients, square roots and
+// arctangent (220 slots) against this form: 131,044 triangles x 1,000 queries 74.0 against 5.6 ms (the groups
+// alone), 100,000 x 65,536 56.5 against 22.0 ms.
 template <int Lanes, class Out>
 __global__ __launch_bounds__(k_exact_block) void exact_plain_kernel(
     tri_record const *__restrict__ tris, std::size_t nt, float const *__restrict__ qx,
@@ -186,10 +147,10 @@ __global__ __launch_bounds__(k_exact_block) void exact_plain_kernel(
 // tiles_per_share.  With one share the winding number goes to `out`; with more, the share's FP64 sum
 // goes to part[y * nq + q] and exact_combine_kernel adds the shares in order.
 //
-// VALU bound (a split pair costs 49 issue slots), so what counts is that every SIMD has waves: a
+// VALU bound (a far split pair costs 49 issue slots), so what counts is that every SIMD has waves: a
 // launch of nq / 256 blocks alone left 32,749 queries on half of the CUs with one wave per SIMD.
 // Measured, split, one share with per-pair edges and arctangents against this form: 100,000 triangles
-// x 32,749 queries 38.1 against 5.0 ms, 131,044 x 1,000 52.3 against 0.48 ms, 25,600 x 600,000 (one
+// x 32,749 queries 38.1 against 4.7 ms, 131,044 x 1,000 52.3 against 0.48 ms, 25,600 x 600,000 (one
 // share in both) 56.9 against 37.0 ms.
 template <int Prec>
 __global__ __launch_bounds__(k_exact_block) void exact_kernel(
@@ -230,7 +191,7 @@ __global__ __launch_bounds__(k_exact_block) void exact_kernel(
                 float const ax = t.f[0] - x, ay = t.f[1] - y, az = t.f[2] - z;
                 float const aa = ax * ax + ay * ay + az * az;
                 bool const near = !(aa > t.f[15]);
-                float const h = half_angle_far_staged(t, ax, ay, az, aa, near);
+                float const h = half_angle_far_staged(t, ax, ay, az, aa, !near);
                 far += near ? 0.0f : h;
                 if (near)
                     sum += solid_angle_split_near(tris[base + k], x, y, z);
@@ -391,8 +352,16 @@ __global__ __launch_bounds__(256) void query_key_kernel(
 }
 
 
+// A wave-uniform value in scalar registers (one read back from LDS otherwise lives in vector ones, and
+// every mask formed from it with it).
+__device__ inline std::uint64_t uniform_u64(std::uint64_t v) {
+    std::uint32_t const lo = __builtin_amdgcn_readfirstlane(static_cast<std::uint32_t>(v));
+    std::uint32_t const hi = __builtin_amdgcn_readfirstlane(static_cast<std::uint32_t>(v >> 32));
+    return (static_cast<std::uint64_t>(hi) << 32) | lo;
+}
+
 // Wave-cooperative traversal (defined below; the batched kernel uses it too).
-template <int Order, int Prec, bool Grad, int StackCap>
+template <int Order, int Prec, bool Grad, int StackCap, bool Count>
 __device__ inline bool taylor_wave_traverse(
     float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node, bool active,
     float x, float y, float z, float beta2, taylor_sums<Prec, Grad> &acc, std::uint32_t &n_tests,
@@ -455,7 +424,7 @@ __global__ __launch_bounds__(256) void taylor_batch_kernel(
                 if constexpr (Mode != 0) {
                     if (__ballot(active) == 0ull)
                         continue;
-                    overflow = taylor_wave_traverse<Order, GWN_PRECISION_PLAIN, false, StackCap>(
+                    overflow = taylor_wave_traverse<Order, GWN_PRECISION_PLAIN, false, StackCap, false>(
                         m.records, m.tris, static_cast<std::uint32_t>(ref_offset(m.root)), active, x, y, z, beta2,
                         acc, n_tests, n_accept, n_leaf, s_node[wave], s_mask[wave]);
                     if (!active)
@@ -483,8 +452,8 @@ __global__ __launch_bounds__(256) void taylor_batch_kernel(
 // The wave-cooperative traversal of one wave's queries (lanes with `active`); s_node / s_mask are
 // this wave's LDS stack.  The wave must hold at least one active lane.  Returns true on overflow.
 // `records` are evaluation records for the value alone and traversal records with the gradient,
-// as for the per-lane traversal.
-template <int Order, int Prec, bool Grad, int StackCap>
+// as for the per-lane traversal.  The work tallies are kept where Count (three adds a slot otherwise).
+template <int Order, int Prec, bool Grad, int StackCap, bool Count>
 __device__ inline bool taylor_wave_traverse(
     float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node, bool active,
     float x, float y, float z, float beta2, taylor_sums<Prec, Grad> &acc, std::uint32_t &n_tests,
@@ -492,14 +461,17 @@ __device__ inline bool taylor_wave_traverse(
 ) {
     constexpr int RV = Grad ? moment_record_vec4(Order) : eval_record_vec4(Order);
     constexpr int B = eval_slot_floats(Order);
-    int const lane = threadIdx.x & 63;
     std::uint64_t mask = __ballot(active);
-    std::uint64_t const my_bit = 1ull << lane;
+    std::uint64_t const my_bit = 1ull << (threadIdx.x & 63);
     std::uint32_t node = root_node;
     int sp = 0;
     bool overflow = false;  // wave-uniform
+    // In a vector register: a product of two scalar ones takes a move first, once per acceptance test.
+    float scale2 = beta2;
+    asm("" : "+v"(scale2));
     while (node != k_invalid && !overflow) {
         node = __builtin_amdgcn_readfirstlane(node);
+        mask = uniform_u64(mask);
         float4 const *rec = records + static_cast<std::size_t>(node) * RV;
         float4 const refs = rec[0];
         float4 const mp = rec[1], px = rec[2], py = rec[3], pz = rec[4];
@@ -510,7 +482,11 @@ __device__ inline bool taylor_wave_traverse(
         float const cx[4] = {px.x, px.y, px.z, px.w};
         float const cy[4] = {py.x, py.y, py.z, py.w};
         float const cz[4] = {pz.x, pz.y, pz.z, pz.w};
-        bool const in = (mask & my_bit) != 0ull;
+        // All of the header at once: left to itself the compiler moves a slot's part past the check of the
+        // slot's reference, a second wait on the node-to-node chain.
+        asm volatile("" ::"s"(mp.x), "s"(mp.y), "s"(mp.z), "s"(mp.w), "s"(px.x), "s"(px.y), "s"(px.z), "s"(px.w),
+                     "s"(py.x), "s"(py.y), "s"(py.z), "s"(py.w), "s"(pz.x), "s"(pz.y), "s"(pz.z), "s"(pz.w));
+        [[maybe_unused]] bool const in = (mask & my_bit) != 0ull;
         std::uint32_t next = k_invalid;
         std::uint64_t next_mask = 0ull;
 #pragma unroll
@@ -518,35 +494,46 @@ __device__ inline bool taylor_wave_traverse(
             std::uint32_t const c = __builtin_amdgcn_readfirstlane(cref[s]);
             if (c == k_invalid || overflow)
                 continue;
-            bool descend = false;
-            if (in) {
-                ++n_tests;
-                float const qrx = x - cx[s], qry = y - cy[s], qrz = z - cz[s];
-                float const ql2 = squared_norm_unfused(qrx, qry, qrz);
-                descend = !(ql2 > 0.0f) || ql2 <= product_unfused(mpd[s], beta2);
-                if (!descend) {
-                    float g[3];
-                    float w;
-                    if constexpr (Grad)
-                        w = taylor_term<Order, true>(fields, s, qrx, qry, qrz, ql2, g);
-                    else
-                        w = taylor_value<Order>(reinterpret_cast<float const *>(rec + 5) + s * B, qrx, qry, qrz,
-                                                ql2);
-                    if (isfinite(w)) {
-                        acc.far_term(w, g);
-                        ++n_accept;
-                    } else {
-                        descend = true;
-                    }
+            // Every lane tests and evaluates; the masks, in scalar registers, say whose result counts.
+            // (Masked instructions issue no faster, and the branches' masks cost vector instructions.)
+            constexpr int k_less = 4, k_less_equal = 5;  // ordered
+            float const qrx = x - cx[s], qry = y - cy[s], qrz = z - cz[s];
+            float const ql2 = squared_norm_unfused(qrx, qry, qrz);
+            // A zero or NaN ql2 descends here or by the test on w below.
+            std::uint64_t dmask = __builtin_amdgcn_fcmpf(ql2, product_unfused(mpd[s], scale2), k_less_equal) & mask;
+            std::uint64_t const fmask = mask & ~dmask;
+            if constexpr (Count)
+                n_tests += in ? 1u : 0u;
+            if (fmask != 0ull) {
+                float g[3];
+                float w;
+                if constexpr (Grad)
+                    w = taylor_term<Order, true>(fields, s, qrx, qry, qrz, ql2, g);
+                else
+                    w = taylor_value<Order>(reinterpret_cast<float const *>(rec + 5) + s * B, qrx, qry, qrz, ql2);
+                std::uint64_t const amask = __builtin_amdgcn_fcmpf(fabsf(w), INFINITY, k_less) & fmask;
+                dmask |= fmask & ~amask;
+                // A lane without a term adds zero, which leaves its sum as it is (never -0).
+                bool const accepted = __builtin_amdgcn_inverse_ballot_w64(amask);
+                w = accepted ? w : 0.0f;
+                if constexpr (Grad) {
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+                        g[k] = accepted ? g[k] : 0.0f;
+                } else {
+                    asm("" : "+v"(w));  // one select on the term, not two on its FP64 value
                 }
+                acc.far_term(w, g);
+                if constexpr (Count)
+                    n_accept += accepted ? 1u : 0u;
             }
-            std::uint64_t const dmask = __ballot(descend);
             if (dmask == 0ull)
                 continue;
             if (c & k_cref_leaf) {
                 tri_record const t = tris[c & ~k_cref_leaf];
-                if (dmask & my_bit) {
-                    ++n_leaf;
+                if (__builtin_amdgcn_inverse_ballot_w64(dmask)) {
+                    if constexpr (Count)
+                        ++n_leaf;
                     acc.leaf(t, x, y, z);
                 }
                 continue;
@@ -574,7 +561,7 @@ __device__ inline bool taylor_wave_traverse(
     return overflow;
 }
 
-template <int Order, int Prec, bool Grad, int StackCap>
+template <int Order, int Prec, bool Grad, int StackCap, bool Count>
 __global__ __launch_bounds__(k_taylor_block) void taylor_wave_kernel(
     float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node,
     float const *__restrict__ qx, float const *__restrict__ qy, float const *__restrict__ qz,
@@ -594,12 +581,12 @@ __global__ __launch_bounds__(k_taylor_block) void taylor_wave_kernel(
         return;
     taylor_sums<Prec, Grad> acc;
     std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;
-    bool const overflow = taylor_wave_traverse<Order, Prec, Grad, StackCap>(
+    bool const overflow = taylor_wave_traverse<Order, Prec, Grad, StackCap, Count>(
         records, tris, root_node, active, x, y, z, beta2, acc, n_tests, n_accept, n_leaf, s_node[wave], s_mask[wave]);
     if (!active)
         return;
     acc.store(overflow, q, o.out, o.gx, o.gy, o.gz);
-    if (o.counters != nullptr) {
+    if constexpr (Count) {
         o.counters[3 * q + 0] = n_tests;
         o.counters[3 * q + 1] = n_accept;
         o.counters[3 * q + 2] = n_leaf;
@@ -1163,10 +1150,18 @@ void launch_taylor_cap(
     // The value alone reads the evaluation records; the gradient the traversal records.
     float4 const *records = Grad ? m.records.ptr : m.eval_records.ptr;
     if (order != nullptr && dense_queries(bvh.triangle_count, n, beta2)) {
-        // Hilbert-ordered dense queries: neighbouring lanes share most of their paths.
-        taylor_wave_kernel<Order, Prec, Grad, Cap><<<grid_for(n, k_taylor_block), k_taylor_block, 0, stream>>>(
-            records, bvh.triangles.ptr, root, qx, qy, qz, order, o, n, beta2
-        );
+        // Hilbert-ordered dense queries: neighbouring lanes share most of their paths.  VALU bound:
+        // 16,777,216 queries of 1,048,576 triangles (order 2, split, scale 6.25) took 69.0 ms with 189,111
+        // instructions a wave, 59.5 ms with the 166,216 of unmasked tests and terms, tallies on demand only
+        // and half_angle_far.
+        if (o.counters != nullptr)
+            taylor_wave_kernel<Order, Prec, Grad, Cap, true><<<grid_for(n, k_taylor_block), k_taylor_block, 0, stream>>>(
+                records, bvh.triangles.ptr, root, qx, qy, qz, order, o, n, beta2
+            );
+        else
+            taylor_wave_kernel<Order, Prec, Grad, Cap, false><<<grid_for(n, k_taylor_block), k_taylor_block, 0, stream>>>(
+                records, bvh.triangles.ptr, root, qx, qy, qz, order, o, n, beta2
+            );
     } else if (n <= k_row_queries) {
         taylor_row_kernel<Order, Prec, Grad, Cap><<<grid_for(16 * n, k_taylor_block), k_taylor_block, 0, stream>>>(
             records, bvh.triangles.ptr, root, qx, qy, qz, order, o, n, beta2
