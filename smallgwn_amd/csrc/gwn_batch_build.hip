@@ -206,15 +206,21 @@ __global__ __launch_bounds__(k_hploc_seg_chunk_block) void seg_hploc_kernel(
                                                parked, words + 4, root_words, words);
 }
 
-// H-PLOC global launch over the ranges the chunk launch parked.
+// H-PLOC global launch over the ranges the chunk launch parked.  A wave's merges run two at a time
+// (one per half), so with one range per lane a step of the climb lasts up to 32 merges; with a half
+// per range (HalfPerRange) it lasts one, but the launch takes 32 times the waves.  A half per range while
+// all of those waves fit the chip at once (8,192).  Measured, one range per lane against one per half: a replay
+// (build, moments, queries) of 128 meshes of 2.1M triangles 9.4 / 7.8 ms, of 8 meshes of 174,000 4.5 / 2.5 ms;
+// 4,096 meshes of 113M triangles (220,000 ranges) the other way round, 101 / 161 ms for the builds.
+template <bool HalfPerRange>
 __global__ __launch_bounds__(k_hploc_block) void seg_hploc_parked_kernel(
     seg_mesh const *__restrict__ meshes, std::uint32_t const *__restrict__ leaf_prefix, std::uint32_t mesh_count,
     std::uint64_t const *__restrict__ codes, aabb const *__restrict__ leaf_boxes, std::uint32_t total,
     std::uint32_t radius, hploc_out o, std::uint32_t *boundary, uint2 const *parked, std::uint32_t *root_words,
     std::uint32_t *words
 ) {
-    std::uint32_t const i = blockIdx.x * k_hploc_block + threadIdx.x;  // one range per lane (they are many and small)
-    bool const active = i < words[4];
+    std::uint32_t const i = HalfPerRange ? hploc_parked_slot(blockIdx.x) : blockIdx.x * k_hploc_block + threadIdx.x;
+    bool const active = i != k_invalid && i < words[4];
     uint2 const r = active ? parked[i] : make_uint2(0u, 0u);
     build_segment const seg = active ? seg_of(meshes, leaf_prefix, mesh_count, r.x) : build_segment{0u, 0u, 0u, 0u};
     hploc_climb<false>(codes, leaf_boxes, total, radius, o, boundary, seg, r.x, r.y, active, 0u, 0u, nullptr, nullptr,
@@ -895,9 +901,15 @@ void batch_trees_enqueue(batch_trees &t, int levels, int binary_levels, std::uin
             t.meshes.ptr, t.leaf_prefix.ptr, M, codes, t.leaf_boxes.ptr, n, t.radius, out_arrays, t.boundary.ptr,
             t.parked.ptr, t.root_words.ptr, t.words.ptr);
         GWN_LAUNCH_CHECK();
-        seg_hploc_parked_kernel<<<blocks_for(t.parked.count, k_hploc_block), k_hploc_block, 0, stream>>>(
-            t.meshes.ptr, t.leaf_prefix.ptr, M, codes, t.leaf_boxes.ptr, n, t.radius, out_arrays, t.boundary.ptr,
-            t.parked.ptr, t.root_words.ptr, t.words.ptr);
+        if (t.parked.count <= 2 * 8192)
+            seg_hploc_parked_kernel<true><<<static_cast<unsigned>(hploc_parked_blocks(t.parked.count)), k_hploc_block, 0,
+                                            stream>>>(
+                t.meshes.ptr, t.leaf_prefix.ptr, M, codes, t.leaf_boxes.ptr, n, t.radius, out_arrays, t.boundary.ptr,
+                t.parked.ptr, t.root_words.ptr, t.words.ptr);
+        else
+            seg_hploc_parked_kernel<false><<<blocks_for(t.parked.count, k_hploc_block), k_hploc_block, 0, stream>>>(
+                t.meshes.ptr, t.leaf_prefix.ptr, M, codes, t.leaf_boxes.ptr, n, t.radius, out_arrays, t.boundary.ptr,
+                t.parked.ptr, t.root_words.ptr, t.words.ptr);
         GWN_LAUNCH_CHECK();
     }
     // Collapse, one plan + one persistent launch per wide level.
