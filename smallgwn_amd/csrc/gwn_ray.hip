@@ -2,7 +2,8 @@
 //
 // Reference: include/gwn/detail/gwn_query_ray_impl.cuh:20-595, include/gwn/gwn_query.cuh:182-290.
 //
-// One ray per lane.  Two traversals, chosen per batch exactly as the reference's launcher does:
+// Four lanes per ray (ray_quad_kernel; one per lane for the work counters and a leaf root).  Two
+// traversals, chosen per batch exactly as the reference's launcher does:
 //   packed    (internal root, fewer than 2^29 nodes, packed_stack_bound within the stack): leaf
 //             and internal children share one near-ordered sequence of 32-bit payloads (leaf =
 //             bit 31 | parent << 2 | slot); the nearest child is entered, the others pushed;
@@ -13,7 +14,10 @@
 //
 // Arithmetic is unfused with correctly rounded division, so every record equals the CPU
 // oracle's replay bit for bit.
+#include <algorithm>
+
 #include "gwn_core.hpp"
+#include "gwn_quad.hpp"
 #include "../../include/gwn/detail/gwn_device_ray.hpp"
 
 #include <cfloat>
@@ -47,6 +51,221 @@ __global__ __launch_bounds__(k_block) void ray_kernel(
     }
 }
 
+constexpr int k_ray_stride = k_block / 4 + 1;  // entry e of quad k's stack at [e * k_ray_stride + k]
+
+// intersect_triangle's result before it meets the best hit: whether the ray meets the triangle at t >= t_min.
+__device__ inline bool triangle_candidate(
+    ray_state const &r, tri_record const &tr, float t_min, float &t, float &bu, float &bv, float (&ng)[3]
+) {
+    best_hit h{INFINITY, 0.0f, 0.0f, {0.0f, 0.0f, 0.0f}, 0u, false};
+    intersect_triangle(r, tr, 0u, t_min, h);
+    t = h.t;
+    bu = h.u;
+    bv = h.v;
+    ng[0] = h.n[0];
+    ng[1] = h.n[1];
+    ng[2] = h.n[2];
+    return h.found;
+}
+
+// Four lanes per ray, lane j of the quad owning child slot j of each node, with the hits of
+// ray_first_hit_lane bit for bit.  The four slab tests, and the triangles of the leaf children (one per
+// leaf in this library's trees; a triangle's hit does not depend on the best found before it), are
+// evaluated side by side, and the quad takes the traversal's steps on them together:
+//   canonical: every leaf near first, then the internal children far to near onto the stack, the nearest
+//     entered.  A hit nearer than its leaf's box is a rounding case that goes leaf by leaf; without one
+//     the smallest t wins, and among equal ones the first in order, whichever leaves the best excludes;
+//   packed: the leaves before the first internal child in near-first order, that child entered, the rest
+//     (leaves too) onto the stack; up to four leaves from the top of the stack are settled at a time.
+// The stack (the quad's column of an LDS array) keeps the slab entry t of each child, and an internal child
+// beyond the best hit is dropped when popped: its children's boxes lie inside its own and every operation
+// of the slab test is monotone in the bounds, so they would all have missed.  A wave hands its next ray to a
+// quad that has finished (18 nodes a ray on average, 500 at most on the 1M-triangle mesh).
+//
+// One ray per lane was bound by the gathers: each of a node's eight 16-byte loads touched 64 lines a
+// wave, and its stack lived in scratch memory; a quad reads a node's 128 bytes in two.  Measured, one lane per
+// ray against this form: 4,194,304 rays on 1,048,576 triangles 5.3 / 3.5 ms (canonical), 4.9 / 3.7 ms
+// (packed), on 5,120 1.90 / 1.73 ms; 1,000 rays on 1,048,576 274 / 88 us.
+template <bool Packed, int Cap>
+__global__ __launch_bounds__(k_block) void ray_quad_kernel(
+    ray_scene sc, std::uint32_t root, float const *__restrict__ ox, float const *__restrict__ oy,
+    float const *__restrict__ oz, float const *__restrict__ dx, float const *__restrict__ dy,
+    float const *__restrict__ dz, ray_hit *__restrict__ out, std::size_t n, float t_min, float t_max
+) {
+    __shared__ std::uint32_t s_node[Cap * k_ray_stride];
+    __shared__ float s_t[Cap * k_ray_stride];
+    std::uint32_t const lane = threadIdx.x & 63u;
+    std::uint32_t const j = lane & 3u;
+    std::uint32_t const shift = lane & 60u;
+    std::uint32_t *const st_node = s_node + (threadIdx.x >> 2);
+    float *const st_t = s_t + (threadIdx.x >> 2);
+    // The wave's t-th ray: 16 consecutive ones, then 16 one grid further on.
+    std::size_t const wave = static_cast<std::size_t>(blockIdx.x) * (k_block / 64) + (threadIdx.x >> 6);
+    std::size_t const waves = static_cast<std::size_t>(gridDim.x) * (k_block / 64);
+    auto const nth = [=](std::size_t k) { return ((k >> 4) * waves + wave) * 16 + (k & 15); };
+    std::size_t taken = 16;  // rays handed out so far, wave-uniform
+    std::size_t i = nth(lane >> 2);
+    bool live = i < n;
+    ray_state r{};
+    best_hit best{};
+    int sp = 0;
+    bvh_child slot{};
+    auto const begin_ray = [&] {
+        r.o[0] = ox[i];
+        r.o[1] = oy[i];
+        r.o[2] = oz[i];
+        r.d[0] = dx[i];
+        r.d[1] = dy[i];
+        r.d[2] = dz[i];
+        best = best_hit{t_max, 0.0f, 0.0f, {0.0f, 0.0f, 0.0f}, 0xffffffffu, false};
+        sp = 0;
+        slot = sc.nodes[root].children[j];
+        float const len2 = r.d[0] * r.d[0] + r.d[1] * r.d[1] + r.d[2] * r.d[2];
+        if (!(len2 > 0.0f))
+            slot.reference = 0;  // a zero direction meets nothing
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            r.zero[k] = r.d[k] == 0.0f;
+            r.inv[k] = r.zero[k] ? 0.0f : 1.0f / r.d[k];
+        }
+        r.parallel = r.zero[0] || r.zero[1] || r.zero[2];
+    };
+    if (live)
+        begin_ray();
+    while (__ballot(live) != 0ull) {
+        bool finished = false;
+        bool overflow = false;
+        if (live) {
+            // Takes the lane marked by `mine` (at most one a quad) as the best hit.
+            auto const take = [&](bool mine, float t, float u, float v, float const (&ng)[3], std::uint32_t rec) {
+                auto const share = [&](float x) { return __uint_as_float(quad_or(mine ? __float_as_uint(x) : 0u)); };
+                best.t = share(t);
+                best.u = share(u);
+                best.v = share(v);
+                best.n[0] = share(ng[0]);
+                best.n[1] = share(ng[1]);
+                best.n[2] = share(ng[2]);
+                best.prim = sc.prim[quad_or(mine ? rec : 0u)];
+                best.found = true;
+            };
+            // Settles the quad's leaf triangles (this lane's: record `rec`, order `at`, entry t `tn`).
+            auto const settle = [&](bool leaf, std::uint32_t rec, std::uint32_t at, float tn) {
+                if (__ballot(leaf) == 0ull)
+                    return;
+                tri_record tr{};
+                if (leaf)
+                    tr = sc.tris[rec];
+                float t, u, v, ng[3];
+                bool const hit = triangle_candidate(r, tr, t_min, t, u, v, ng) && leaf;
+                if (!Packed && __ballot(hit && t < tn) != 0ull) {
+                    for (std::uint32_t s = 0; s < 4; ++s) {
+                        bool const mine =
+                            hit && at == s && tn <= best.t && (best.found ? t < best.t : t <= best.t);
+                        if (quad_or(mine ? 1u : 0u) != 0u)
+                            take(mine, t, u, v, ng, rec);
+                    }
+                } else {
+                    float const m = quad_min(hit ? t : INFINITY);
+                    bool const any = quad_or(hit ? 1u : 0u) != 0u;
+                    if (any && (best.found ? m < best.t : m <= best.t)) {
+                        std::uint32_t const key = hit && t == m ? at : 4u;
+                        take(key == quad_min(key) && key < 4u, t, u, v, ng, rec);
+                    }
+                }
+            };
+            std::uint32_t const child = static_cast<std::uint32_t>(ref_offset(slot.reference));
+            float tn = INFINITY;
+            bool hit = ref_valid(slot.reference);
+            if constexpr (Packed)
+                hit = hit && box_packed(r, slot.bounds, t_min, best.t, tn) && tn != INFINITY;
+            else
+                hit = hit && box_canonical(r, slot.bounds, t_min, best.t, tn);
+            bool const is_leaf = ref_leaf(slot.reference);
+            std::uint32_t const mask = Packed ? 15u : static_cast<std::uint32_t>(__ballot(hit) >> shift) & 15u;
+            std::uint64_t ties;
+            std::uint32_t const pos = near_first_position(tn, hit, mask, j, ties);
+            std::uint32_t const inner = quad_or(hit && !is_leaf ? 1u << pos : 0u);
+            // Positions that go onto the stack or, the first internal one, are entered.
+            std::uint32_t const first = inner != 0u ? static_cast<std::uint32_t>(__builtin_ctz(inner)) : 4u;
+            std::uint32_t behind = inner;
+            if constexpr (Packed)
+                behind = quad_or(hit && pos >= first ? 1u << pos : 0u);
+            bool found = inner != 0u;
+            int const count = __popc(behind);
+            int const to = sp + count - 1 - __popc(behind & ((1u << pos) - 1u));
+            bool const stacked = hit && (Packed ? pos > first : !is_leaf && pos > first);
+            if (stacked && to < Cap) {
+                st_node[to * k_ray_stride] = is_leaf ? (k_payload_leaf | child) : child;
+                st_t[to * k_ray_stride] = tn;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            std::uint32_t next = quad_or(hit && pos == first ? child : 0u);
+            float next_t = __uint_as_float(quad_or(hit && pos == first ? __float_as_uint(tn) : 0u));
+            if (found) {
+                sp += count - 1;
+                overflow = sp > Cap;
+            }
+            // Requested before the leaf triangles are evaluated.
+            bvh_child ahead = slot;
+            if (found)
+                ahead = sc.nodes[next].children[j];
+            settle(hit && is_leaf && (!Packed || pos < first), child, pos, tn);
+            found = found && !(next_t > best.t);
+            bool popped = false;
+            while (!found && sp > 0 && !overflow) {
+                // The four topmost entries: leaves are settled and excluded nodes dropped up to the first
+                // node that is neither.
+                int const e = sp - 1 - static_cast<int>(j);
+                std::uint32_t const en = e >= 0 ? st_node[e * k_ray_stride] : 0u;
+                float const et = e >= 0 ? st_t[e * k_ray_stride] : 0.0f;
+                bool const entry_leaf = Packed && e >= 0 && (en & k_payload_leaf) != 0u;
+                std::uint32_t const open =
+                    static_cast<std::uint32_t>(__ballot(e >= 0 && !entry_leaf && !(et > best.t)) >> shift) & 15u;
+                std::uint32_t const run = open != 0u ? static_cast<std::uint32_t>(__builtin_ctz(open)) : 4u;
+                if constexpr (Packed)
+                    settle(entry_leaf && j < run, en & ~k_payload_leaf, j, et);
+                if (open != 0u) {
+                    next = quad_or(j == run ? en : 0u);
+                    next_t = __uint_as_float(quad_or(j == run ? __float_as_uint(et) : 0u));
+                    found = !(next_t > best.t);
+                    popped = found;
+                    sp -= static_cast<int>(run) + 1;
+                } else {
+                    sp = sp > 4 ? sp - 4 : 0;
+                }
+            }
+            if (popped)
+                ahead = sc.nodes[next].children[j];
+            slot = ahead;
+            finished = !found || overflow;
+        }
+        std::uint64_t const ended = __ballot(finished);
+        if (ended != 0ull) {
+            if (finished) {
+                std::uint32_t const status = overflow ? 2u : (best.found ? 1u : 0u);
+                // Each lane writes two of the record's eight words.
+                std::uint32_t const lo =
+                    j == 0u ? __float_as_uint(best.found ? best.t : -1.0f)
+                            : __float_as_uint(j == 1u ? best.v : best.n[1]);
+                std::uint32_t const hi = j == 0u   ? __float_as_uint(best.u)
+                                         : j == 3u ? status
+                                                   : __float_as_uint(j == 1u ? best.n[0] : best.n[2]);
+                reinterpret_cast<uint2 *>(out + i)[j] = make_uint2(j == 3u ? best.prim : lo, hi);
+                i = nth(taken + static_cast<std::size_t>(__popcll(ended & ((1ull << shift) - 1ull)) >> 2));
+                live = i < n;
+                if (live)
+                    begin_ray();
+            }
+            taken += static_cast<std::size_t>(__popcll(ended) >> 2);
+        }
+    }
+}
+
+// Blocks of the quad traversal: two waves for each of the 8,192 that fit the chip, fewer where every quad
+// has its ray at once (4M rays on 1M triangles 3.8-3.9 ms with 2,048 to 4,096 blocks, 5.4 ms with a quad per
+// ray; on 5,120 triangles 1.88 ms with 2,048, 1.73 ms with 4,096).
+inline unsigned ray_quad_grid(std::size_t n) { return std::min(grid_for(4 * n, k_block), 4096u); }
+
 template <bool Packed, int Cap>
 void launch_ray(
     gwn_bvh_handle const &bvh, float const *ox, float const *oy, float const *oz, float const *dx,
@@ -57,6 +276,10 @@ void launch_ray(
     if (counters != nullptr)
         ray_kernel<Packed, Cap, true><<<grid_for(n, k_block), k_block, 0, stream>>>(
             sc, bvh.root.reference, ox, oy, oz, dx, dy, dz, nullptr, n, t_min, t_max, counters);
+    else if (ref_internal(bvh.root.reference))
+        ray_quad_kernel<Packed, Cap><<<ray_quad_grid(n), k_block, 0, stream>>>(
+            sc, static_cast<std::uint32_t>(ref_offset(bvh.root.reference)), ox, oy, oz, dx, dy, dz,
+            static_cast<ray_hit *>(out), n, t_min, t_max);
     else
         ray_kernel<Packed, Cap><<<grid_for(n, k_block), k_block, 0, stream>>>(
             sc, bvh.root.reference, ox, oy, oz, dx, dy, dz, static_cast<ray_hit *>(out), n, t_min, t_max);
