@@ -481,13 +481,15 @@ typedef struct gwn_batch_item {
 
 typedef struct gwn_batch_tuning {
     int32_t block_size;      /* 64, 128, 192 or 256 threads */
-    int32_t chunk;           /* queries per work item, a multiple of block_size */
+    int32_t chunk;           /* queries per work item of a wave-cooperative mesh, a multiple of
+                                block_size (four lanes per query: block_size / 4 queries) */
     int32_t blocks_per_cu;   /* persistent grid = blocks_per_cu x compute units */
-    int32_t traversal;       /* 0: one query per lane; 1: wave-cooperative over each mesh's
-                                Hilbert query order (computed at create); 2: per mesh, wave-
+    int32_t traversal;       /* 0: four lanes per query; 1: wave-cooperative over each mesh's
+                                Hilbert query order (computed at create) where the mesh's queries
+                                are dense enough for that to pay, four lanes elsewhere; 2: wave-
                                 cooperative where the mesh has at least wave_queries_per_triangle
-                                queries per triangle, one query per lane elsewhere.  All three
-                                give the same results. */
+                                queries per triangle, four lanes elsewhere.  All three give the
+                                same results. */
     int32_t stack_capacity;  /* compiled traversal stack: 32, 64 or 128, at least every tree's
                                 internal_stack_bound; 0 in gwn_batch_set_tuning keeps it */
     float wave_queries_per_triangle; /* traversal 2's density threshold (positive, finite); read

@@ -102,8 +102,12 @@ namespace {
 void layout_chunks(gwn_batch_handle &b) {
     std::uint64_t first = 0;
     for (auto &m : b.host_meshes) {
+        // Four lanes per query: as many as a block holds at once, for queries of a large tree take long
+        // and a chunk of more of them can be the launch's last (128 meshes: 4.12 ms, with half a
+        // whole-wave chunk of 1,024 4.39; 8 meshes: 1.28, 1.51).
+        m.chunk = static_cast<std::uint32_t>(m.wave != 0u ? b.chunk : b.block / 4);
         m.first_chunk = first;
-        first += (m.count + static_cast<std::uint64_t>(b.chunk) - 1) / static_cast<std::uint64_t>(b.chunk);
+        first += (m.count + m.chunk - 1) / m.chunk;
     }
     b.total_chunks = first;
 }
@@ -119,21 +123,24 @@ void note_work(gwn_batch_handle &b, hipStream_t stream) {
     b.have_work = true;
 }
 
-// Traversal 2: a mesh with a query order and at least wave_queries_per_triangle queries per
-// triangle walks its tree wave-cooperatively, the rest one query per lane.
+// Traversal 1: the meshes whose queries are dense (batch_dense_queries) walk their trees
+// wave-cooperatively; 2: those with at least wave_queries_per_triangle queries per triangle.  The rest,
+// meshes without a query order and traversal 0 take four lanes per query.
 void set_wave_flags(gwn_batch_handle &b) {
     for (std::size_t i = 0; i < b.host_meshes.size(); ++i) {
         batch_mesh &m = b.host_meshes[i];
-        bool const dense = static_cast<double>(m.count) >=
-                           static_cast<double>(b.wave_queries_per_triangle) * static_cast<double>(b.mesh_triangles[i]);
-        m.wave = b.traversal == 1 || (b.traversal == 2 && m.order != nullptr && dense) ? 1u : 0u;
+        bool const dense =
+            b.traversal == 1 ? batch_dense_queries(b.mesh_triangles[i], m.count, b.accuracy_scale)
+                             : static_cast<double>(m.count) >= static_cast<double>(b.wave_queries_per_triangle) *
+                                                                   static_cast<double>(b.mesh_triangles[i]);
+        m.wave = b.traversal != 0 && m.order != nullptr && dense ? 1u : 0u;
     }
 }
 
 void upload_table(gwn_batch_handle &b, hipStream_t stream) {
     wait_last_work(b);
-    layout_chunks(b);
     set_wave_flags(b);
+    layout_chunks(b);
     GWN_HIP(hipMemcpyAsync(b.meshes.ptr, b.host_meshes.data(), b.host_meshes.size() * sizeof(batch_mesh),
                            hipMemcpyHostToDevice, stream));
     GWN_HIP(hipStreamSynchronize(stream));
@@ -188,8 +195,7 @@ void enqueue_query(gwn_batch_handle &b, hipStream_t stream) {
     fill_u32(reinterpret_cast<std::uint32_t *>(b.counter.ptr), 0u, 2, stream);
     int const grid = std::max(1, b.blocks_per_cu * b.cu_count);
     taylor_batch_launch(b.meshes.ptr, static_cast<std::uint32_t>(b.host_meshes.size()), b.total_chunks,
-                        static_cast<std::uint32_t>(b.chunk), b.accuracy_scale, b.counter.ptr, b.order, b.cap,
-                        b.block, grid, b.traversal, stream);
+                        b.accuracy_scale, b.counter.ptr, b.order, b.cap, b.block, grid, b.traversal != 0, stream);
 }
 
 // The refit table: every mesh with an internal root, and for every depth the meshes' node ranges
@@ -399,12 +405,12 @@ void batch_set_tuning(gwn_batch_handle &b, int block, int chunk, int blocks_per_
     if (stack_capacity != 0 && static_cast<std::uint32_t>(stack_capacity) < b.stack_bound)
         throw_invalid("Batched query stack capacity is below a tree's traversal stack bound.");
     if (traversal < 0 || traversal > 2)
-        throw_invalid("Batched query traversal must be 0 (per lane), 1 (wave) or 2 (per mesh).");
+        throw_invalid("Batched query traversal must be 0 (four lanes), 1 (wave) or 2 (per mesh).");
     if (traversal == 2 && !(wave_queries_per_triangle > 0.0f && std::isfinite(wave_queries_per_triangle)))
         throw_invalid("Batched query wave_queries_per_triangle must be positive and finite for traversal 2.");
     // The graph and any query in flight read the table and the counter: finish them first.
     wait_last_work(b);
-    bool const relayout = chunk != b.chunk || traversal != b.traversal ||
+    bool const relayout = chunk != b.chunk || block != b.block || traversal != b.traversal ||
                           (traversal == 2 && wave_queries_per_triangle != b.wave_queries_per_triangle);
     b.block = block;
     b.chunk = chunk;

@@ -337,15 +337,18 @@ struct batch_mesh {
     std::uint64_t count;
     std::uint64_t first_chunk;   // exclusive prefix of chunk counts over earlier meshes
     std::uint32_t const *order;  // visiting order of the queries (Hilbert), or null
-    std::uint32_t wave;          // per-mesh traversal (traversal 2): 1 wave-cooperative, 0 per lane
+    std::uint32_t wave;          // 1 wave-cooperative, 0 four lanes per query
+    std::uint32_t chunk;         // queries a block takes at a time
 };
 // Persistent batched Taylor winding (plain precision): `grid` blocks of `block` threads take
-// chunks of `chunk` queries from *counter (which must be zero) until total_chunks are done.
+// chunks of their mesh's `chunk` queries from *counter (which must be zero) until total_chunks are done.
+// `waves`: whether any mesh has its wave flag set.
 void taylor_batch_launch(
-    batch_mesh const *meshes, std::uint32_t mesh_count, std::uint64_t total_chunks, std::uint32_t chunk,
-    float accuracy_scale, std::uint64_t *counter, int order, int cap, int block, int grid, int traversal,
-    hipStream_t stream
+    batch_mesh const *meshes, std::uint32_t mesh_count, std::uint64_t total_chunks, float accuracy_scale,
+    std::uint64_t *counter, int order, int cap, int block, int grid, bool waves, hipStream_t stream
 );
+// Whether a batch walks a mesh of `triangles` with whole waves (its queries are dense enough).
+bool batch_dense_queries(std::size_t triangles, std::size_t queries, float accuracy_scale);
 // Segmented builds (gwn_batch_build.hip): the H-PLOC BVH trees and Taylor moments of many meshes,
 // built side by side in one pass of a fixed sequence of launches that allocates nothing and never
 // reads back to the host, so the whole pass can be captured into a graph.  Each mesh's tree,

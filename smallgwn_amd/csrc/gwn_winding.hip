@@ -368,21 +368,33 @@ __device__ inline bool taylor_wave_traverse(
     std::uint32_t &n_accept, std::uint32_t &n_leaf, std::uint32_t *s_node, std::uint64_t *s_mask
 );
 
-// Batched persistent traversal: many meshes, one launch.  Work is a list of chunks of `chunk`
-// consecutive queries of one mesh; every block takes chunks from a global counter until none is
-// left (no wave waits for another), and its lanes evaluate one query each with that mesh's
-// records and the per-lane traversal above, so each result equals the single-mesh batch's.
-// Mode 0: one query per lane; 1: wave-cooperative; 2: each mesh as its `wave` flag says (a wave
-// walks the union of its lanes' paths, which pays where a mesh's queries are dense and costs
-// where a few queries are spread over a large tree).  Every mode gives the same results.
-template <int Order, int StackCap, int Mode>
+// Four lanes per query (defined below; the batched kernel uses it too).
+template <int Order, int Prec, bool Grad, int StackCap>
+__device__ inline bool taylor_quad_traverse(
+    float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node, float x, float y,
+    float z, float beta2, taylor_sums<Prec, Grad> &acc, std::uint32_t &n_tests, std::uint32_t &n_accept,
+    std::uint32_t &n_leaf, std::uint32_t *stack, int stride
+);
+
+// Batched persistent traversal: many meshes, one launch.  Work is a list of chunks of consecutive
+// queries of one mesh (the mesh's `chunk` of them); every block takes chunks from a global counter
+// until none is left (no wave waits for another) and evaluates them with that mesh's records and the
+// traversals of the single-mesh batch, so each result equals that batch's.  A mesh whose `wave` flag
+// is set is walked by whole waves, any other with four lanes per query (a wave walks the union of its
+// lanes' paths, which pays where a mesh's queries are dense and costs where a few queries are spread
+// over a large tree: one such wave alone can last as long as the rest of the launch).  Waves: whether
+// any mesh may have its flag set.  Rebuild and query of 128 meshes of up to 100,000 triangles, recorded:
+// 8.04 ms with whole waves for every mesh, 4.16 now (2.36M queries in all); of 8 meshes with 174,131:
+// 4.69, 1.28; of 512 with 9.0M: 14.2, 11.5.
+template <int Order, int StackCap, bool Waves>
 __global__ __launch_bounds__(256) void taylor_batch_kernel(
-    batch_mesh const *__restrict__ meshes, std::uint32_t mesh_count, std::uint64_t total_chunks, std::uint32_t chunk,
-    float beta2, std::uint64_t *counter
+    batch_mesh const *__restrict__ meshes, std::uint32_t mesh_count, std::uint64_t total_chunks, float beta2,
+    std::uint64_t *counter
 ) {
     __shared__ std::uint64_t s_chunk;
-    __shared__ std::uint32_t s_node[4][Mode != 0 ? StackCap : 1];
-    __shared__ std::uint64_t s_mask[4][Mode != 0 ? StackCap : 1];
+    __shared__ std::uint32_t s_node[4][Waves ? StackCap : 1];
+    __shared__ std::uint64_t s_mask[4][Waves ? StackCap : 1];
+    __shared__ std::uint32_t s_quad[StackCap * 64];  // entry e of quad k's stack at [e * 64 + k]
     int const wave = threadIdx.x >> 6;
     for (;;) {
         if (threadIdx.x == 0)
@@ -402,8 +414,24 @@ __global__ __launch_bounds__(256) void taylor_batch_kernel(
                 hi = mid;
         }
         batch_mesh const m = meshes[lo];
+        std::uint32_t const chunk = m.chunk;
         std::uint64_t const base = (c - m.first_chunk) * chunk;
-        bool const leaf_root = ref_leaf(m.root);
+        if (!ref_leaf(m.root) && !(Waves && m.wave != 0u)) {  // uniform over the block
+            for (std::uint32_t t = threadIdx.x >> 2; t < chunk; t += blockDim.x >> 2) {  // whole quads
+                std::uint64_t const p = base + t;
+                if (p >= m.count)
+                    break;
+                std::uint64_t const q = m.order ? m.order[p] : p;
+                taylor_sums<GWN_PRECISION_PLAIN, false> acc;
+                std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;
+                bool const overflow = taylor_quad_traverse<Order, GWN_PRECISION_PLAIN, false, StackCap>(
+                    m.records, m.tris, static_cast<std::uint32_t>(ref_offset(m.root)), m.qx[q], m.qy[q], m.qz[q], beta2,
+                    acc, n_tests, n_accept, n_leaf, s_quad + (threadIdx.x >> 2), 64);
+                if ((threadIdx.x & 3u) == 0u)
+                    acc.store(overflow, q, m.out, nullptr, nullptr, nullptr);
+            }
+            continue;
+        }
         // Whole waves step through the chunk together, so the wave traversal sees uniform meshes.
         for (std::uint32_t t = threadIdx.x; t - (threadIdx.x & 63u) < chunk; t += blockDim.x) {
             std::uint64_t const p = base + t;
@@ -411,31 +439,23 @@ __global__ __launch_bounds__(256) void taylor_batch_kernel(
             std::uint64_t const q = active ? (m.order ? m.order[p] : p) : 0;
             float const x = active ? m.qx[q] : 0.0f, y = active ? m.qy[q] : 0.0f, z = active ? m.qz[q] : 0.0f;
             taylor_sums<GWN_PRECISION_PLAIN, false> acc;
-            std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;
             bool overflow = false;
-            if (leaf_root) {
+            if (ref_leaf(m.root)) {
                 if (!active)
                     continue;
                 std::uint64_t const off = ref_offset(m.root);
                 std::uint32_t const cnt = ref_count(m.root);
                 for (std::uint32_t k = 0; k < cnt; ++k)
                     acc.leaf(m.tris[off + k], x, y, z);
-            } else if (Mode == 1 || (Mode == 2 && m.wave != 0u)) {  // uniform over the block
-                if constexpr (Mode != 0) {
-                    if (__ballot(active) == 0ull)
-                        continue;
-                    overflow = taylor_wave_traverse<Order, GWN_PRECISION_PLAIN, false, StackCap, false>(
-                        m.records, m.tris, static_cast<std::uint32_t>(ref_offset(m.root)), active, x, y, z, beta2,
-                        acc, n_tests, n_accept, n_leaf, s_node[wave], s_mask[wave]);
-                    if (!active)
-                        continue;
-                }
-            } else {
+            } else if constexpr (Waves) {
+                if (__ballot(active) == 0ull)
+                    continue;
+                std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;
+                overflow = taylor_wave_traverse<Order, GWN_PRECISION_PLAIN, false, StackCap, false>(
+                    m.records, m.tris, static_cast<std::uint32_t>(ref_offset(m.root)), active, x, y, z, beta2, acc,
+                    n_tests, n_accept, n_leaf, s_node[wave], s_mask[wave]);
                 if (!active)
                     continue;
-                overflow = taylor_traverse<Order, GWN_PRECISION_PLAIN, false, StackCap>(
-                    m.records, m.tris, static_cast<std::uint32_t>(ref_offset(m.root)), x, y, z, beta2, acc, n_tests,
-                    n_accept, n_leaf);
             }
             acc.store(overflow, q, m.out, nullptr, nullptr, nullptr);
         }
@@ -744,24 +764,14 @@ template <int Order, bool Grad> struct slot_test {
 // they are evaluated with more lanes active (5-20 %); handing a finished quad another query of the wave
 // (0-40 %: a wave's queries are then no longer neighbours, and their reads no longer shared).
 template <int Order, int Prec, bool Grad, int StackCap>
-__global__ __launch_bounds__(k_taylor_block) void taylor_quad_kernel(
-    float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node,
-    float const *__restrict__ qx, float const *__restrict__ qy, float const *__restrict__ qz,
-    std::uint32_t const *__restrict__ order, taylor_outputs o, std::size_t n, float beta2
+__device__ inline bool taylor_quad_traverse(
+    float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node, float x, float y,
+    float z, float beta2, taylor_sums<Prec, Grad> &acc, std::uint32_t &n_tests, std::uint32_t &n_accept,
+    std::uint32_t &n_leaf, std::uint32_t *stack, int stride
 ) {
     using slot_type = quad_slot<Order, Grad>;
-    constexpr int k_quads = k_taylor_block / 4;
-    __shared__ std::uint32_t s_stack[StackCap * k_quads];  // entry e of quad k at [e * k_quads + k]
-    std::size_t const i = (static_cast<std::size_t>(blockIdx.x) * k_taylor_block + threadIdx.x) >> 2;
-    if (i >= n)
-        return;  // whole quads
     int const j = static_cast<int>(threadIdx.x & 3);
     int const shift = static_cast<int>(threadIdx.x & 60);
-    std::uint32_t *const stack = s_stack + (threadIdx.x >> 2);
-    std::size_t const q = order ? order[i] : i;
-    float const x = qx[q], y = qy[q], z = qz[q];
-    taylor_sums<Prec, Grad> acc;
-    std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;  // this lane's
     int sp = 0;
     bool overflow = false;
     bool live = true;
@@ -783,14 +793,14 @@ __global__ __launch_bounds__(k_taylor_block) void taylor_quad_kernel(
         std::uint32_t next = bits & 8u ? c3 : (bits & 4u ? c2 : (bits & 2u ? c1 : c0));
         int const at = sp + __popc(bits & ((1u << j) - 1u));
         if (v.inner && (bits >> j) != 1u && at < StackCap)
-            stack[at * k_quads] = c;
+            stack[at * stride] = c;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         if (pushed >= 0) {
             sp += pushed;
             overflow = sp > StackCap;
             live = !overflow;
         } else if (sp > 0) {
-            next = stack[--sp * k_quads];
+            next = stack[--sp * stride];
         } else {
             live = false;
         }
@@ -802,6 +812,27 @@ __global__ __launch_bounds__(k_taylor_block) void taylor_quad_kernel(
             term.leaf(t, x, y, z);
         add_terms<4>(acc, term);
     }
+    return overflow;
+}
+
+template <int Order, int Prec, bool Grad, int StackCap>
+__global__ __launch_bounds__(k_taylor_block) void taylor_quad_kernel(
+    float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node,
+    float const *__restrict__ qx, float const *__restrict__ qy, float const *__restrict__ qz,
+    std::uint32_t const *__restrict__ order, taylor_outputs o, std::size_t n, float beta2
+) {
+    constexpr int k_quads = k_taylor_block / 4;
+    __shared__ std::uint32_t s_stack[StackCap * k_quads];  // entry e of quad k at [e * k_quads + k]
+    std::size_t const i = (static_cast<std::size_t>(blockIdx.x) * k_taylor_block + threadIdx.x) >> 2;
+    if (i >= n)
+        return;  // whole quads
+    int const j = static_cast<int>(threadIdx.x & 3);
+    std::size_t const q = order ? order[i] : i;
+    taylor_sums<Prec, Grad> acc;
+    std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;  // this lane's
+    bool const overflow = taylor_quad_traverse<Order, Prec, Grad, StackCap>(
+        records, tris, root_node, qx[q], qy[q], qz[q], beta2, acc, n_tests, n_accept, n_leaf,
+        s_stack + (threadIdx.x >> 2), k_quads);
     if (j == 0)
         acc.store(overflow, q, o.out, o.gx, o.gy, o.gz);
     if (o.counters != nullptr) {
@@ -1429,12 +1460,11 @@ void launch_taylor_adjoint(
     GWN_LAUNCH_CHECK();
 }
 
-template <int Order, int Mode>
-void launch_batch_cap(batch_mesh const *meshes, std::uint32_t mesh_count, std::uint64_t total_chunks,
-                      std::uint32_t chunk, float beta2, std::uint64_t *counter, int cap, int block, int grid,
-                      hipStream_t stream) {
-#define GWN_BATCH(C)                                                                                      \
-    taylor_batch_kernel<Order, C, Mode><<<grid, block, 0, stream>>>(meshes, mesh_count, total_chunks, chunk, beta2, counter)
+template <int Order, bool Waves>
+void launch_batch_cap(batch_mesh const *meshes, std::uint32_t mesh_count, std::uint64_t total_chunks, float beta2,
+                      std::uint64_t *counter, int cap, int block, int grid, hipStream_t stream) {
+#define GWN_BATCH(C) \
+    taylor_batch_kernel<Order, C, Waves><<<grid, block, 0, stream>>>(meshes, mesh_count, total_chunks, beta2, counter)
     if (cap <= 32)
         GWN_BATCH(32);
     else if (cap <= 64)
@@ -1449,23 +1479,27 @@ void launch_batch_cap(batch_mesh const *meshes, std::uint32_t mesh_count, std::u
 
 } // namespace
 
+// The single-mesh rule, or 32 queries per triangle at beta 2: among many meshes the chip is full and the
+// work decides, not the longest wave, so small meshes' wave walks pay earlier.  2,048 meshes of up to
+// 2,000 triangles with up to 400,000 queries: 23.6 ms by the single-mesh rule alone, 20.4 from 16 queries
+// per triangle on, 21.3 from 64; 512 of up to 20,000 with 100,000: 3.84, 3.82, 3.70; 128 of up to 100,000
+// with 400,000: 2.54, 2.83, 2.44.
+bool batch_dense_queries(std::size_t triangles, std::size_t queries, float accuracy_scale) {
+    double const beta = std::max(1.0, double(accuracy_scale));
+    return dense_queries(triangles, queries, accuracy_scale * accuracy_scale) ||
+           double(queries) >= 32.0 * double(triangles) * std::pow(2.0 / beta, 1.5);
+}
+
 void taylor_batch_launch(
-    batch_mesh const *meshes, std::uint32_t mesh_count, std::uint64_t total_chunks, std::uint32_t chunk,
-    float accuracy_scale, std::uint64_t *counter, int order, int cap, int block, int grid, int traversal,
-    hipStream_t stream
+    batch_mesh const *meshes, std::uint32_t mesh_count, std::uint64_t total_chunks, float accuracy_scale,
+    std::uint64_t *counter, int order, int cap, int block, int grid, bool waves, hipStream_t stream
 ) {
     float const beta2 = accuracy_scale * accuracy_scale;
     if (block <= 0 || block > 256 || (block & 63) != 0)
         throw_invalid("Batched query block size must be 64, 128, 192 or 256.");
-    if (traversal < 0 || traversal > 2)
-        throw_invalid("Batched query traversal must be 0 (per lane), 1 (wave) or 2 (per mesh).");
-#define GWN_BATCH_ORDER(O)                                                                                      \
-    (traversal == 0   ? launch_batch_cap<O, 0>(meshes, mesh_count, total_chunks, chunk, beta2, counter, cap, block, \
-                                               grid, stream)                                                     \
-     : traversal == 1 ? launch_batch_cap<O, 1>(meshes, mesh_count, total_chunks, chunk, beta2, counter, cap, block, \
-                                               grid, stream)                                                     \
-                      : launch_batch_cap<O, 2>(meshes, mesh_count, total_chunks, chunk, beta2, counter, cap, block, \
-                                               grid, stream))
+#define GWN_BATCH_ORDER(O)                                                                                     \
+    (waves ? launch_batch_cap<O, true>(meshes, mesh_count, total_chunks, beta2, counter, cap, block, grid, stream) \
+           : launch_batch_cap<O, false>(meshes, mesh_count, total_chunks, beta2, counter, cap, block, grid, stream))
     switch (order) {
     case 0: GWN_BATCH_ORDER(0); break;
     case 1: GWN_BATCH_ORDER(1); break;

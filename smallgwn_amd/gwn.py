@@ -945,9 +945,9 @@ class BatchObject:
 
     def set_tuning(self, block_size: int, chunk: int, blocks_per_cu: int, traversal: int = 0,
                    stack_capacity: int = 0, wave_queries_per_triangle: float = 1.0, stream=None) -> Status:
-        """traversal 0: one query per lane; 1: wave-cooperative over each mesh's Hilbert order;
-        2: wave-cooperative for meshes with at least wave_queries_per_triangle queries per
-        triangle, one query per lane for the rest.  stack_capacity: 0 keeps the compiled
+        """traversal 0: four lanes per query; 1: wave-cooperative over each mesh's Hilbert order
+        for meshes whose queries are dense enough for it to pay; 2: for meshes with at least
+        wave_queries_per_triangle queries per triangle; four lanes per query for the rest.  stack_capacity: 0 keeps the compiled
         traversal stack, else 32, 64 or 128."""
         t = _BatchTuning(block_size, chunk, blocks_per_cu, traversal, stack_capacity, wave_queries_per_triangle,
                          0, 0)
