@@ -3,7 +3,7 @@
 // Replaces the CUB DeviceRadixSort::SortPairs calls of the reference build
 // (include/gwn/detail/gwn_bvh_build_common.cuh:325-347, gwn_bvh_reorder.cuh:104-116).
 //
-// Design (reduce-then-scan, 8-bit digits, 4096-key tiles of one 256-thread block):
+// Design (reduce-then-scan, 8-bit digits, tiles of 1,024 to 4,096 keys of one 256-thread block):
 //   1. one histogram sweep counts every digit of every pass at once, and one scan turns the
 //      counts into per-pass digit bases;
 //   2. per pass, a count kernel records each tile's digit counts (digit-major table), a scan
@@ -22,8 +22,15 @@ namespace {
 constexpr int k_sort_block = 256;
 constexpr int k_sort_waves = k_sort_block / 64;
 constexpr int k_radix = 256;
-constexpr int k_items = 16;
-constexpr int k_tile = k_sort_block * k_items;
+// Keys a thread takes.  A thread ranks its keys one after the other (each waits for the counters that
+// the one before it left in LDS), so few keys per thread shorten a pass while tiles of them leave the
+// chip idle; more of them write longer runs and scan fewer tile counts.  64-bit keys, 63 bits, 16 / 8 /
+// 4 / 2 keys per thread: 65,537 keys 192 / 147 / 122 / 133 us; 262,144 202 / 160 / 142 / 160; 500,009
+// 219 / 174 / 175 / 212; 1,000,003 230 / 218 / 245 / 335; 4,000,000 472 / 505 / 637 / 887.
+// The lines keep the tile table of a sort of up to 2^20 keys within 256 tiles, the scratch that callers
+// who bring their own have laid out for it.
+constexpr int k_items_large = 16, k_items_medium = 8, k_items_small = 4;
+constexpr std::size_t k_medium_sort = std::size_t(1) << 19, k_small_sort = std::size_t(1) << 18;
 constexpr int k_max_passes = 8;
 
 constexpr std::size_t k_max_sort_count = (std::size_t(1) << 31) - 1u;
@@ -104,7 +111,7 @@ __global__ __launch_bounds__(k_sort_block) void scan_histogram_kernel(std::uint3
 // wave*64*k_items + it*64 + l of the tile, so ranking items in (it, lane) order ranks elements
 // in input order.  For each item, `match` is the set of lanes holding the same digit; the lowest
 // such lane advances the wave's digit counter.
-template <class Key>
+template <class Key, int k_items>
 __device__ inline void rank_tile_items(
     Key const (&key)[k_items], int tile_count, int wave_base, int shift, unsigned digit_mask,
     std::uint32_t *wave_count, std::uint32_t (&rank)[k_items]
@@ -136,11 +143,12 @@ __device__ inline void rank_tile_items(
 }
 
 // counts[d * tiles + t] = number of keys of tile t whose digit is d.
-template <class Key>
+template <class Key, int k_items>
 __global__ __launch_bounds__(k_sort_block) void tile_count_kernel(
     Key const *__restrict__ keys, std::size_t n, int shift, unsigned digit_mask, std::uint32_t tiles,
     std::uint32_t *__restrict__ counts
 ) {
+    constexpr int k_tile = k_sort_block * k_items;
     __shared__ std::uint32_t s_count[k_sort_waves][k_radix];
     int const lane = threadIdx.x & 63;
     int const wave = threadIdx.x >> 6;
@@ -158,7 +166,7 @@ __global__ __launch_bounds__(k_sort_block) void tile_count_kernel(
         key[it] = local < tile_count ? keys[tile_begin + local] : Key(0);
     }
     std::uint32_t rank[k_items];
-    rank_tile_items<Key>(key, tile_count, wave_base, shift, digit_mask, s_count[wave], rank);
+    rank_tile_items(key, tile_count, wave_base, shift, digit_mask, s_count[wave], rank);
     __syncthreads();
     std::uint32_t total = 0;
 #pragma unroll
@@ -186,7 +194,7 @@ __global__ __launch_bounds__(k_sort_block) void tile_scan_kernel(
     }
 }
 
-template <class Key> struct scatter_smem {
+template <class Key, int k_tile> struct scatter_smem {
     Key keys[k_tile];
     std::uint32_t vals[k_tile];
     std::uint32_t wave_count[k_sort_waves][k_radix];
@@ -195,13 +203,14 @@ template <class Key> struct scatter_smem {
     std::uint32_t wave_totals[k_sort_waves];
 };
 
-template <class Key>
+template <class Key, int k_items>
 __global__ __launch_bounds__(k_sort_block) void scatter_kernel(
     Key const *__restrict__ keys_in, Key *__restrict__ keys_out,
     std::uint32_t const *__restrict__ vals_in, std::uint32_t *__restrict__ vals_out, std::size_t n,
     int shift, unsigned digit_mask, std::uint32_t tiles, std::uint32_t const *__restrict__ offsets
 ) {
-    __shared__ scatter_smem<Key> s;
+    constexpr int k_tile = k_sort_block * k_items;
+    __shared__ scatter_smem<Key, k_tile> s;
     int const lane = threadIdx.x & 63;
     int const wave = threadIdx.x >> 6;
     for (int i = threadIdx.x; i < k_sort_waves * k_radix; i += k_sort_block)
@@ -223,7 +232,7 @@ __global__ __launch_bounds__(k_sort_block) void scatter_kernel(
         key[it] = valid ? keys_in[tile_begin + local] : Key(0);
         val[it] = valid ? vals_in[tile_begin + local] : 0u;
     }
-    rank_tile_items<Key>(key, tile_count, wave_base, shift, digit_mask, s.wave_count[wave], rank);
+    rank_tile_items(key, tile_count, wave_base, shift, digit_mask, s.wave_count[wave], rank);
     __syncthreads();
 
     // One thread per digit: per-wave prefixes and the tile's digit total.
@@ -268,7 +277,29 @@ std::size_t sort_base_words(int begin_bit, int end_bit) {
     return static_cast<std::size_t>((end_bit - begin_bit + 7) / 8) * k_radix;
 }
 
-std::size_t sort_table_words(std::size_t n) { return (n + k_tile - 1) / k_tile * k_radix; }
+std::size_t sort_tiles(std::size_t n, int items) {
+    std::size_t const tile = std::size_t(k_sort_block) * static_cast<std::size_t>(items);
+    return (n + tile - 1) / tile;
+}
+// Holds the table of every sort of at most n elements.
+std::size_t sort_table_words(std::size_t n) {
+    return std::max({sort_tiles(n, k_items_large), sort_tiles(std::min(n, k_medium_sort), k_items_medium),
+                     sort_tiles(std::min(n, k_small_sort), k_items_small)}) *
+           k_radix;
+}
+
+template <class Key, int Items>
+void sort_pass(
+    Key const *kin, Key *kout, std::uint32_t const *vin, std::uint32_t *vout, std::size_t n, int shift, unsigned mask,
+    std::uint32_t tiles, std::uint32_t *table, std::uint32_t const *digit_base, hipStream_t stream
+) {
+    tile_count_kernel<Key, Items><<<tiles, k_sort_block, 0, stream>>>(kin, n, shift, mask, tiles, table);
+    GWN_LAUNCH_CHECK();
+    tile_scan_kernel<<<k_radix, k_sort_block, 0, stream>>>(table, tiles, digit_base);
+    GWN_LAUNCH_CHECK();
+    scatter_kernel<Key, Items><<<tiles, k_sort_block, 0, stream>>>(kin, kout, vin, vout, n, shift, mask, tiles, table);
+    GWN_LAUNCH_CHECK();
+}
 
 template <class Key>
 void radix_sort_pairs(
@@ -285,7 +316,8 @@ void radix_sort_pairs(
     int const passes = (end_bit - begin_bit + 7) / 8;
     if (passes > k_max_passes)
         throw_invalid("radix sort: bit range exceeds the key width.");
-    std::size_t const tiles = (n + k_tile - 1) / k_tile;
+    int const items = n <= k_small_sort ? k_items_small : n <= k_medium_sort ? k_items_medium : k_items_large;
+    std::size_t const tiles = sort_tiles(n, items);
     std::size_t const base_words = sort_base_words(begin_bit, end_bit);
     device_buffer<std::uint32_t> own;
     if (workspace == nullptr) {
@@ -310,12 +342,12 @@ void radix_sort_pairs(
         int const shift = begin_bit + 8 * p;
         int const width = end_bit - shift < 8 ? end_bit - shift : 8;
         unsigned const mask = (1u << width) - 1u;
-        tile_count_kernel<Key><<<ntiles, k_sort_block, 0, stream>>>(kin, n, shift, mask, ntiles, table);
-        GWN_LAUNCH_CHECK();
-        tile_scan_kernel<<<k_radix, k_sort_block, 0, stream>>>(table, ntiles, hist + p * k_radix);
-        GWN_LAUNCH_CHECK();
-        scatter_kernel<Key><<<ntiles, k_sort_block, 0, stream>>>(kin, kout, vin, vout, n, shift, mask, ntiles, table);
-        GWN_LAUNCH_CHECK();
+        if (items == k_items_small)
+            sort_pass<Key, k_items_small>(kin, kout, vin, vout, n, shift, mask, ntiles, table, hist + p * k_radix, stream);
+        else if (items == k_items_medium)
+            sort_pass<Key, k_items_medium>(kin, kout, vin, vout, n, shift, mask, ntiles, table, hist + p * k_radix, stream);
+        else
+            sort_pass<Key, k_items_large>(kin, kout, vin, vout, n, shift, mask, ntiles, table, hist + p * k_radix, stream);
         std::swap(kin, kout);
         std::swap(vin, vout);
     }
