@@ -79,8 +79,11 @@ __device__ inline bool triangle_candidate(
 //     (leaves too) onto the stack; up to four leaves from the top of the stack are settled at a time.
 // The stack (the quad's column of an LDS array) keeps the slab entry t of each child, and an internal child
 // beyond the best hit is dropped when popped: its children's boxes lie inside its own and every operation
-// of the slab test is monotone in the bounds, so they would all have missed.  A wave hands its next ray to a
-// quad that has finished (18 nodes a ray on average, 500 at most on the 1M-triangle mesh).
+// of the slab test is monotone in the bounds, so they would all have missed.  The packed test is not where
+// a direction component's reciprocal is infinite: a side of a child's box in the origin's plane gives
+// 0 * inf, and that child is met at any t.  Such rays drop nothing.  (The canonical test skips an axis
+// with such a product, so a child's entry is still no nearer than its parent's.)  A wave hands its next ray
+// to a quad that has finished (18 nodes a ray on average, 500 at most on the 1M-triangle mesh).
 //
 // One ray per lane was bound by the gathers: each of a node's eight 16-byte loads touched 64 lines a
 // wave, and its stack lived in scratch memory; a quad reads a node's 128 bytes in two.  Measured, one lane per
@@ -109,6 +112,7 @@ __global__ __launch_bounds__(k_block) void ray_quad_kernel(
     ray_state r{};
     best_hit best{};
     int sp = 0;
+    [[maybe_unused]] bool keep = false;  // packed: a reciprocal is infinite
     bvh_child slot{};
     auto const begin_ray = [&] {
         r.o[0] = ox[i];
@@ -129,6 +133,8 @@ __global__ __launch_bounds__(k_block) void ray_quad_kernel(
             r.inv[k] = r.zero[k] ? 0.0f : 1.0f / r.d[k];
         }
         r.parallel = r.zero[0] || r.zero[1] || r.zero[2];
+        if constexpr (Packed)
+            keep = fmaxf(fmaxf(fabsf(r.inv[0]), fabsf(r.inv[1])), fabsf(r.inv[2])) == INFINITY;
     };
     if (live)
         begin_ray();
@@ -193,14 +199,16 @@ __global__ __launch_bounds__(k_block) void ray_quad_kernel(
             bool found = inner != 0u;
             int const count = __popc(behind);
             int const to = sp + count - 1 - __popc(behind & ((1u << pos) - 1u));
+            // The t beyond which the child is dropped.
+            float const bound = Packed && keep ? -INFINITY : tn;
             bool const stacked = hit && (Packed ? pos > first : !is_leaf && pos > first);
             if (stacked && to < Cap) {
                 st_node[to * k_ray_stride] = is_leaf ? (k_payload_leaf | child) : child;
-                st_t[to * k_ray_stride] = tn;
+                st_t[to * k_ray_stride] = bound;
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             std::uint32_t next = quad_or(hit && pos == first ? child : 0u);
-            float next_t = __uint_as_float(quad_or(hit && pos == first ? __float_as_uint(tn) : 0u));
+            float next_t = __uint_as_float(quad_or(hit && pos == first ? __float_as_uint(bound) : 0u));
             if (found) {
                 sp += count - 1;
                 overflow = sp > Cap;

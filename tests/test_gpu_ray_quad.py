@@ -61,3 +61,30 @@ def test_rays_handed_out_within_a_wave(gwn, orc, dev, canonical):
     for k in (0, 262140, 695001):
         _same(got[k:k + 5000], _rays(gwn, dev, bvh, o[k:k + 5000], d[k:k + 5000], stack=stack))
     _same(got[::997], _oracle(orc, mesh, o[::997], d[::997], stack=stack))
+
+
+@pytest.mark.parametrize("canonical", [False, True])
+@pytest.mark.parametrize("seed", [0, 2, 4, 10])
+def test_directions_with_infinite_reciprocals(gwn, orc, dev, seed, canonical):
+    """Subnormal direction components and origins in the planes of flat boxes: a child's slab test gives 0 * inf and
+    meets the box at any t, so no entry beyond the best hit may be dropped by its own box's t."""
+    r = np.random.default_rng(100 + seed)
+    count, side = int(r.integers(40, 600)), int(r.integers(2, 6))
+    tri = np.repeat(r.integers(0, side + 1, (count, 3))[:, None], 3, 1)
+    axis = r.integers(0, 3, count)
+    for k in (1, 2):
+        off = r.integers(-2, 3, (count, 3))
+        off[np.arange(count), axis] = 0
+        tri[:, k] += off
+    v, f = tri.reshape(-1, 3).astype(np.float32), np.arange(3 * count).reshape(-1, 3).astype(np.uint32)
+    mesh = synth.Mesh(*(np.ascontiguousarray(v[:, k]) for k in range(3)), *(np.ascontiguousarray(f[:, k]) for k in range(3)))
+    _, bvh = build_gpu(gwn, mesh)
+    info = bvh.info()
+    stack = info["internal_stack_bound"] if canonical else max(64, info["packed_stack_bound"])
+    n = 300000
+    o = r.integers(-4, 2 * side + 5, (n, 3)) / 2.0
+    d = r.integers(-2, 3, (n, 3)).astype(np.float64)
+    d = np.where(r.random((n, 3)) < 0.5, r.choice([1e-40, -1e-40, 3e-39, -1e-44], (n, 3)), d)
+    o, d = o.astype(np.float32), d.astype(np.float32)
+    for t_min in (0.0, -5.0, -float("inf")):
+        _same(_rays(gwn, dev, bvh, o, d, t_min, stack=stack), _oracle(orc, mesh, o, d, t_min, stack=stack))
