@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "gwn_core.hpp"
+#include "gwn_slices.hpp"
 #include "../../include/gwn/detail/gwn_device_winding.hpp"
 
 #include <algorithm>
@@ -819,11 +820,11 @@ template <int Order, int Prec, bool Grad, int StackCap>
 __global__ __launch_bounds__(k_taylor_block) void taylor_quad_kernel(
     float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node,
     float const *__restrict__ qx, float const *__restrict__ qy, float const *__restrict__ qz,
-    std::uint32_t const *__restrict__ order, taylor_outputs o, std::size_t n, float beta2
+    std::uint32_t const *__restrict__ order, taylor_outputs o, std::size_t first, std::size_t n, float beta2
 ) {
     constexpr int k_quads = k_taylor_block / 4;
     __shared__ std::uint32_t s_stack[StackCap * k_quads];  // entry e of quad k at [e * k_quads + k]
-    std::size_t const i = (static_cast<std::size_t>(blockIdx.x) * k_taylor_block + threadIdx.x) >> 2;
+    std::size_t const i = first + ((static_cast<std::size_t>(blockIdx.x) * k_taylor_block + threadIdx.x) >> 2);
     if (i >= n)
         return;  // whole quads
     int const j = static_cast<int>(threadIdx.x & 3);
@@ -1198,9 +1199,11 @@ void launch_taylor_cap(
             records, bvh.triangles.ptr, root, qx, qy, qz, order, o, n, beta2
         );
     } else {
-        taylor_quad_kernel<Order, Prec, Grad, Cap><<<grid_for(4 * n, k_taylor_block), k_taylor_block, 0, stream>>>(
-            records, bvh.triangles.ptr, root, qx, qy, qz, order, o, n, beta2
-        );
+        for_each_slice(n, k_quad_slice, [&](std::size_t first, std::size_t count) {
+            taylor_quad_kernel<Order, Prec, Grad, Cap><<<grid_for(4 * count, k_taylor_block), k_taylor_block, 0, stream>>>(
+                records, bvh.triangles.ptr, root, qx, qy, qz, order, o, first, first + count, beta2
+            );
+        });
     }
     GWN_LAUNCH_CHECK();
 }

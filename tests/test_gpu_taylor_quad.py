@@ -56,3 +56,25 @@ def test_quad_equals_wave_bit_for_bit(gwn, dev, order, split, grad):
                 fa, fb = a.view(np.float32), b.view(np.float32)
                 same = (a == b) | (np.isnan(fa) & np.isnan(fb) if k != 1 else False)
                 assert same.all(), (beta, n, k)
+
+
+def test_quads_beyond_one_launch(gwn, dev):
+    """2^28 + 77 unsorted queries (two launches): both ends equal the same queries in a batch of their own."""
+    import torch
+
+    mesh = synth.torus(40, 20)
+    _, bvh = build_gpu(gwn, mesh)
+    mom = gwn.MomentObject(0)
+    gwn.gwn_refit_bvh_moment(bvh, mom).raise_if_error()
+    n, k = (1 << 28) + 77, 70000
+    g = torch.Generator(device=dev)
+    g.manual_seed(1)
+    d = [torch.rand(n, generator=g, device=dev) * 3 - 1.5 for _ in range(3)]
+    out = torch.full((n,), 7.0, device=dev)
+    cfg = gwn.QueryConfig(sort_queries=0)
+    gwn.gwn_compute_winding_number_taylor_batch(bvh, mom, *d, out, accuracy_scale=2.0, config=cfg).raise_if_error()
+    for part in (slice(0, k), slice(n - k, n)):
+        e = [a[part].clone() for a in d]
+        want = torch.empty(k, device=dev)
+        gwn.gwn_compute_winding_number_taylor_batch(bvh, mom, *e, want, accuracy_scale=2.0, config=cfg).raise_if_error()
+        assert torch.equal(out[part], want)
