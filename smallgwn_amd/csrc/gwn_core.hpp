@@ -85,6 +85,17 @@ template <class T> struct device_buffer {
         count = n;
         ptr = n ? static_cast<T *>(device_alloc(n * sizeof(T), s)) : nullptr;
     }
+    // For scratch that a caller can do without: false, with no error left behind, where there is none.
+    bool try_allocate(std::size_t n, hipStream_t s) noexcept {
+        try {
+            allocate(n, s);
+            return true;
+        } catch (...) {
+            count = 0;
+            (void)hipGetLastError();
+            return false;
+        }
+    }
     void release() noexcept {
         if (ptr != nullptr)
             device_free(ptr, stream);

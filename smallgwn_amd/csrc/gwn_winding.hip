@@ -248,11 +248,13 @@ void launch_exact(
     std::size_t shares = exact_shares(nt, nq);
     if (shares > 1 && stream_capturing(stream))  // a captured batch stays one launch without an allocation
         shares = 1;
-    std::size_t const tiles_per_share = tiles == 0 ? 1 : (tiles + shares - 1) / shares;
+    std::size_t tiles_per_share = tiles == 0 ? 1 : (tiles + shares - 1) / shares;
     shares = tiles == 0 ? 1 : (tiles + tiles_per_share - 1) / tiles_per_share;  // none is empty
     device_buffer<double> part;
-    if (shares > 1)
-        part.allocate(shares * nq, stream);
+    if (shares > 1 && !part.try_allocate(shares * nq, stream)) {  // no memory for the sums: no shares
+        shares = 1;
+        tiles_per_share = tiles;
+    }
     dim3 const grid(grid_for(nq, k_exact_block), static_cast<unsigned>(shares));
     exact_kernel<Prec><<<grid, k_exact_block, 0, stream>>>(bvh.triangles.ptr, nt, qx, qy, qz, out, part.ptr, nq,
                                                            tiles_per_share);
