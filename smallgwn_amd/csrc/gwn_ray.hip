@@ -15,6 +15,7 @@
 // Arithmetic is unfused with correctly rounded division, so every record equals the CPU
 // oracle's replay bit for bit.
 #include <algorithm>
+#include <type_traits>
 
 #include "gwn_core.hpp"
 #include "gwn_quad.hpp"
@@ -53,6 +54,41 @@ __global__ __launch_bounds__(k_block) void ray_kernel(
 
 constexpr int k_ray_stride = k_block / 4 + 1;  // entry e of quad k's stack at [e * k_ray_stride + k]
 
+// The quads' stacks of a block: per entry a node and the t beyond which it is dropped.  Whole: both words of an
+// entry side by side, one 8-byte access.  Half: the nodes, then the upper 16 bits of the largest floats that
+// have no others and are not above t (t is not NaN), 6 bytes an entry.
+template <bool Half> struct ray_stack;
+template <> struct ray_stack<false> {
+    static constexpr std::size_t k_entry = sizeof(uint2);
+    uint2 *at;
+    __device__ ray_stack(std::uint32_t *lds, int, int quad) : at(reinterpret_cast<uint2 *>(lds) + quad) {}
+    __device__ void put(int e, std::uint32_t node, float t) { at[e * k_ray_stride] = make_uint2(node, __float_as_uint(t)); }
+    __device__ std::uint32_t get(int e, float &t) const {
+        uint2 const v = at[e * k_ray_stride];
+        t = __uint_as_float(v.y);
+        return v.x;
+    }
+};
+template <> struct ray_stack<true> {
+    static constexpr std::size_t k_entry = sizeof(std::uint32_t) + sizeof(std::uint16_t);
+    std::uint32_t *node;
+    std::uint16_t *bound;
+    __device__ ray_stack(std::uint32_t *lds, int entries, int quad)
+        : node(lds + quad), bound(reinterpret_cast<std::uint16_t *>(lds + entries * k_ray_stride) + quad) {}
+    __device__ void put(int e, std::uint32_t n, float t) {
+        std::uint32_t const b = __float_as_uint(t);
+        node[e * k_ray_stride] = n;
+        bound[e * k_ray_stride] = static_cast<std::uint16_t>((b + (b >> 31 != 0u ? 0xffffu : 0u)) >> 16);
+    }
+    __device__ std::uint32_t get(int e, float &t) const {
+        t = __uint_as_float(static_cast<std::uint32_t>(bound[e * k_ray_stride]) << 16);
+        return node[e * k_ray_stride];
+    }
+};
+constexpr std::size_t ray_stack_bytes(int entries, bool half) {
+    return static_cast<std::size_t>(entries) * k_ray_stride * (half ? ray_stack<true>::k_entry : ray_stack<false>::k_entry);
+}
+
 // intersect_triangle's result before it meets the best hit: whether the ray meets the triangle at t >= t_min.
 __device__ inline bool triangle_candidate(
     ray_state const &r, tri_record const &tr, float t_min, float &t, float &bu, float &bv, float (&ng)[3]
@@ -77,31 +113,29 @@ __device__ inline bool triangle_candidate(
 //     the smallest t wins, and among equal ones the first in order, whichever leaves the best excludes;
 //   packed: the leaves before the first internal child in near-first order, that child entered, the rest
 //     (leaves too) onto the stack; up to four leaves from the top of the stack are settled at a time.
-// The stack (the quad's column of an LDS array) keeps the slab entry t of each child, and an internal child
-// beyond the best hit is dropped when popped: its children's boxes lie inside its own and every operation
-// of the slab test is monotone in the bounds, so they would all have missed.  The packed test is not where
-// a direction component's reciprocal is infinite: a side of a child's box in the origin's plane gives
-// 0 * inf, and that child is met at any t.  Such rays drop nothing.  (The canonical test skips an axis
-// with such a product, so a child's entry is still no nearer than its parent's.)  A wave hands its next ray
-// to a quad that has finished (18 nodes a ray on average, 500 at most on the 1M-triangle mesh).
+// The stack (the quad's column of an LDS array) keeps the slab entry t of each child or a 16-bit lower bound of
+// it, and an internal child beyond the best hit is dropped when popped: its children's boxes lie inside its
+// own and every operation of the slab test is monotone in the bounds, so they would all have missed.  The
+// packed test is not where a direction component's reciprocal is infinite: a side of a child's box in the
+// origin's plane gives 0 * inf, and that child is met at any t.  Such rays drop nothing.  (The canonical test
+// skips an axis with such a product, so a child's entry is still no nearer than its parent's.)  A wave hands
+// its next ray to a quad that has finished (18 nodes a ray on average, 500 at most on the 1M-triangle mesh).
 //
 // One ray per lane was bound by the gathers: each of a node's eight 16-byte loads touched 64 lines a
 // wave, and its stack lived in scratch memory; a quad reads a node's 128 bytes in two.  Measured, one lane per
-// ray against this form: 4,194,304 rays on 1,048,576 triangles 5.3 / 3.5 ms (canonical), 4.9 / 3.7 ms
-// (packed), on 5,120 1.90 / 1.73 ms; 1,000 rays on 1,048,576 274 / 88 us.
-template <bool Packed, int Cap>
+// ray against this form: 4,194,304 rays on 1,048,576 triangles 5.3 / 3.1 ms (canonical), 4.3 / 3.5 ms
+// (packed), on 5,120 1.91 / 1.69 ms; 1,000 rays on 1,048,576 285 / 91 us.
+template <bool Packed, bool Half>
 __global__ __launch_bounds__(k_block) void ray_quad_kernel(
-    ray_scene sc, std::uint32_t root, float const *__restrict__ ox, float const *__restrict__ oy,
+    ray_scene sc, std::uint32_t root, int cap, float const *__restrict__ ox, float const *__restrict__ oy,
     float const *__restrict__ oz, float const *__restrict__ dx, float const *__restrict__ dy,
     float const *__restrict__ dz, ray_hit *__restrict__ out, std::size_t n, float t_min, float t_max
 ) {
-    __shared__ std::uint32_t s_node[Cap * k_ray_stride];
-    __shared__ float s_t[Cap * k_ray_stride];
+    extern __shared__ __align__(8) std::uint32_t s_stack[];
     std::uint32_t const lane = threadIdx.x & 63u;
     std::uint32_t const j = lane & 3u;
     std::uint32_t const shift = lane & 60u;
-    std::uint32_t *const st_node = s_node + (threadIdx.x >> 2);
-    float *const st_t = s_t + (threadIdx.x >> 2);
+    ray_stack<Half> stack(s_stack, cap, static_cast<int>(threadIdx.x >> 2));
     // The wave's t-th ray: 16 consecutive ones, then 16 one grid further on.
     std::size_t const wave = static_cast<std::size_t>(blockIdx.x) * (k_block / 64) + (threadIdx.x >> 6);
     std::size_t const waves = static_cast<std::size_t>(gridDim.x) * (k_block / 64);
@@ -202,16 +236,14 @@ __global__ __launch_bounds__(k_block) void ray_quad_kernel(
             // The t beyond which the child is dropped.
             float const bound = Packed && keep ? -INFINITY : tn;
             bool const stacked = hit && (Packed ? pos > first : !is_leaf && pos > first);
-            if (stacked && to < Cap) {
-                st_node[to * k_ray_stride] = is_leaf ? (k_payload_leaf | child) : child;
-                st_t[to * k_ray_stride] = bound;
-            }
+            if (stacked && to < cap)
+                stack.put(to, is_leaf ? (k_payload_leaf | child) : child, bound);
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             std::uint32_t next = quad_or(hit && pos == first ? child : 0u);
             float next_t = __uint_as_float(quad_or(hit && pos == first ? __float_as_uint(bound) : 0u));
             if (found) {
                 sp += count - 1;
-                overflow = sp > Cap;
+                overflow = sp > cap;
             }
             // Requested before the leaf triangles are evaluated.
             bvh_child ahead = slot;
@@ -224,8 +256,8 @@ __global__ __launch_bounds__(k_block) void ray_quad_kernel(
                 // The four topmost entries: leaves are settled and excluded nodes dropped up to the first
                 // node that is neither.
                 int const e = sp - 1 - static_cast<int>(j);
-                std::uint32_t const en = e >= 0 ? st_node[e * k_ray_stride] : 0u;
-                float const et = e >= 0 ? st_t[e * k_ray_stride] : 0.0f;
+                float et = 0.0f;
+                std::uint32_t const en = e >= 0 ? stack.get(e, et) : 0u;
                 bool const entry_leaf = Packed && e >= 0 && (en & k_payload_leaf) != 0u;
                 std::uint32_t const open =
                     static_cast<std::uint32_t>(__ballot(e >= 0 && !entry_leaf && !(et > best.t)) >> shift) & 15u;
@@ -269,14 +301,34 @@ __global__ __launch_bounds__(k_block) void ray_quad_kernel(
     }
 }
 
-// Blocks of the quad traversal: two waves for each of the 8,192 that fit the chip, fewer where every quad
-// has its ray at once (4M rays on 1M triangles 3.8-3.9 ms with 2,048 to 4,096 blocks, 5.4 ms with a quad per
-// ray; on 5,120 triangles 1.88 ms with 2,048, 1.73 ms with 4,096).
+// Blocks of the quad traversal: 16,384 waves where at most 6,144 fit the chip, so that the last ones even out,
+// fewer where every quad has its ray at once (4M rays on 1M triangles 3.8-3.9 ms with 2,048 to 4,096 blocks,
+// 5.4 ms with a quad per ray; on 5,120 triangles 1.88 ms with 2,048, 1.73 ms with 4,096).
 inline unsigned ray_quad_grid(std::size_t n) { return std::min(grid_for(4 * n, k_block), 4096u); }
+
+constexpr std::size_t k_lds_per_cu = std::size_t(160) << 10, k_lds_per_block = std::size_t(64) << 10;
+
+// Whether the stacks keep 16-bit bounds: where LDS with whole floats holds fewer blocks per CU than registers
+// do (6) and the grid has more than those.  The arrays are as long as the tree's own stack bound.  4,194,304
+// rays, H-PLOC trees, one lane per ray / whole floats at a compiled 64 or 128 entries / this: 1,048,576
+// triangles canonical (59 entries) 5.34 / 3.52 / 3.06 ms, packed (94) 4.29 / 5.51 / 3.47 ms; 4,194,304 packed
+// (108) 6.32 / 6.44 / 5.18 ms.  Where few blocks run, the conversions only lengthen the chain: 1,000 rays of
+// 1,048,576 triangles 93.7 us with 16 bits, 90.5 us without.
+bool ray_half_bounds(int entries, unsigned grid) {
+    std::size_t const bytes = ray_stack_bytes(entries, false);
+    return bytes > k_lds_per_block || (6 * bytes > k_lds_per_cu && grid > 256 * (k_lds_per_cu / bytes));
+}
+
+// LDS to ask for: no less than lets the blocks of a grid that fits the chip lie on it evenly (65,536 rays of
+// 2,097,152 triangles, four blocks a CU: 767 us, 850 us with room for more of them on one CU).
+std::size_t ray_lds_bytes(int entries, bool half, unsigned grid) {
+    std::size_t const per_cu = (grid + 255u) / 256u;
+    return std::max(ray_stack_bytes(entries, half), std::min(k_lds_per_block, k_lds_per_cu / (per_cu + 1) + 8));
+}
 
 template <bool Packed, int Cap>
 void launch_ray(
-    gwn_bvh_handle const &bvh, float const *ox, float const *oy, float const *oz, float const *dx,
+    gwn_bvh_handle const &bvh, int need, float const *ox, float const *oy, float const *oz, float const *dx,
     float const *dy, float const *dz, void *out, std::size_t n, float t_min, float t_max,
     std::uint32_t *counters, hipStream_t stream
 ) {
@@ -284,11 +336,16 @@ void launch_ray(
     if (counters != nullptr)
         ray_kernel<Packed, Cap, true><<<grid_for(n, k_block), k_block, 0, stream>>>(
             sc, bvh.root.reference, ox, oy, oz, dx, dy, dz, nullptr, n, t_min, t_max, counters);
-    else if (ref_internal(bvh.root.reference))
-        ray_quad_kernel<Packed, Cap><<<ray_quad_grid(n), k_block, 0, stream>>>(
-            sc, static_cast<std::uint32_t>(ref_offset(bvh.root.reference)), ox, oy, oz, dx, dy, dz,
-            static_cast<ray_hit *>(out), n, t_min, t_max);
-    else
+    else if (ref_internal(bvh.root.reference)) {
+        unsigned const grid = ray_quad_grid(n);
+        std::uint32_t const root = static_cast<std::uint32_t>(ref_offset(bvh.root.reference));
+        if (ray_half_bounds(need, grid))
+            ray_quad_kernel<Packed, true><<<grid, k_block, ray_lds_bytes(need, true, grid), stream>>>(
+                sc, root, need, ox, oy, oz, dx, dy, dz, static_cast<ray_hit *>(out), n, t_min, t_max);
+        else
+            ray_quad_kernel<Packed, false><<<grid, k_block, ray_lds_bytes(need, false, grid), stream>>>(
+                sc, root, need, ox, oy, oz, dx, dy, dz, static_cast<ray_hit *>(out), n, t_min, t_max);
+    } else
         ray_kernel<Packed, Cap><<<grid_for(n, k_block), k_block, 0, stream>>>(
             sc, bvh.root.reference, ox, oy, oz, dx, dy, dz, static_cast<ray_hit *>(out), n, t_min, t_max);
     GWN_LAUNCH_CHECK();
@@ -301,11 +358,11 @@ void launch_ray_cap(
     hipStream_t stream
 ) {
     if (need <= 32)
-        launch_ray<Packed, 32>(bvh, ox, oy, oz, dx, dy, dz, out, n, t_min, t_max, counters, stream);
+        launch_ray<Packed, 32>(bvh, need, ox, oy, oz, dx, dy, dz, out, n, t_min, t_max, counters, stream);
     else if (need <= 64)
-        launch_ray<Packed, 64>(bvh, ox, oy, oz, dx, dy, dz, out, n, t_min, t_max, counters, stream);
+        launch_ray<Packed, 64>(bvh, need, ox, oy, oz, dx, dy, dz, out, n, t_min, t_max, counters, stream);
     else if (need <= 128)
-        launch_ray<Packed, 128>(bvh, ox, oy, oz, dx, dy, dz, out, n, t_min, t_max, counters, stream);
+        launch_ray<Packed, 128>(bvh, need, ox, oy, oz, dx, dy, dz, out, n, t_min, t_max, counters, stream);
     else
         throw_invalid("Traversal stack bound exceeds the largest compiled stack (128).");
 }

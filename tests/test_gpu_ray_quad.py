@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from smallgwn_amd import synth
+from tests.helpers import nested_octants
 from tests.test_gpu_build import build_gpu
 from tests.test_gpu_ray import _oracle, _rays, _same
 
@@ -87,4 +88,23 @@ def test_directions_with_infinite_reciprocals(gwn, orc, dev, seed, canonical):
     d = np.where(r.random((n, 3)) < 0.5, r.choice([1e-40, -1e-40, 3e-39, -1e-44], (n, 3)), d)
     o, d = o.astype(np.float32), d.astype(np.float32)
     for t_min in (0.0, -5.0, -float("inf")):
+        _same(_rays(gwn, dev, bvh, o, d, t_min, stack=stack), _oracle(orc, mesh, o, d, t_min, stack=stack))
+
+
+@pytest.mark.parametrize("canonical", [False, True])
+@pytest.mark.parametrize("n", [1000, 100003])
+def test_deep_stacks(gwn, orc, dev, n, canonical):
+    """Stacks of more than 64 entries, with whole bounds (few rays) and 16-bit ones (more blocks than LDS holds with
+    whole ones)."""
+    mesh = nested_octants(16)
+    _, bvh = build_gpu(gwn, mesh)
+    info = bvh.info()
+    assert info["packed_stack_bound"] > info["internal_stack_bound"] > 64
+    stack = info["internal_stack_bound"] if canonical else 128
+    r = np.random.default_rng(n)
+    v = mesh.vertices()
+    o = r.normal(size=(n, 3))
+    o = (o / np.linalg.norm(o, axis=1, keepdims=True) * 2.0 ** -r.integers(0, 18, (n, 1))).astype(np.float32)
+    d = (v[r.integers(0, v.shape[0], n)] - o).astype(np.float32)
+    for t_min in (0.0, -1.0):
         _same(_rays(gwn, dev, bvh, o, d, t_min, stack=stack), _oracle(orc, mesh, o, d, t_min, stack=stack))
