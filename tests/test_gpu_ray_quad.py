@@ -108,3 +108,15 @@ def test_deep_stacks(gwn, orc, dev, n, canonical):
     d = (v[r.integers(0, v.shape[0], n)] - o).astype(np.float32)
     for t_min in (0.0, -1.0):
         _same(_rays(gwn, dev, bvh, o, d, t_min, stack=stack), _oracle(orc, mesh, o, d, t_min, stack=stack))
+
+
+@pytest.mark.parametrize("triangles", [12, 64, 65])
+def test_many_rays_of_a_few_triangles(gwn, orc, dev, triangles):
+    """Both sides of the rule that gives large batches over a few triangles one lane per ray."""
+    mesh = synth.open_soup(16, 8)
+    mesh = synth.Mesh(mesh.vx, mesh.vy, mesh.vz, mesh.i0[:triangles].copy(), mesh.i1[:triangles].copy(), mesh.i2[:triangles].copy())
+    _, bvh = build_gpu(gwn, mesh)
+    o, d = _set(mesh, (1 << 19) + 5, triangles)
+    for n in ((1 << 19) - 1, (1 << 19) + 5):
+        got = _rays(gwn, dev, bvh, o[:n], d[:n])
+        _same(got[-20000:], _oracle(orc, mesh, o[n - 20000:n], d[n - 20000:n]))
