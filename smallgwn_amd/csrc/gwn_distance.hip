@@ -547,14 +547,17 @@ __device__ inline void distance_quad_range(
         finish);
 }
 
-// Up to this many points every point has a row of 16 lanes from the start: their rows hardly fill the
-// chip, and the batch lasts as long as its longest point.  Measured, a row per point against a quad per
-// point: 65,536 points of 1,048,576 triangles 3.6 / 7.9 ms, 262,144 6.1 / 10.0 ms, of 131,072 2.3 / 3.6 ms;
-// 1,000,000 points of 1,048,576 15.4 / 14.3 ms, of 5,120 1.7 / 1.3 ms.
-constexpr std::size_t k_row_points = std::size_t(1) << 18;
+// Up to this many points every point has a row of 16 lanes from the start: their rows hardly fill the chip, and
+// the batch lasts as long as its longest point.  Beyond, quads that hand out points (and rows for the last
+// ones) do less in all.  Measured, a row per point / quads: 16,384 points of 500 triangles 83 / 98 us, of
+// 1,048,576 2.8 / 3.4 ms; 65,536 of 12 90 / 87 us, of 5,120 301 / 332 us, of 131,072 1.21 / 1.50 ms, of 1,048,576
+// 3.6 / 4.0 ms; 131,072 of 500 240 / 194 us, of 5,120 457 / 388 us, of 131,072 2.02 / 2.01 ms, of 1,048,576 6.2 /
+// 6.2 ms; 262,144 of 12 165 / 120 us, of 131,072 2.41 / 2.20 ms, of 1,048,576 7.3 / 7.5 ms; 1,000,003 of 1,048,576
+// 18.1 / 13.9 ms.
+constexpr std::size_t k_row_points = std::size_t(1) << 16;
 
-// Blocks of the quad traversal.  A quad per point: two waves for each of the 8,192 that fit the chip
-// (half or twice as many measured 5-25 % slower from 1M points on).
+// Blocks of the quad traversal.  Quads: 16,384 waves where 2,048 to 6,144 fit the chip, as the stacks' LDS lets
+// them (half or twice as many measured 5-25 % slower from 1M points on).
 inline unsigned distance_quad_grid(std::size_t n) {
     return n <= k_row_points ? grid_for(16 * n, k_block) : std::min(grid_for(4 * n, k_block), 4096u);
 }

@@ -10,7 +10,7 @@ from tests.test_gpu_build import build_gpu
 
 pytestmark = pytest.mark.gpu
 
-ROW_POINTS = 1 << 18
+ROW_POINTS = 1 << 16
 
 
 def _meshes():
@@ -47,7 +47,7 @@ def _points(mesh, n, seed):
 
 
 @pytest.mark.parametrize("name,mesh", list(_meshes()), ids=[m[0] for m in _meshes()])
-@pytest.mark.parametrize("n", [1, 3, 4, 5, 17, 1023, 20000, ROW_POINTS, ROW_POINTS + 1, 700001])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 17, 1023, 20000, ROW_POINTS, ROW_POINTS + 1, 1 << 18, (1 << 18) + 1, 700001])
 def test_rows_and_quads_equal_the_lane_kernel(gwn, dev, name, mesh, n):
     _, bvh = build_gpu(gwn, mesh)
     q = _points(mesh, n, seed=n)
