@@ -822,11 +822,11 @@ template <int Order, int Prec, bool Grad, int StackCap>
 __global__ __launch_bounds__(k_taylor_block) void taylor_quad_kernel(
     float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node,
     float const *__restrict__ qx, float const *__restrict__ qy, float const *__restrict__ qz,
-    std::uint32_t const *__restrict__ order, taylor_outputs o, std::size_t first, std::size_t n, float beta2
+    std::uint32_t const *__restrict__ order, taylor_outputs o, std::size_t n, float beta2
 ) {
     constexpr int k_quads = k_taylor_block / 4;
     __shared__ std::uint32_t s_stack[StackCap * k_quads];  // entry e of quad k at [e * k_quads + k]
-    std::size_t const i = first + ((static_cast<std::size_t>(blockIdx.x) * k_taylor_block + threadIdx.x) >> 2);
+    std::size_t const i = (static_cast<std::size_t>(blockIdx.x) * k_taylor_block + threadIdx.x) >> 2;
     if (i >= n)
         return;  // whole quads
     int const j = static_cast<int>(threadIdx.x & 3);
@@ -1174,6 +1174,14 @@ bool dense_queries(std::size_t triangles, std::size_t n, float beta2) {
     return double(n) >= 4500.0 * std::sqrt(double(triangles)) * std::pow(2.0 / beta, 1.5);
 }
 
+// The outputs of the queries from `at` on.
+inline taylor_outputs outputs_from(taylor_outputs o, std::size_t at) {
+    for (float **p : {&o.out, &o.gx, &o.gy, &o.gz})
+        *p = *p != nullptr ? *p + at : nullptr;
+    o.counters = o.counters != nullptr ? o.counters + 3 * at : nullptr;
+    return o;
+}
+
 template <int Order, int Prec, bool Grad, int Cap>
 void launch_taylor_cap(
     gwn_bvh_handle const &bvh, gwn_moment_handle const &m, float const *qx, float const *qy,
@@ -1202,8 +1210,11 @@ void launch_taylor_cap(
         );
     } else {
         for_each_slice(n, k_quad_slice, [&](std::size_t first, std::size_t count) {
+            // With an order its entries say where a query lies, without one it lies at its own place.
+            std::size_t const at = order != nullptr ? 0 : first;
             taylor_quad_kernel<Order, Prec, Grad, Cap><<<grid_for(4 * count, k_taylor_block), k_taylor_block, 0, stream>>>(
-                records, bvh.triangles.ptr, root, qx, qy, qz, order, o, first, first + count, beta2
+                records, bvh.triangles.ptr, root, qx + at, qy + at, qz + at, order != nullptr ? order + first : nullptr,
+                outputs_from(o, at), count, beta2
             );
         });
     }
