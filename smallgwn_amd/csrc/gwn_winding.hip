@@ -931,9 +931,12 @@ __global__ __launch_bounds__(k_taylor_block) void taylor_row_kernel(
 }
 
 // Up to this many queries each has a row: the chip is not full, and the batch lasts as long as its longest
-// query.  Measured, a row against a quad per query (scale 2): 1,000 of 5,120 triangles 90 / 177 us, 8,000
-// of 131,072 280 / 590 us, 65,536 of 131,072 430 / 600 us, 4,096 of 1,048,576 600 / 1,180 us; but 200,000
-// of 5,120 468 / 415 us, of 131,072 754 / 720 us, and 262,144 of 131,072 at scale 6.25 5.4 / 4.1 ms.
+// query.  Measured, a row against a quad per query, sort included, order 2, scale 2: 1,000 of 5,120 triangles
+// 109 / 171 us, 20,000 of 500 99 / 114, 65,536 of 500 149 / 130, of 5,120 200 / 198, of 131,072 337 / 506, of
+// 1,048,576 0.67 / 1.23 ms; 131,072 of 5,120 287 / 252 us, of 131,072 453 / 552, of 1,048,576 0.77 / 1.30 ms; 262,144
+// of 5,120 467 / 355 us, of 131,072 703 / 672, of 1,048,576 0.97 / 1.46 ms; split, scale 6.25: 65,536 of 5,120 0.95 /
+// 0.78 ms, of 131,072 1.81 / 1.90, 262,144 of 131,072 4.6 / 3.8, of 1,048,576 6.5 / 6.9.  So the crossing rises with
+// the triangles, from some 40,000 queries at 500 to more than 262,144 at 1,048,576; one line in the middle.
 constexpr std::size_t k_row_queries = std::size_t(1) << 16;
 
 // Reciprocal square root and reciprocal in FP64 from the hardware approximations and Newton
@@ -1164,14 +1167,27 @@ __global__ __launch_bounds__(k_taylor_block) void taylor_adjoint_kernel(
 // union of paths grows with the square root of the triangles near it and with beta; the quad
 // traversal's time is proportional to the queries.  Measured (MI355X, mixed queries, sort included),
 // wave against quad, order 2:
-//   beta 2:    5,120 triangles, 262k queries 463 / 463 us, 1M 696 / 963 us; 131,072, 1M 1.88 / 1.44 ms,
-//              4M 2.75 / 4.31 ms; 1,048,576, 1M 5.23 / 2.30 ms, 4M 5.86 / 4.88 ms
-//   beta 6.25 (split): 5,120, 66k 1.47 / 0.95 ms, 262k 1.57 / 2.12 ms; 131,072, 262k 4.78 / 4.09 ms,
-//              1M 6.62 / 9.97 ms; 1,048,576, 262k 13.1 / 6.6 ms, 1M 13.4 / 14.1 ms
-// The crossings lie near 4500 sqrt(triangles) (2 / beta)^1.5.
+//   beta 2:    500 triangles, 131k queries 181 / 167 us, 262k 205 / 240; 5,120, 262k 391 / 355, 1M 559 / 881;
+//              131,072, 1M 1.54 / 1.37 ms, 4M 2.41 / 4.15; 1,048,576, 1M 3.99 / 2.12, 4M 4.86 / 4.75
+//   beta 6.25 (split): 2,000, 131k 884 / 959 us; 5,120, 131k 1.21 / 1.21 ms, 262k 1.47 / 1.93; 131,072, 262k
+//              4.23 / 3.82 ms, 1M 6.39 / 9.66; 1,048,576, 262k 12.0 / 6.9, 1M 12.8 / 14.1
+// The crossings lie near 4500 sqrt(triangles) (2 / beta)^1.5, for few triangles above it.
 bool dense_queries(std::size_t triangles, std::size_t n, float beta2) {
     double const beta = std::sqrt(std::max(1.0, double(beta2)));
     return double(n) >= 4500.0 * std::sqrt(double(triangles)) * std::pow(2.0 / beta, 1.5);
+}
+
+// Whether a single batch takes whole waves.  Dense queries, but below 100,000 of them only where the tree is tiny:
+// elsewhere a row or a quad per query is the faster form there (wave against row, beta 6.25: 65,536 queries of 350
+// triangles 304 / 447 us, of 2,000 878 / 781, of 5,120 1,300 / 949).  And, in any order of the queries, trees so tiny
+// for their beta that a query descends most of them anyway (unsorted, wave against row or quad: beta 2, 65,536 of
+// 12 triangles 21 / 32 us, of 50 52 / 53, 1,000,003 of 50 197 / 402, of 200 779 / 671; beta 6.25, 65,536 of 200
+// 177 / 277, of 500 454 / 391, 1,000,003 of 500 2.64 / 4.74 ms, of 2,000 9.6 / 8.0; 20,000 of 50 36 / 31 us).
+bool whole_waves(std::size_t triangles, std::size_t n, float beta2, bool sorted) {
+    double const scale = std::max(1.0, double(beta2));
+    bool const tiny = double(triangles) <= 25.0 * scale;
+    return (tiny && double(n) >= 32768.0 + 4000.0 * double(triangles) / scale) ||
+           (sorted && (tiny || n >= 100000) && dense_queries(triangles, n, beta2));
 }
 
 // The outputs of the queries from `at` on.
@@ -1191,8 +1207,8 @@ void launch_taylor_cap(
     std::uint32_t const root = static_cast<std::uint32_t>(ref_offset(bvh.root.reference));
     // The value alone reads the evaluation records; the gradient the traversal records.
     float4 const *records = Grad ? m.records.ptr : m.eval_records.ptr;
-    if (order != nullptr && dense_queries(bvh.triangle_count, n, beta2)) {
-        // Hilbert-ordered dense queries: neighbouring lanes share most of their paths.  VALU bound:
+    if (whole_waves(bvh.triangle_count, n, beta2, order != nullptr)) {
+        // Neighbouring lanes share most of their paths.  VALU bound:
         // 16,777,216 queries of 1,048,576 triangles (order 2, split, scale 6.25) took 69.0 ms with 189,111
         // instructions a wave, 59.5 ms with the 166,216 of unmasked tests and terms, tallies on demand only
         // and half_angle_far.

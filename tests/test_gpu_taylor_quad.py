@@ -78,3 +78,27 @@ def test_quads_beyond_one_launch(gwn, dev):
         want = torch.empty(k, device=dev)
         gwn.gwn_compute_winding_number_taylor_batch(bvh, mom, *e, want, accuracy_scale=2.0, config=cfg).raise_if_error()
         assert torch.equal(out[part], want)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("triangles,beta", [(8, 2.0), (16, 2.0), (101, 2.0), (300, 6.25)])
+def test_whole_waves_of_tiny_trees_in_any_order(gwn, dev, triangles, beta, grad):
+    """Unsorted batches on both sides of the rule that walks a tree with whole waves where every query descends most
+    of it: the same bits as rows (a smaller batch of the same queries), work counters too."""
+    full = synth.torus(20, 10)
+    mesh = synth.Mesh(full.vx, full.vy, full.vz, full.i0[:triangles].copy(), full.i1[:triangles].copy(), full.i2[:triangles].copy())
+    _, bvh = build_gpu(gwn, mesh)
+    for order, precision in ((1, gwn.Precision.PLAIN), (2, gwn.Precision.SPLIT)):
+        mom = gwn.MomentObject(order)
+        gwn.gwn_refit_bvh_moment(bvh, mom).raise_if_error()
+        q = synth.mixed_queries(mesh, 70000, seed=triangles)
+        q[0][5], q[1][6] = np.nan, np.inf
+        small = [_run(gwn, dev, bvh, mom, _first([a[at:] for a in q], 7000, dev), 0, precision, beta, grad)
+                 for at in range(0, 70000, 7000)]
+        want = [np.concatenate(parts) for parts in zip(*small)]
+        for n in (32767, 40768, 48767, 48768, 48769, 63487, 63488, 63489, 70000):
+            got = _run(gwn, dev, bvh, mom, _first(q, n, dev), 0, precision, beta, grad)
+            for k, (a, b) in enumerate(zip(got, want)):
+                b = b[:a.shape[0]]
+                fa, fb = a.view(np.float32), b.view(np.float32)
+                assert ((a == b) | (np.isnan(fa) & np.isnan(fb) if k != 1 else False)).all(), (n, k)
