@@ -153,7 +153,11 @@ __global__ __launch_bounds__(k_exact_block) void exact_plain_kernel(
 // Measured, split, one share with per-pair edges and arctangents against this form: 100,000 triangles
 // x 32,749 queries 38.1 against 4.7 ms, 131,044 x 1,000 52.3 against 0.48 ms, 25,600 x 600,000 (one
 // share in both) 56.9 against 37.0 ms.
-template <int Prec>
+//
+// OneTile: at most 256 triangles, most of them near most queries.  Waves without a far pair skip its arithmetic,
+// and near triangles come from LDS (elsewhere the test costs 2 % and the larger tile 3-5 %): 4,000,000 queries of 24
+// triangles 365 us without, 293 with, 1,000 of 24 15.8 and 11.9 us.
+template <int Prec, bool OneTile>
 __global__ __launch_bounds__(k_exact_block) void exact_kernel(
     tri_record const *__restrict__ tris, std::size_t nt, float const *__restrict__ qx,
     float const *__restrict__ qy, float const *__restrict__ qz, double *__restrict__ out, double *__restrict__ part,
@@ -162,6 +166,7 @@ __global__ __launch_bounds__(k_exact_block) void exact_kernel(
     static_assert(Prec == GWN_PRECISION_SPLIT || Prec == GWN_PRECISION_FP64, "FP64 sums");
     constexpr bool k_raw = Prec == GWN_PRECISION_FP64;
     __shared__ std::conditional_t<k_raw, tri_record, exact_item> tile[k_exact_block];
+    __shared__ tri_record raw[OneTile && !k_raw ? k_exact_block : 1];
     std::size_t const qi = static_cast<std::size_t>(blockIdx.x) * k_exact_block + threadIdx.x;
     bool const active = qi < nq;
     float const x = active ? qx[qi] : 0.0f;
@@ -179,6 +184,8 @@ __global__ __launch_bounds__(k_exact_block) void exact_kernel(
                 tile[threadIdx.x] = tris[base + threadIdx.x];
             else
                 stage_exact_item<Prec>(tris[base + threadIdx.x], tile[threadIdx.x]);
+            if constexpr (OneTile && !k_raw)
+                raw[threadIdx.x] = tris[base + threadIdx.x];
         }
         __syncthreads();
         if constexpr (k_raw) {
@@ -192,10 +199,12 @@ __global__ __launch_bounds__(k_exact_block) void exact_kernel(
                 float const ax = t.f[0] - x, ay = t.f[1] - y, az = t.f[2] - z;
                 float const aa = ax * ax + ay * ay + az * az;
                 bool const near = !(aa > t.f[15]);
-                float const h = half_angle_far_staged(t, ax, ay, az, aa, !near);
-                far += near ? 0.0f : h;
+                if (!OneTile || __ballot(!near) != 0ull) {
+                    float const h = half_angle_far_staged(t, ax, ay, az, aa, !near);
+                    far += near ? 0.0f : h;
+                }
                 if (near)
-                    sum += solid_angle_split_near(tris[base + k], x, y, z);
+                    sum += solid_angle_split_near(OneTile ? raw[k] : tris[base + k], x, y, z);
             }
             sum += 2.0 * double(far);
         }
@@ -256,8 +265,9 @@ void launch_exact(
         tiles_per_share = tiles;
     }
     dim3 const grid(grid_for(nq, k_exact_block), static_cast<unsigned>(shares));
-    exact_kernel<Prec><<<grid, k_exact_block, 0, stream>>>(bvh.triangles.ptr, nt, qx, qy, qz, out, part.ptr, nq,
-                                                           tiles_per_share);
+    auto const kernel = tiles <= 1 && Prec == GWN_PRECISION_SPLIT ? exact_kernel<Prec, Prec == GWN_PRECISION_SPLIT>
+                                                                  : exact_kernel<Prec, false>;
+    kernel<<<grid, k_exact_block, 0, stream>>>(bvh.triangles.ptr, nt, qx, qy, qz, out, part.ptr, nq, tiles_per_share);
     GWN_LAUNCH_CHECK();
     if (shares > 1) {
         exact_combine_kernel<<<grid_for(nq, 256), 256, 0, stream>>>(part.ptr, shares, out, nq);
