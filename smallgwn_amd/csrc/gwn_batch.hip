@@ -193,9 +193,14 @@ void enqueue_query(gwn_batch_handle &b, hipStream_t stream) {
     if (b.total_chunks == 0)
         return;
     fill_u32(reinterpret_cast<std::uint32_t *>(b.counter.ptr), 0u, 2, stream);
-    int const grid = std::max(1, b.blocks_per_cu * b.cu_count);
+    bool waves = false, quads = false;
+    for (batch_mesh const &m : b.host_meshes)
+        (m.wave != 0u ? waves : quads) = true;
+    // Trees that the batch does not rebuild keep to their own bound, whatever stack was asked for.
+    int const entries = b.trees ? b.cap : std::clamp(static_cast<int>(b.stack_bound), 1, b.cap);
     taylor_batch_launch(b.meshes.ptr, static_cast<std::uint32_t>(b.host_meshes.size()), b.total_chunks,
-                        b.accuracy_scale, b.counter.ptr, b.order, b.cap, b.block, grid, b.traversal != 0, stream);
+                        b.accuracy_scale, b.counter.ptr, b.order, entries, b.block, b.blocks_per_cu, b.cu_count, waves, quads,
+                        stream);
 }
 
 // The refit table: every mesh with an internal root, and for every depth the meshes' node ranges

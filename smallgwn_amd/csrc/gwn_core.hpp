@@ -351,12 +351,13 @@ struct batch_mesh {
     std::uint32_t wave;          // 1 wave-cooperative, 0 four lanes per query
     std::uint32_t chunk;         // queries a block takes at a time
 };
-// Persistent batched Taylor winding (plain precision): `grid` blocks of `block` threads take
+// Persistent batched Taylor winding (plain precision): blocks_per_cu x cu_count blocks of `block` threads take
 // chunks of their mesh's `chunk` queries from *counter (which must be zero) until total_chunks are done.
-// `waves`: whether any mesh has its wave flag set.
+// `waves`, `quads`: whether any mesh has its wave flag set, or not set.  Stacks hold `cap` entries.
 void taylor_batch_launch(
     batch_mesh const *meshes, std::uint32_t mesh_count, std::uint64_t total_chunks, float accuracy_scale,
-    std::uint64_t *counter, int order, int cap, int block, int grid, bool waves, hipStream_t stream
+    std::uint64_t *counter, int order, int cap, int block, int blocks_per_cu, int cu_count, bool waves, bool quads,
+    hipStream_t stream
 );
 // Whether a batch walks a mesh of `triangles` with whole waves (its queries are dense enough).
 bool batch_dense_queries(std::size_t triangles, std::size_t queries, float accuracy_scale);

@@ -374,19 +374,19 @@ __device__ inline std::uint64_t uniform_u64(std::uint64_t v) {
 }
 
 // Wave-cooperative traversal (defined below; the batched kernel uses it too).
-template <int Order, int Prec, bool Grad, int StackCap, bool Count>
+template <int Order, int Prec, bool Grad, bool Count>
 __device__ inline bool taylor_wave_traverse(
     float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node, bool active,
     float x, float y, float z, float beta2, taylor_sums<Prec, Grad> &acc, std::uint32_t &n_tests,
-    std::uint32_t &n_accept, std::uint32_t &n_leaf, std::uint32_t *s_node, std::uint64_t *s_mask
+    std::uint32_t &n_accept, std::uint32_t &n_leaf, std::uint32_t *s_node, std::uint64_t *s_mask, int cap
 );
 
 // Four lanes per query (defined below; the batched kernel uses it too).
-template <int Order, int Prec, bool Grad, int StackCap>
+template <int Order, int Prec, bool Grad>
 __device__ inline bool taylor_quad_traverse(
     float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node, float x, float y,
     float z, float beta2, taylor_sums<Prec, Grad> &acc, std::uint32_t &n_tests, std::uint32_t &n_accept,
-    std::uint32_t &n_leaf, std::uint32_t *stack, int stride
+    std::uint32_t &n_leaf, std::uint32_t *stack, int stride, int cap
 );
 
 // Batched persistent traversal: many meshes, one launch.  Work is a list of chunks of consecutive
@@ -395,20 +395,24 @@ __device__ inline bool taylor_quad_traverse(
 // traversals of the single-mesh batch, so each result equals that batch's.  A mesh whose `wave` flag
 // is set is walked by whole waves, any other with four lanes per query (a wave walks the union of its
 // lanes' paths, which pays where a mesh's queries are dense and costs where a few queries are spread
-// over a large tree: one such wave alone can last as long as the rest of the launch).  Waves: whether
-// any mesh may have its flag set.  Rebuild and query of 128 meshes of up to 100,000 triangles, recorded:
+// over a large tree: one such wave alone can last as long as the rest of the launch).  Waves, Quads:
+// whether any mesh may be walked either way.  A block walks one way at a time, so both kinds of stacks share
+// its LDS, batch_lds_bytes of it for `cap` entries (both at a compiled 128 entries and a block of 256 held four
+// blocks a CU: 20M queries of 200 meshes of 1,000 triangles 5.92 ms, 4.92 now; in blocks of 64 15.3, 4.6).  Rebuild and query of 128 meshes of up to 100,000 triangles, recorded:
 // 8.04 ms with whole waves for every mesh, 4.16 now (2.36M queries in all); of 8 meshes with 174,131:
 // 4.69, 1.28; of 512 with 9.0M: 14.2, 11.5.
-template <int Order, int StackCap, bool Waves>
+template <int Order, bool Waves, bool Quads>
 __global__ __launch_bounds__(256) void taylor_batch_kernel(
-    batch_mesh const *__restrict__ meshes, std::uint32_t mesh_count, std::uint64_t total_chunks, float beta2,
+    batch_mesh const *__restrict__ meshes, std::uint32_t mesh_count, std::uint64_t total_chunks, float beta2, int cap,
     std::uint64_t *counter
 ) {
     __shared__ std::uint64_t s_chunk;
-    __shared__ std::uint32_t s_node[4][Waves ? StackCap : 1];
-    __shared__ std::uint64_t s_mask[4][Waves ? StackCap : 1];
-    __shared__ std::uint32_t s_quad[StackCap * 64];  // entry e of quad k's stack at [e * 64 + k]
+    extern __shared__ std::uint64_t s_stacks[];
     int const wave = threadIdx.x >> 6;
+    int const quads = static_cast<int>(blockDim.x >> 2);
+    std::uint64_t *const s_mask = s_stacks + wave * cap;
+    std::uint32_t *const s_node = reinterpret_cast<std::uint32_t *>(s_stacks + static_cast<int>(blockDim.x >> 6) * cap) + wave * cap;
+    std::uint32_t *const s_quad = reinterpret_cast<std::uint32_t *>(s_stacks) + (threadIdx.x >> 2);  // entry e at [e * quads]
     for (;;) {
         if (threadIdx.x == 0)
             s_chunk = atomicAdd(reinterpret_cast<unsigned long long *>(counter), 1ull);
@@ -429,7 +433,7 @@ __global__ __launch_bounds__(256) void taylor_batch_kernel(
         batch_mesh const m = meshes[lo];
         std::uint32_t const chunk = m.chunk;
         std::uint64_t const base = (c - m.first_chunk) * chunk;
-        if (!ref_leaf(m.root) && !(Waves && m.wave != 0u)) {  // uniform over the block
+        if (Quads && !ref_leaf(m.root) && !(Waves && m.wave != 0u)) {  // uniform over the block
             for (std::uint32_t t = threadIdx.x >> 2; t < chunk; t += blockDim.x >> 2) {  // whole quads
                 std::uint64_t const p = base + t;
                 if (p >= m.count)
@@ -437,9 +441,9 @@ __global__ __launch_bounds__(256) void taylor_batch_kernel(
                 std::uint64_t const q = m.order ? m.order[p] : p;
                 taylor_sums<GWN_PRECISION_PLAIN, false> acc;
                 std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;
-                bool const overflow = taylor_quad_traverse<Order, GWN_PRECISION_PLAIN, false, StackCap>(
+                bool const overflow = taylor_quad_traverse<Order, GWN_PRECISION_PLAIN, false>(
                     m.records, m.tris, static_cast<std::uint32_t>(ref_offset(m.root)), m.qx[q], m.qy[q], m.qz[q], beta2,
-                    acc, n_tests, n_accept, n_leaf, s_quad + (threadIdx.x >> 2), 64);
+                    acc, n_tests, n_accept, n_leaf, s_quad, quads, cap);
                 if ((threadIdx.x & 3u) == 0u)
                     acc.store(overflow, q, m.out, nullptr, nullptr, nullptr);
             }
@@ -464,9 +468,9 @@ __global__ __launch_bounds__(256) void taylor_batch_kernel(
                 if (__ballot(active) == 0ull)
                     continue;
                 std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;
-                overflow = taylor_wave_traverse<Order, GWN_PRECISION_PLAIN, false, StackCap, false>(
+                overflow = taylor_wave_traverse<Order, GWN_PRECISION_PLAIN, false, false>(
                     m.records, m.tris, static_cast<std::uint32_t>(ref_offset(m.root)), active, x, y, z, beta2, acc,
-                    n_tests, n_accept, n_leaf, s_node[wave], s_mask[wave]);
+                    n_tests, n_accept, n_leaf, s_node, s_mask, cap);
                 if (!active)
                     continue;
             }
@@ -486,11 +490,11 @@ __global__ __launch_bounds__(256) void taylor_batch_kernel(
 // this wave's LDS stack.  The wave must hold at least one active lane.  Returns true on overflow.
 // `records` are evaluation records for the value alone and traversal records with the gradient,
 // as for the per-lane traversal.  The work tallies are kept where Count (three adds a slot otherwise).
-template <int Order, int Prec, bool Grad, int StackCap, bool Count>
+template <int Order, int Prec, bool Grad, bool Count>
 __device__ inline bool taylor_wave_traverse(
     float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node, bool active,
     float x, float y, float z, float beta2, taylor_sums<Prec, Grad> &acc, std::uint32_t &n_tests,
-    std::uint32_t &n_accept, std::uint32_t &n_leaf, std::uint32_t *s_node, std::uint64_t *s_mask
+    std::uint32_t &n_accept, std::uint32_t &n_leaf, std::uint32_t *s_node, std::uint64_t *s_mask, int cap
 ) {
     constexpr int RV = Grad ? moment_record_vec4(Order) : eval_record_vec4(Order);
     constexpr int B = eval_slot_floats(Order);
@@ -572,7 +576,7 @@ __device__ inline bool taylor_wave_traverse(
                 continue;
             }
             if (next != k_invalid) {
-                if (sp < StackCap) {
+                if (sp < cap) {
                     s_node[sp] = next;
                     s_mask[sp] = next_mask;
                     ++sp;
@@ -614,8 +618,9 @@ __global__ __launch_bounds__(k_taylor_block) void taylor_wave_kernel(
         return;
     taylor_sums<Prec, Grad> acc;
     std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;
-    bool const overflow = taylor_wave_traverse<Order, Prec, Grad, StackCap, Count>(
-        records, tris, root_node, active, x, y, z, beta2, acc, n_tests, n_accept, n_leaf, s_node[wave], s_mask[wave]);
+    bool const overflow = taylor_wave_traverse<Order, Prec, Grad, Count>(
+        records, tris, root_node, active, x, y, z, beta2, acc, n_tests, n_accept, n_leaf, s_node[wave], s_mask[wave],
+        StackCap);
     if (!active)
         return;
     acc.store(overflow, q, o.out, o.gx, o.gy, o.gz);
@@ -776,11 +781,11 @@ template <int Order, bool Grad> struct slot_test {
 // Tried and slower: holding a quad's leaf triangles back until half of the wave's quads have some, so that
 // they are evaluated with more lanes active (5-20 %); handing a finished quad another query of the wave
 // (0-40 %: a wave's queries are then no longer neighbours, and their reads no longer shared).
-template <int Order, int Prec, bool Grad, int StackCap>
+template <int Order, int Prec, bool Grad>
 __device__ inline bool taylor_quad_traverse(
     float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node, float x, float y,
     float z, float beta2, taylor_sums<Prec, Grad> &acc, std::uint32_t &n_tests, std::uint32_t &n_accept,
-    std::uint32_t &n_leaf, std::uint32_t *stack, int stride
+    std::uint32_t &n_leaf, std::uint32_t *stack, int stride, int cap
 ) {
     using slot_type = quad_slot<Order, Grad>;
     int const j = static_cast<int>(threadIdx.x & 3);
@@ -805,12 +810,12 @@ __device__ inline bool taylor_quad_traverse(
         int const pushed = __popc(bits) - 1;
         std::uint32_t next = bits & 8u ? c3 : (bits & 4u ? c2 : (bits & 2u ? c1 : c0));
         int const at = sp + __popc(bits & ((1u << j) - 1u));
-        if (v.inner && (bits >> j) != 1u && at < StackCap)
+        if (v.inner && (bits >> j) != 1u && at < cap)
             stack[at * stride] = c;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         if (pushed >= 0) {
             sp += pushed;
-            overflow = sp > StackCap;
+            overflow = sp > cap;
             live = !overflow;
         } else if (sp > 0) {
             next = stack[--sp * stride];
@@ -843,9 +848,9 @@ __global__ __launch_bounds__(k_taylor_block) void taylor_quad_kernel(
     std::size_t const q = order ? order[i] : i;
     taylor_sums<Prec, Grad> acc;
     std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;  // this lane's
-    bool const overflow = taylor_quad_traverse<Order, Prec, Grad, StackCap>(
+    bool const overflow = taylor_quad_traverse<Order, Prec, Grad>(
         records, tris, root_node, qx[q], qy[q], qz[q], beta2, acc, n_tests, n_accept, n_leaf,
-        s_stack + (threadIdx.x >> 2), k_quads);
+        s_stack + (threadIdx.x >> 2), k_quads, StackCap);
     if (j == 0)
         acc.store(overflow, q, o.out, o.gx, o.gy, o.gz);
     if (o.counters != nullptr) {
@@ -1502,21 +1507,10 @@ void launch_taylor_adjoint(
     GWN_LAUNCH_CHECK();
 }
 
-template <int Order, bool Waves>
-void launch_batch_cap(batch_mesh const *meshes, std::uint32_t mesh_count, std::uint64_t total_chunks, float beta2,
-                      std::uint64_t *counter, int cap, int block, int grid, hipStream_t stream) {
-#define GWN_BATCH(C) \
-    taylor_batch_kernel<Order, C, Waves><<<grid, block, 0, stream>>>(meshes, mesh_count, total_chunks, beta2, counter)
-    if (cap <= 32)
-        GWN_BATCH(32);
-    else if (cap <= 64)
-        GWN_BATCH(64);
-    else if (cap <= 128)
-        GWN_BATCH(128);
-    else
-        throw_invalid("Traversal stack bound exceeds the largest compiled stack (128).");
-#undef GWN_BATCH
-    GWN_LAUNCH_CHECK();
+// LDS of the stacks: 12 bytes an entry and wave, 4 bytes an entry and quad.
+std::size_t batch_lds_bytes(int cap, int block, bool waves, bool quads) {
+    std::size_t const entries = static_cast<std::size_t>(cap) * static_cast<std::size_t>(block);
+    return std::max(waves ? entries / 64 * 12 : 0, quads ? entries : 0);
 }
 
 } // namespace
@@ -1534,20 +1528,25 @@ bool batch_dense_queries(std::size_t triangles, std::size_t queries, float accur
 
 void taylor_batch_launch(
     batch_mesh const *meshes, std::uint32_t mesh_count, std::uint64_t total_chunks, float accuracy_scale,
-    std::uint64_t *counter, int order, int cap, int block, int grid, bool waves, hipStream_t stream
+    std::uint64_t *counter, int order, int cap, int block, int blocks_per_cu, int cu_count, bool waves, bool quads,
+    hipStream_t stream
 ) {
     float const beta2 = accuracy_scale * accuracy_scale;
     if (block <= 0 || block > 256 || (block & 63) != 0)
         throw_invalid("Batched query block size must be 64, 128, 192 or 256.");
-#define GWN_BATCH_ORDER(O)                                                                                     \
-    (waves ? launch_batch_cap<O, true>(meshes, mesh_count, total_chunks, beta2, counter, cap, block, grid, stream) \
-           : launch_batch_cap<O, false>(meshes, mesh_count, total_chunks, beta2, counter, cap, block, grid, stream))
+    int const grid = std::max(1, blocks_per_cu * cu_count);
+    std::size_t const lds = batch_lds_bytes(cap, block, waves, quads);
+#define GWN_BATCH(O, W, Q) \
+    taylor_batch_kernel<O, W, Q><<<grid, block, lds, stream>>>(meshes, mesh_count, total_chunks, beta2, cap, counter)
+#define GWN_BATCH_ORDER(O) \
+    (waves && quads ? GWN_BATCH(O, true, true) : waves ? GWN_BATCH(O, true, false) : GWN_BATCH(O, false, true))
     switch (order) {
     case 0: GWN_BATCH_ORDER(0); break;
     case 1: GWN_BATCH_ORDER(1); break;
     default: GWN_BATCH_ORDER(2); break;
     }
 #undef GWN_BATCH_ORDER
+#undef GWN_BATCH
 }
 
 void taylor_adjoint_traverse(
