@@ -99,13 +99,20 @@ void batch_drop_graph(gwn_batch_handle &b);
 
 namespace {
 
+// Queries per work item with four lanes each: no more than a block of 256 holds at once, for queries of a large
+// tree take long and a chunk of more of them can be the launch's last (128 meshes: 4.12 ms, with half a whole-wave
+// chunk of 1,024 4.39; 8 meshes: 1.28, 1.51).  A smaller block takes no more than it holds where there is little
+// for each block to do (512 meshes with 100 queries each, blocks of 64: 176 us, 250 with 64 queries), else 64 too,
+// or the chunk counter and the search for the chunk's mesh take its time (512 meshes with 20,000: 7.82 / 3.90 ms).
+std::uint32_t quad_chunk(gwn_batch_handle const &b) {
+    std::uint64_t const blocks = static_cast<std::uint64_t>(b.blocks_per_cu) * static_cast<std::uint64_t>(b.cu_count);
+    return static_cast<std::uint32_t>(b.total_queries >= 256 * blocks ? 64 : b.block / 4);
+}
+
 void layout_chunks(gwn_batch_handle &b) {
     std::uint64_t first = 0;
     for (auto &m : b.host_meshes) {
-        // Four lanes per query: as many as a block holds at once, for queries of a large tree take long
-        // and a chunk of more of them can be the launch's last (128 meshes: 4.12 ms, with half a
-        // whole-wave chunk of 1,024 4.39; 8 meshes: 1.28, 1.51).
-        m.chunk = static_cast<std::uint32_t>(m.wave != 0u ? b.chunk : b.block / 4);
+        m.chunk = m.wave != 0u ? static_cast<std::uint32_t>(b.chunk) : quad_chunk(b);
         m.first_chunk = first;
         first += (m.count + m.chunk - 1) / m.chunk;
     }
@@ -130,7 +137,7 @@ void set_wave_flags(gwn_batch_handle &b) {
     for (std::size_t i = 0; i < b.host_meshes.size(); ++i) {
         batch_mesh &m = b.host_meshes[i];
         bool const dense =
-            b.traversal == 1 ? batch_dense_queries(b.mesh_triangles[i], m.count, b.accuracy_scale)
+            b.traversal == 1 ? batch_dense_queries(b.mesh_triangles[i], m.count, b.total_queries, b.accuracy_scale)
                              : static_cast<double>(m.count) >= static_cast<double>(b.wave_queries_per_triangle) *
                                                                    static_cast<double>(b.mesh_triangles[i]);
         m.wave = b.traversal != 0 && m.order != nullptr && dense ? 1u : 0u;
@@ -415,7 +422,8 @@ void batch_set_tuning(gwn_batch_handle &b, int block, int chunk, int blocks_per_
         throw_invalid("Batched query wave_queries_per_triangle must be positive and finite for traversal 2.");
     // The graph and any query in flight read the table and the counter: finish them first.
     wait_last_work(b);
-    bool const relayout = chunk != b.chunk || block != b.block || traversal != b.traversal ||
+    bool const relayout = chunk != b.chunk || block != b.block || blocks_per_cu != b.blocks_per_cu ||
+                          traversal != b.traversal ||
                           (traversal == 2 && wave_queries_per_triangle != b.wave_queries_per_triangle);
     b.block = block;
     b.chunk = chunk;

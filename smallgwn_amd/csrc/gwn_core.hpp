@@ -359,8 +359,8 @@ void taylor_batch_launch(
     std::uint64_t *counter, int order, int cap, int block, int blocks_per_cu, int cu_count, bool waves, bool quads,
     hipStream_t stream
 );
-// Whether a batch walks a mesh of `triangles` with whole waves (its queries are dense enough).
-bool batch_dense_queries(std::size_t triangles, std::size_t queries, float accuracy_scale);
+// Whether a batch of total_queries walks a mesh of `triangles` with whole waves (its queries are dense enough).
+bool batch_dense_queries(std::size_t triangles, std::size_t queries, std::size_t total_queries, float accuracy_scale);
 // Segmented builds (gwn_batch_build.hip): the H-PLOC BVH trees and Taylor moments of many meshes,
 // built side by side in one pass of a fixed sequence of launches that allocates nothing and never
 // reads back to the host, so the whole pass can be captured into a graph.  Each mesh's tree,

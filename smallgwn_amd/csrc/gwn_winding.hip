@@ -1515,15 +1515,21 @@ std::size_t batch_lds_bytes(int cap, int block, bool waves, bool quads) {
 
 } // namespace
 
-// The single-mesh rule, or 32 queries per triangle at beta 2: among many meshes the chip is full and the
-// work decides, not the longest wave, so small meshes' wave walks pay earlier.  2,048 meshes of up to
-// 2,000 triangles with up to 400,000 queries: 23.6 ms by the single-mesh rule alone, 20.4 from 16 queries
-// per triangle on, 21.3 from 64; 512 of up to 20,000 with 100,000: 3.84, 3.82, 3.70; 128 of up to 100,000
-// with 400,000: 2.54, 2.83, 2.44.
-bool batch_dense_queries(std::size_t triangles, std::size_t queries, float accuracy_scale) {
-    double const beta = std::max(1.0, double(accuracy_scale));
-    return dense_queries(triangles, queries, accuracy_scale * accuracy_scale) ||
-           double(queries) >= 32.0 * double(triangles) * std::pow(2.0 / beta, 1.5);
+// The single-mesh rule or 32 queries per triangle at beta 2, or fewer where the batch is ten times as long as a wave
+// of the mesh: its work decides then and not its longest wave.  That wave takes some 4 us sqrt(triangles), the
+// batch with four lanes per query 0.5 ns a query at beta 2.  Measured, 6M queries over equal meshes, four lanes /
+// whole waves: beta 2, 16 queries per triangle of 300 2.01 / 1.79 ms, of 3,000 2.69 / 2.50, of 20,000 2.70 / 2.86
+// (25.6M queries of 64 meshes, 20 per triangle of 20,000: 11.2 / 8.8), 8 per triangle of 300 1.13 / 1.15, of 3,000
+// 2.86 / 2.99; beta 4, 4 per triangle of 300 1.85 / 1.90, 8 of 300 3.36 / 2.51, 1 of 3,000 7.7 / 8.2, 2 of 3,000 14.0 /
+// 11.7, 2 of 20,000 14.8 / 12.4, 2 of 100,000 14.3 / 13.9, 4 of 100,000 13.8 / 11.1.  128 uneven meshes of up to
+// 100,000 triangles with 5.1M queries: 2.24 ms, 2.67 with the waves of three meshes of 6,700 to 12,000 triangles, of
+// which the batch is only six to eight times as long.
+bool batch_dense_queries(std::size_t triangles, std::size_t queries, std::size_t total_queries, float accuracy_scale) {
+    double const beta = std::max(1.0, double(accuracy_scale)) / 2.0, t = double(triangles), n = double(queries);
+    bool const lasting = 0.5e-3 * double(total_queries) * std::pow(beta, 2.25) >= 10.0 * 4.0 * std::sqrt(t);
+    bool const dense = n >= 1500.0 && n >= 12.0 * t * std::pow(beta, -3.3) * std::pow(std::max(1.0, t / 4000.0), 0.25);
+    return (lasting && dense) || dense_queries(triangles, queries, accuracy_scale * accuracy_scale) ||
+           n >= 32.0 * t * std::pow(beta, -1.5);
 }
 
 void taylor_batch_launch(
