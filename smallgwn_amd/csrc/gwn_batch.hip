@@ -12,9 +12,10 @@
 //     running 4096 launches back to back; every result equals the single-mesh batch's;
 //   - graph: the refits, the counter reset (a fill kernel, not a memset) and the query launch are
 //     captured once into a hipGraph on the batch's own stream and replayed with hipGraphLaunch;
-//   - traversal: one query per lane, or wave-cooperative (a wave walks the tree once for its 64
-//     queries) over each mesh's Hilbert query order, computed once when the batch is made (any
-//     order gives the same results; Hilbert order keeps a wave's queries close together);
+//   - traversal: four lanes per query, or, for meshes whose queries are dense, wave-cooperative (a
+//     wave walks the tree once for its 64 queries), over each mesh's Hilbert query order, computed
+//     once when the batch is made (any order gives the same results; Hilbert order keeps a wave's
+//     queries close together);
 //   - tune: traversal, block size, chunk length, blocks per CU and the compiled traversal stack
 //     are chosen by timing candidate launches;
 //   - builds: a batch made over geometries (batch_create_built) owns every mesh's tree and
@@ -22,6 +23,7 @@
 //     hold too, so a replay is builds + refits + queries; its tuner also picks the BVH width and
 //     the H-PLOC search radius.
 #include "gwn_core.hpp"
+#include "gwn_tune.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -67,7 +69,7 @@ struct gwn_batch_handle {
     int block = 256;
     int chunk = 256;
     int blocks_per_cu = 4;
-    int traversal = 0;                 // 0 per lane, 1 wave, 2 per mesh (wave_queries_per_triangle)
+    int traversal = 0;                 // 0 quads; waves for dense meshes: 1 by rule, 2 by wave_queries_per_triangle
     float wave_queries_per_triangle = 1.0f;
     int cu_count = 1;
     hipStream_t own_stream = nullptr;
@@ -438,8 +440,8 @@ void batch_set_tuning(gwn_batch_handle &b, int block, int chunk, int blocks_per_
     batch_drop_graph(b);
 }
 
-// Times each candidate (traversal, block size, chunk length, blocks per CU) with one launch
-// after a warm-up and keeps the fastest, then each compiled traversal stack that holds the trees'
+// Times each candidate (traversal, block size, chunk length, blocks per CU: batch_shapes) with one
+// launch after a warm-up and keeps the fastest, then each compiled traversal stack that holds the trees'
 // bound for that shape, then the per-mesh traversal at a few densities; returns the best time in
 // milliseconds.
 float batch_tune(gwn_batch_handle &b, hipStream_t stream) {
@@ -450,11 +452,8 @@ float batch_tune(gwn_batch_handle &b, hipStream_t stream) {
     };
     std::vector<cand> cands;
     float const density = b.wave_queries_per_triangle;
-    for (int traversal : {0, 1})
-        for (int block : {64, 128, 256})
-            for (int mult : {1, 4})
-                for (int bpc : {2, 4, 8})
-                    cands.push_back({block, block * mult, bpc, traversal, density});
+    for (batch_shape const &s : batch_shapes())
+        cands.push_back({s.block, s.chunk, s.blocks_per_cu, s.traversal, density});
     check_storage(b, true);
     hipEvent_t e0, e1;
     GWN_HIP(hipEventCreate(&e0));
