@@ -208,10 +208,11 @@ __global__ __launch_bounds__(k_hploc_seg_chunk_block) void seg_hploc_kernel(
 
 // H-PLOC global launch over the ranges the chunk launch parked.  A wave's merges run two at a time
 // (one per half), so with one range per lane a step of the climb lasts up to 32 merges; with a half
-// per range (HalfPerRange) it lasts one, but the launch takes 32 times the waves.  A half per range while
-// all of those waves fit the chip at once (8,192).  Measured, one range per lane against one per half: a replay
-// (build, moments, queries) of 128 meshes of 2.1M triangles 9.4 / 7.8 ms, of 8 meshes of 174,000 4.5 / 2.5 ms;
-// 4,096 meshes of 113M triangles (220,000 ranges) the other way round, 101 / 161 ms for the builds.
+// per range (HalfPerRange) it lasts one, but the launch takes 32 times the waves.  A half per range up to
+// 12,288 ranges (6,144 waves).  Measured, one range per lane against one per half, builds and moments: 8 meshes of
+// 100,000 triangles 4.21 / 2.24 ms, 512 of 2,000 3.58 / 1.84, 40 of 100,000 (7,800 ranges) 6.81 / 5.84, 60
+// (11,700) 8.50 / 8.39, 80 (15,600) 10.10 / 10.69, 4,000 of 2,000 9.57 / 9.87; 4,096 meshes of 113M triangles (220,000)
+// 101 / 161 ms.
 template <bool HalfPerRange>
 __global__ __launch_bounds__(k_hploc_block) void seg_hploc_parked_kernel(
     seg_mesh const *__restrict__ meshes, std::uint32_t const *__restrict__ leaf_prefix, std::uint32_t mesh_count,
@@ -901,7 +902,7 @@ void batch_trees_enqueue(batch_trees &t, int levels, int binary_levels, std::uin
             t.meshes.ptr, t.leaf_prefix.ptr, M, codes, t.leaf_boxes.ptr, n, t.radius, out_arrays, t.boundary.ptr,
             t.parked.ptr, t.root_words.ptr, t.words.ptr);
         GWN_LAUNCH_CHECK();
-        if (t.parked.count <= 2 * 8192)
+        if (t.parked.count <= 12288)
             seg_hploc_parked_kernel<true><<<static_cast<unsigned>(hploc_parked_blocks(t.parked.count)), k_hploc_block, 0,
                                             stream>>>(
                 t.meshes.ptr, t.leaf_prefix.ptr, M, codes, t.leaf_boxes.ptr, n, t.radius, out_arrays, t.boundary.ptr,

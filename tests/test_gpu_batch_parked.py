@@ -1,4 +1,4 @@
-"""H-PLOC over a batch large enough (more than 8.4M leaves) that the global launch takes one parked range per
+"""H-PLOC over a batch large enough (more than 6.3M leaves) that the global launch takes one parked range per
 lane instead of one per half wave: trees, moments and results still equal the single-mesh build's bit for bit."""
 
 import numpy as np
