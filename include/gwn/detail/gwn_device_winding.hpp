@@ -28,7 +28,7 @@ constexpr float k_pi_f = 3.14159265358979323846f;
 constexpr double k_pi_d = 3.14159265358979323846;
 
 // atan2(y, x) for max(|x|, |y|) in [2^-100, 2^100]: |t| <= 1 by one reciprocal, an odd polynomial of
-// degree 17 (a weighted minimax fit of atan(t) / t in t^2, 1.7e-8 relative) and the octants.  Within 3 ulps;
+// degree 17 (a weighted minimax fit of atan(t) / t in t^2, 2.1e-8 relative) and the octants.  Within 4 ulps;
 // 22 issue slots where the library's arctangent, with its exponent scaling and special cases, takes 35.
 __device__ inline float atan2_in_range(float y, float x) {
 #pragma clang fp contract(on)

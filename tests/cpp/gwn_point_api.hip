@@ -3,7 +3,8 @@
 // gwn_winding_gradient_taylor, gwn_winding_number_antipodal and gwn_winding_gradient_antipodal,
 // with a callback that records stack overflow per query (the reference's overflow_probe,
 // tests/unit_gwn_query_distance_ray.cu:86-110).  Built by tests/cpp/build.py with the library's
-// flags; the GPU tests compare every result with the corresponding batch's.
+// flags; the GPU tests compare every result with the corresponding batch's.  gwn_angle_run evaluates the
+// plain solid angle's own arctangent and normalisation on given operands.
 #include <gwn/gwn.hpp>
 #include <gwn/gwn_device.hpp>
 
@@ -95,7 +96,33 @@ void launch_taylor(gwn_bvh_t b, gwn_moment_t m, queries q, float beta, float *ou
     taylor_kernel<Order, Cap><<<grid(q.n), 256, 0, s>>>(ba, ma, q, beta, out, gx, gy, gz, flags);
 }
 
+__global__ void arctangent_kernel(float const *y, float const *x, std::uint64_t n, float *out) {
+    std::uint64_t const i = std::uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < n)
+        out[i] = gwn::detail::winding::atan2_in_range(y[i], x[i]);
+}
+
+__global__ void normalize_kernel(float const *ss, float *x, float *y, float *z, std::uint64_t n) {
+    std::uint64_t const i = std::uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= n)
+        return;
+    float v[3] = {x[i], y[i], z[i]};
+    gwn::detail::winding::normalize_in_range(ss[i], v[0], v[1], v[2]);
+    x[i] = v[0];
+    y[i] = v[1];
+    z[i] = v[2];
+}
+
 } // namespace
+
+// out = arctangent of (y, x); or, with squared lengths ss, (x, y, z) over their square roots in place.
+extern "C" int gwn_angle_run(float const *ss, float *x, float *y, float *z, std::uint64_t n, float *out, hipStream_t stream) {
+    if (ss != nullptr)
+        normalize_kernel<<<grid(n), 256, 0, stream>>>(ss, x, y, z, n);
+    else
+        arctangent_kernel<<<grid(n), 256, 0, stream>>>(y, x, n, out);
+    return hipGetLastError();
+}
 
 // op: 0 exact, 1 Taylor + gradient (order, beta), 2 distance (band), 3 first hit (t_min = a,
 // t_max = b), 4 antipodal winding + gradient.  cap: the compiled stack capacity, 64 or 1 (1 makes

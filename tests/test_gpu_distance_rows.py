@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from smallgwn_amd import synth
+from tests.helpers import nested_octants
 from tests.test_gpu_build import build_gpu
 
 pytestmark = pytest.mark.gpu
@@ -18,6 +19,7 @@ def _meshes():
     yield "layers", synth.layered_triangles(37)          # flat boxes
     yield "sphere", synth.displaced_sphere(48, 32)
     yield "soup", synth.open_soup(64, 40)
+    yield "octants", nested_octants(16)                  # stacks of more than 64 entries
 
 
 def _run(gwn, dev, bvh, q, lanes, band, nearest):
@@ -28,7 +30,7 @@ def _run(gwn, dev, bvh, q, lanes, band, nearest):
     out = torch.full((n,), 7.0, dtype=torch.float32, device=dev)
     near = torch.full((n,), 7, dtype=torch.int32, device=dev) if nearest else None
     gwn.gwn_compute_unsigned_distance_batch(bvh, *d, out, culling_band=band, nearest=near,
-                                            config=gwn.QueryConfig(lanes_per_point=lanes)).raise_if_error()
+                                            config=gwn.QueryConfig(lanes_per_point=lanes, stack_capacity=128)).raise_if_error()
     torch.cuda.synchronize()
     return out.cpu().numpy().view(np.uint32), near.cpu().numpy() if nearest else None
 

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from smallgwn_amd import synth
+from tests.helpers import nested_octants
 from tests.test_gpu_build import build_gpu
 
 pytestmark = pytest.mark.gpu
@@ -23,7 +24,7 @@ def _run(gwn, dev, bvh, mom, d, sort, precision, beta, grad):
     n = d[0].numel()
     out = torch.full((n,), 7.0, dtype=torch.float32, device=dev)
     cnt = torch.zeros(3 * n, dtype=torch.int32, device=dev)
-    cfg = gwn.QueryConfig(sort_queries=sort)
+    cfg = gwn.QueryConfig(sort_queries=sort, stack_capacity=128)
     if grad:
         g = [torch.full_like(out, 7.0) for _ in range(3)]
         gwn.gwn_compute_winding_gradient_taylor_batch(bvh, mom, *d, *g, accuracy_scale=beta, config=cfg,
@@ -102,3 +103,29 @@ def test_whole_waves_of_tiny_trees_in_any_order(gwn, dev, triangles, beta, grad)
                 b = b[:a.shape[0]]
                 fa, fb = a.view(np.float32), b.view(np.float32)
                 assert ((a == b) | (np.isnan(fa) & np.isnan(fb) if k != 1 else False)).all(), (n, k)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("order", [0, 1, 2])
+@pytest.mark.parametrize("name", ["sphere", "octants"])
+def test_rows_and_quads_equal_waves_on_deep_trees(gwn, dev, name, order, split, grad):
+    """Accepted terms, leaves and stacks of many entries (more than 64 allowed for the octants) together: a sorted
+    batch dense enough for whole waves, the same queries unsorted in rows and in quads."""
+    mesh = synth.displaced_sphere(40, 32) if name == "sphere" else nested_octants(16)
+    precision = gwn.Precision.SPLIT if split else gwn.Precision.PLAIN
+    _, bvh = build_gpu(gwn, mesh)
+    assert name == "sphere" or bvh.info()["internal_stack_bound"] > 64
+    mom = gwn.MomentObject(order)
+    gwn.gwn_refit_bvh_moment(bvh, mom).raise_if_error()
+    n_wave = 250000
+    assert n_wave >= 4500 * np.sqrt(mesh.i0.shape[0])  # dense at scale 2
+    q = synth.mixed_queries(mesh, n_wave, seed=order + 3)
+    if name == "octants":
+        for a in q:
+            a[:40000] *= np.float32(2.0) ** -(np.arange(40000) % 18).astype(np.float32)
+    want = _run(gwn, dev, bvh, mom, _first(q, n_wave, dev), 1, precision, 2.0, grad)
+    for n in (1000, 65536, 65537):
+        got = _run(gwn, dev, bvh, mom, _first(q, n, dev), 0, precision, 2.0, grad)
+        for k, (a, b) in enumerate(zip(got, want)):
+            assert np.array_equal(a, b[:a.shape[0]]), (n, k)
