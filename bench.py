@@ -493,7 +493,7 @@ def large_extras(args, dev, stream, bvh, d, idx) -> dict:
     hit_frac = float((status == int(gwn.RayStatus.HIT)).to(torch.float32).mean())
     res["ray_first_hit"] = {"mrays_per_s": n / (ms * 1e-3) / 1e6, "ms": ms, "rays": n, "hit_fraction": hit_frac,
                             "work": {"slab_tests": rbox, "triangle_tests": rtri},
-                            "roofline": _valu_roofline(ray_flops, ms, "ray_kernel<packed>",
+                            "roofline": _valu_roofline(ray_flops, ms, "ray_quad_kernel",
                                                        "14 FLOP per slab test, 60 per Pluecker triangle test")}
     log(f"rays: {ms:.2f} ms ({n / (ms * 1e-3) / 1e6:.1f} Mrays/s), hit fraction {hit_frac:.3f}, "
         f"frac {res['ray_first_hit']['roofline']['frac']}")
