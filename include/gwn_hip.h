@@ -67,10 +67,10 @@ typedef struct gwn_batch_handle *gwn_batch_t;
  * for its 64 points, each point pruning by its own best distance).  Its distances are each
  * point's minimum over the triangles it reaches, which can differ from the reference order's in
  * the last FP32 bits where a box distance rounds above a contained triangle's distance.
- * lanes_per_point (unsigned distance batch only; other batches ignore it): 0 (default: four or 16),
- * 1, or 4.  With four, the lanes of a quad share each BVH4 node, one child slot each; distances
- * and nearest records equal the one-lane traversal's bit for bit.  Ignored with
- * sort_queries = 2. */
+ * lanes_per_point (unsigned distance batch only; other batches ignore it): 1, or 0 and 4, which are the
+ * same: four lanes, one child slot of each BVH4 node each, and 16 for the points of small batches and
+ * the last ones of a wave.  Distances and nearest records equal the one-lane traversal's bit for bit.
+ * Ignored with sort_queries = 2. */
 typedef struct gwn_query_config {
     int32_t block_size;
     int32_t stack_capacity;
@@ -327,7 +327,10 @@ int gwn_compute_winding_number_taylor_batch_f64(
     hipStream_t stream);
 
 /* Precision-split and FP64 forms (no reference counterpart: the reference computes in the
- * geometry's Real).  The exact form writes double results for every precision. */
+ * geometry's Real).  The exact form writes double results for every precision.  Its split and FP64
+ * batches may share the triangles out over the machine and add the shares' FP64 sums: that takes up to
+ * 64 MiB of stream-ordered scratch (none in a captured stream, or where there is no memory for it), and
+ * the last FP64 bits of a result then depend on the number of queries and on capture. */
 int gwn_compute_winding_number_exact_batch_ex_f32(
     gwn_bvh_t bvh, const float *qx, const float *qy, const float *qz, double *out, uint64_t count,
     int32_t precision, const gwn_query_config *config, hipStream_t stream);
@@ -482,15 +485,16 @@ typedef struct gwn_batch_item {
 typedef struct gwn_batch_tuning {
     int32_t block_size;      /* 64, 128, 192 or 256 threads */
     int32_t chunk;           /* queries per work item of a wave-cooperative mesh, a multiple of
-                                block_size (four lanes per query: block_size / 4 queries) */
+                                block_size (four lanes per query: block_size / 4 queries, or 64
+                                where every block has many) */
     int32_t blocks_per_cu;   /* persistent grid = blocks_per_cu x compute units */
     int32_t traversal;       /* 0: four lanes per query; 1: wave-cooperative over each mesh's
                                 Hilbert query order (computed at create) where the mesh's queries
                                 are dense enough for that to pay, four lanes elsewhere; 2: wave-
                                 cooperative where the mesh has at least wave_queries_per_triangle
-                                queries per triangle, four lanes elsewhere.  All three give the
-                                same results. */
-    int32_t stack_capacity;  /* compiled traversal stack: 32, 64 or 128, at least every tree's
+                                queries per triangle, four lanes elsewhere (a tiny threshold makes
+                                every mesh wave-cooperative).  All three give the same results. */
+    int32_t stack_capacity;  /* largest traversal stack: 32, 64 or 128, at least every tree's
                                 internal_stack_bound; 0 in gwn_batch_set_tuning keeps it */
     float wave_queries_per_triangle; /* traversal 2's density threshold (positive, finite); read
                                 only for traversal 2.  It fills what was padding, so the layout

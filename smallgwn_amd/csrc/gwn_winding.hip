@@ -780,7 +780,7 @@ template <int Order, bool Grad> struct slot_test {
 // unsorted, one lane per query against this form: 262,144 of 131,072 2.26 / 1.38 ms.
 // Tried and slower: holding a quad's leaf triangles back until half of the wave's quads have some, so that
 // they are evaluated with more lanes active (5-20 %); handing a finished quad another query of the wave
-// (0-40 %: a wave's queries are then no longer neighbours, and their reads no longer shared).
+// (15-70 %: a wave's queries are then no longer neighbours, and their reads no longer shared).
 template <int Order, int Prec, bool Grad>
 __device__ inline bool taylor_quad_traverse(
     float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node, float x, float y,

@@ -121,7 +121,7 @@ class QueryConfig:
     block_size: int = DEFAULT_BLOCK_SIZE
     stack_capacity: int = DEFAULT_STACK_CAPACITY
     sort_queries: int = -1
-    lanes_per_point: int = 0  # unsigned distance: 0 (four or 16) or 1 or 4 lanes per point, same results
+    lanes_per_point: int = 0  # unsigned distance: 1 lane per point, or 0 and 4: four or 16, same results
 
 
 class _CConfig(ctypes.Structure):
