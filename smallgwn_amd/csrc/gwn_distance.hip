@@ -140,18 +140,6 @@ __global__ __launch_bounds__(k_block) void distance_wave_kernel(
     }
 }
 
-// Over the 16 lanes of a row: row_half_mirror joins quads 0-1 and 2-3, row_mirror the two halves.
-__device__ inline std::uint32_t row_or(std::uint32_t v) {
-    v = quad_or(v);
-    v |= static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xf, 0xf, false));
-    return v | static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xf, 0xf, false));
-}
-__device__ inline std::uint32_t row_min(std::uint32_t v) {
-    v = quad_min(v);
-    v = min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xf, 0xf, false)));
-    return min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xf, 0xf, false)));
-}
-
 // box_distance2 for a child's box (min <= max): at most one of the two excesses of an axis is positive,
 // so their sum is the larger of them and zero.
 __device__ inline float child_box_distance2(float x, float y, float z, aabb const &b) {

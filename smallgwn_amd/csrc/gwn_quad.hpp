@@ -1,5 +1,5 @@
-// gwn_quad.hpp - four lanes per query: exchange within a quad and the near-first order of a BVH4 node's
-// children, shared by the distance and ray batches.
+// gwn_quad.hpp - four lanes per query: exchange within a quad and a row of 16, and the near-first order of a
+// BVH4 node's children, shared by the distance, ray and winding batches.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -13,10 +13,16 @@ namespace gwn {
 namespace {
 
 // Every lane of a quad (lanes 4k..4k+3) receives lane S's value.
-template <int S>
-__device__ inline std::uint32_t quad_bcast(std::uint32_t v) {
-    return static_cast<std::uint32_t>(
-        __builtin_amdgcn_update_dpp(0, static_cast<int>(v), S * 0x55, 0xf, 0xf, false));  // quad_perm [S,S,S,S]
+template <int S, class T> __device__ inline T quad_bcast(T v) {
+    if constexpr (sizeof(T) == 8) {
+        std::uint64_t const b = __builtin_bit_cast(std::uint64_t, v);
+        std::uint64_t const lo = quad_bcast<S>(static_cast<std::uint32_t>(b));
+        std::uint64_t const hi = quad_bcast<S>(static_cast<std::uint32_t>(b >> 32));
+        return __builtin_bit_cast(T, (hi << 32) | lo);
+    } else {
+        return __builtin_bit_cast(
+            T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), S * 0x55, 0xf, 0xf, false));  // quad_perm [S, S, S, S]
+    }
 }
 
 // The other lane's value: quad_perm [1, 0, 3, 2] and [2, 3, 0, 1].
@@ -37,6 +43,27 @@ __device__ inline float quad_min(float v) {  // no NaN
 __device__ inline std::uint32_t quad_min(std::uint32_t v) {
     v = min(v, quad_swap1(v));
     return min(v, quad_swap2(v));
+}
+
+__device__ inline std::uint32_t quad_sum(std::uint32_t v) {
+    return quad_bcast<0>(v) + quad_bcast<1>(v) + quad_bcast<2>(v) + quad_bcast<3>(v);
+}
+
+// Over the 16 lanes of a row: row_half_mirror joins quads 0-1 and 2-3, row_mirror the two halves.
+__device__ inline std::uint32_t row_or(std::uint32_t v) {
+    v = quad_or(v);
+    v |= static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xf, 0xf, false));
+    return v | static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xf, 0xf, false));
+}
+__device__ inline std::uint32_t row_min(std::uint32_t v) {
+    v = quad_min(v);
+    v = min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xf, 0xf, false)));
+    return min(v, static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xf, 0xf, false)));
+}
+__device__ inline std::uint32_t row_sum(std::uint32_t v) {
+    v = quad_sum(v);
+    v += static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xf, 0xf, false));
+    return v + static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xf, 0xf, false));
 }
 
 // Slot lists of the 16 passing masks: bits 2t..2t+1 hold the t-th slot, the passing ones first, each

@@ -27,6 +27,7 @@
 #include "gwn_core.hpp"
 #include "gwn_slices.hpp"
 #include "../../include/gwn/detail/gwn_device_winding.hpp"
+#include "gwn_quad.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -652,19 +653,6 @@ __global__ __launch_bounds__(256) void leaf_root_kernel(
     }
 }
 
-// Every lane of a quad (lanes 4k..4k+3) receives lane S's value.
-template <int S, class T> __device__ inline T quad_bcast(T v) {
-    if constexpr (sizeof(T) == 8) {
-        std::uint64_t const b = __builtin_bit_cast(std::uint64_t, v);
-        std::uint64_t const lo = quad_bcast<S>(static_cast<std::uint32_t>(b));
-        std::uint64_t const hi = quad_bcast<S>(static_cast<std::uint32_t>(b >> 32));
-        return __builtin_bit_cast(T, (hi << 32) | lo);
-    } else {
-        return __builtin_bit_cast(
-            T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), S * 0x55, 0xf, 0xf, false));  // quad_perm [S, S, S, S]
-    }
-}
-
 // What one lane of a quad reads of a node: its slot's reference, acceptance fields and coefficients.
 template <int Order, bool Grad> struct quad_slot {
     static constexpr int k_fields = moment_field_count(Order);
@@ -700,16 +688,6 @@ template <int Order, bool Grad> struct quad_slot {
         return s;
     }
 };
-
-__device__ inline std::uint32_t quad_sum(std::uint32_t v) {
-    return quad_bcast<0>(v) + quad_bcast<1>(v) + quad_bcast<2>(v) + quad_bcast<3>(v);
-}
-// Over the 16 lanes of a row: row_half_mirror joins quads 0-1 and 2-3, row_mirror the halves.
-__device__ inline std::uint32_t row_sum(std::uint32_t v) {
-    v = quad_sum(v);
-    v += static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xf, 0xf, false));
-    return v + static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xf, 0xf, false));
-}
 
 // Adds the terms of a row's 16 lanes (or a quad's four) to the sum in lane order.
 template <int Lanes> __device__ inline void ordered_add(float &sum, float v) { add_in_lane_order<Lanes>(sum, v); }
