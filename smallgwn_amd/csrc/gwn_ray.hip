@@ -319,13 +319,6 @@ bool ray_half_bounds(int entries, unsigned grid) {
     return bytes > k_lds_per_block || (6 * bytes > k_lds_per_cu && grid > 256 * (k_lds_per_cu / bytes));
 }
 
-// LDS to ask for: no less than lets the blocks of a grid that fits the chip lie on it evenly (65,536 rays of
-// 2,097,152 triangles, four blocks a CU: 767 us, 850 us with room for more of them on one CU).
-std::size_t ray_lds_bytes(int entries, bool half, unsigned grid) {
-    std::size_t const per_cu = (grid + 255u) / 256u;
-    return std::max(ray_stack_bytes(entries, half), std::min(k_lds_per_block, k_lds_per_cu / (per_cu + 1) + 8));
-}
-
 // Large batches over a few nodes keep one ray per lane: nearly every ray meets all of them, so there is no chain
 // to shorten and the lanes' work is even.  One lane against four, 4,194,304 rays of 24 triangles 591 / 721 us, of
 // 50 775 / 889, of 500 1,291 / 1,243; 1,000,003 of 24 166 / 186; 65,536 of 24 41 / 23.
@@ -345,10 +338,10 @@ void launch_ray(
         unsigned const grid = ray_quad_grid(n);
         std::uint32_t const root = static_cast<std::uint32_t>(ref_offset(bvh.root.reference));
         if (ray_half_bounds(need, grid))
-            ray_quad_kernel<Packed, true><<<grid, k_block, ray_lds_bytes(need, true, grid), stream>>>(
+            ray_quad_kernel<Packed, true><<<grid, k_block, ray_stack_bytes(need, true), stream>>>(
                 sc, root, need, ox, oy, oz, dx, dy, dz, static_cast<ray_hit *>(out), n, t_min, t_max);
         else
-            ray_quad_kernel<Packed, false><<<grid, k_block, ray_lds_bytes(need, false, grid), stream>>>(
+            ray_quad_kernel<Packed, false><<<grid, k_block, ray_stack_bytes(need, false), stream>>>(
                 sc, root, need, ox, oy, oz, dx, dy, dz, static_cast<ray_hit *>(out), n, t_min, t_max);
     } else
         ray_kernel<Packed, Cap><<<grid_for(n, k_block), k_block, 0, stream>>>(
