@@ -383,7 +383,7 @@ __device__ inline bool taylor_wave_traverse(
 );
 
 // Four lanes per query (defined below; the batched kernel uses it too).
-template <int Order, int Prec, bool Grad>
+template <int Order, int Prec, bool Grad, int StackCap>
 __device__ inline bool taylor_quad_traverse(
     float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node, float x, float y,
     float z, float beta2, taylor_sums<Prec, Grad> &acc, std::uint32_t &n_tests, std::uint32_t &n_accept,
@@ -442,7 +442,7 @@ __global__ __launch_bounds__(256) void taylor_batch_kernel(
                 std::uint64_t const q = m.order ? m.order[p] : p;
                 taylor_sums<GWN_PRECISION_PLAIN, false> acc;
                 std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;
-                bool const overflow = taylor_quad_traverse<Order, GWN_PRECISION_PLAIN, false>(
+                bool const overflow = taylor_quad_traverse<Order, GWN_PRECISION_PLAIN, false, 0>(
                     m.records, m.tris, static_cast<std::uint32_t>(ref_offset(m.root)), m.qx[q], m.qy[q], m.qz[q], beta2,
                     acc, n_tests, n_accept, n_leaf, s_quad, quads, cap);
                 if ((threadIdx.x & 3u) == 0u)
@@ -748,7 +748,8 @@ template <int Order, bool Grad> struct slot_test {
 // added in slot order (add_terms; a slot without a term adds zero, which leaves every sum as it is, since
 // a sum starts at +0 and never becomes -0); descended children are pushed in slot order and the last one
 // entered, as taylor_traverse does.  Decisions, terms and the order of every sum are those of the per-lane
-// traversal, so the results are too, bit for bit.  The stack is the quad's column of an LDS array.
+// traversal, so the results are too, bit for bit.  The stack is the quad's column of an LDS array, of StackCap
+// entries or, with StackCap 0, of `cap`.
 //
 // A chain of dependent node reads per query: one lane per query waited for the header, then for each
 // accepted slot's coefficients and each leaf's triangle in turn (about eight waits a node); here a node's
@@ -759,13 +760,14 @@ template <int Order, bool Grad> struct slot_test {
 // Tried and slower: holding a quad's leaf triangles back until half of the wave's quads have some, so that
 // they are evaluated with more lanes active (5-20 %); handing a finished quad another query of the wave
 // (15-70 %: a wave's queries are then no longer neighbours, and their reads no longer shared).
-template <int Order, int Prec, bool Grad>
+template <int Order, int Prec, bool Grad, int StackCap>
 __device__ inline bool taylor_quad_traverse(
     float4 const *__restrict__ records, tri_record const *__restrict__ tris, std::uint32_t root_node, float x, float y,
     float z, float beta2, taylor_sums<Prec, Grad> &acc, std::uint32_t &n_tests, std::uint32_t &n_accept,
     std::uint32_t &n_leaf, std::uint32_t *stack, int stride, int cap
 ) {
     using slot_type = quad_slot<Order, Grad>;
+    int const limit = StackCap != 0 ? StackCap : cap;
     int const j = static_cast<int>(threadIdx.x & 3);
     int const shift = static_cast<int>(threadIdx.x & 60);
     int sp = 0;
@@ -788,12 +790,12 @@ __device__ inline bool taylor_quad_traverse(
         int const pushed = __popc(bits) - 1;
         std::uint32_t next = bits & 8u ? c3 : (bits & 4u ? c2 : (bits & 2u ? c1 : c0));
         int const at = sp + __popc(bits & ((1u << j) - 1u));
-        if (v.inner && (bits >> j) != 1u && at < cap)
+        if (v.inner && (bits >> j) != 1u && at < limit)
             stack[at * stride] = c;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         if (pushed >= 0) {
             sp += pushed;
-            overflow = sp > cap;
+            overflow = sp > limit;
             live = !overflow;
         } else if (sp > 0) {
             next = stack[--sp * stride];
@@ -826,7 +828,7 @@ __global__ __launch_bounds__(k_taylor_block) void taylor_quad_kernel(
     std::size_t const q = order ? order[i] : i;
     taylor_sums<Prec, Grad> acc;
     std::uint32_t n_tests = 0, n_accept = 0, n_leaf = 0;  // this lane's
-    bool const overflow = taylor_quad_traverse<Order, Prec, Grad>(
+    bool const overflow = taylor_quad_traverse<Order, Prec, Grad, StackCap>(
         records, tris, root_node, qx[q], qy[q], qz[q], beta2, acc, n_tests, n_accept, n_leaf,
         s_stack + (threadIdx.x >> 2), k_quads, StackCap);
     if (j == 0)
